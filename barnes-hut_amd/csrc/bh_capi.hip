@@ -179,7 +179,7 @@ int reserve(bh_ctx* c, size_t n)
     t.bsys = c->bsys_w;
     MixedBuffers& m = c->mb;
     A(m.node, 2 * N); A(m.slot, 2 * N); A(m.base, N); A(m.gfirst, N + 1); A(m.gdepth, N);
-    A(m.g_inter, N); A(m.g_visit, N); A(m.g_work, N); A(m.g_t0, N); A(m.g_t1, N); A(m.g_worker, N); A(m.order, N); A(m.chunk, 65536); A(m.gcost, N);
+    A(m.g_inter, N); A(m.g_visit, N); A(m.g_work, N); A(m.g_t0, N); A(m.g_t1, N); A(m.g_worker, N); A(m.order, N); A(m.chunk, bh::kMaxShared); A(m.gcost, N); A(m.gbig, N);
     c->heavy_item_cap = static_cast<size_t>(bh::kMaxHeavy) * (N / bh::kHeavyChunk + bh::kMaxSystems + 1);
     A(m.hpart, 3 * c->heavy_item_cap);
     A(c->md.feat, static_cast<size_t>(bh::kModelFeatures) * N);
@@ -238,6 +238,7 @@ int run_force(bh_ctx* c, int form, double theta, double G, double soft2, bool ki
     } else {
         tb.deep_from = bh::kMaxDepth;   // the light-moment pyramid needs no list of deep nodes
     }
+    c->mb.walk_waves = c->mixed_blocks * 4;
     bh::launch_build_tree(c->cur, c->n, tb, !mixed, s);
     if (mixed) {
         // The slot layout and extent limits need the topology only.  From 2^20
@@ -701,6 +702,7 @@ int bh_set_bodies(bh_ctx* c, int64_t n, const bh_vec3* pos, const bh_vec3* vel, 
     }
     HIP_TRY(c, hipMemcpyAsync(c->cur.id, ids, n * 8, hipMemcpyHostToDevice, s));
     HIP_TRY(c, hipMemsetAsync(c->cur.pcost, 0, n * sizeof(uint32_t), s));
+    HIP_TRY(c, hipMemsetAsync(&c->tb.sc->work_sum, 0, sizeof(StepScalars) - offsetof(StepScalars, work_sum), s));
     rc = configure_systems(c, std::vector<int64_t>{n}, mass);
     if (rc) return rc;
     HIP_TRY(c, hipMemsetAsync(c->cur.ax, 0, n * 8, s));

@@ -78,14 +78,30 @@ struct StepScalars {
     uint64_t n_full;     // node count of the reference's full-chain map
     uint32_t error;          // kErr* bits raised by bounds guards
     uint32_t n_groups;       // walk groups of the mixed forms
-    uint32_t group_counter;  // dynamic work queue of the mixed walk (cost order, split schedule)
     uint32_t cost_total;     // sum of the group weights of the split schedule
-    uint32_t part_counter[8];   // one work queue per group part (kWalkParts)
-    uint32_t heavy_counter;     // heavy-sum work items taken in the walk's tail
     uint32_t sched_hist[8][128];   // groups per cost bucket of the heaviest-first order, one copy per XCD
     uint32_t sched_cursor[128]; // groups placed per bucket so far (both cleared by k_kick_drift_box)
     uint32_t n_deep;            // branching nodes at depth >= TreeBuffers::deep_from (listed in deep)
+    // Queue counters of the mixed walk, one 128-byte line each (kQ*), so that
+    // takes from different queues do not wait for each other and the scalars
+    // above are read without waiting for them.
+    alignas(128) uint32_t queue[12][32];
+    // Work of the walk (its groups' g_work), summed by XCD; k_keys moves the
+    // sum to work_prev when there is one.  work_prev 0: no walk since the
+    // bodies were set.
+    alignas(128) uint64_t work_sum[8][16];
+    uint64_t work_prev;
+    uint32_t groups_prev;   // groups of that walk
+    uint32_t n_big;    // key order: groups shared by a block's wavefronts (listed in MixedBuffers::chunk)
+    uint32_t n_coop;   // cost order: the same, the first of the order
 };
+
+// StepScalars::queue rows: 0..7 the group parts (kWalkParts), then the one
+// queue of the cost order and the split schedule, the heavy-sum items, the
+// shared groups, and the mask of the closed parts
+constexpr uint32_t kQOrder = 8, kQHeavy = 9, kQShared = 10, kQClosed = 11;
+constexpr uint32_t kQueues = 12;
+constexpr uint32_t kMaxShared = 65536;   // entries of MixedBuffers::chunk
 
 // In key order the mixed walk deals its groups out in runs of kWalkRun
 // consecutive groups, run r to part r mod kWalkParts, one part per XCD
@@ -161,6 +177,35 @@ __device__ inline uint32_t scan_block_excl(uint32_t v, const uint32_t* tsum, siz
     uint32_t off = direct ? p4[0] + p4[1] + p4[2] + p4[3] : tsum[blockIdx.x];
     for (int q = 0; q < w; ++q) off += w4[q];
     return off + inc - v;
+}
+
+// 1.0 / sqrt(x) for x in [2^-767, 2^1000], bit for bit: the instruction
+// sequence the compiler emits for the IEEE FP64 square root (reciprocal
+// square-root estimate refined by Goldschmidt steps) followed by the one for
+// the IEEE division 1 / s (reciprocal estimate, two Newton steps, remainder
+// correction), without their range handling.  In this range the square root
+// needs no exponent scaling and is finite and nonzero, and 1 / s with
+// s in [2^-500, 2^500] needs no scaling and no fix-up, so the range handling
+// leaves every value unchanged there and dropping it saves 12 instructions.
+__device__ inline double inv_sqrt_in_range(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y;
+    double h = y * 0.5;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    double d = __builtin_fma(-g, g, x);
+    g = __builtin_fma(d, h, g);
+    d = __builtin_fma(-g, g, x);
+    g = __builtin_fma(d, h, g);   // sqrt(x), correctly rounded
+    double q = __builtin_amdgcn_rcp(g);
+    double e = __builtin_fma(-g, q, 1.0);
+    q = __builtin_fma(q, e, q);
+    e = __builtin_fma(-g, q, 1.0);
+    q = __builtin_fma(q, e, q);
+    e = __builtin_fma(-g, q, 1.0);
+    return __builtin_fma(e, q, q);   // 1 / sqrt(x), correctly rounded
 }
 
 // ----------------------------------------------------------------- sort
@@ -301,14 +346,22 @@ struct MNode {
     double x, y, z;   // centre of mass of the light bodies (FP64); a one-body
                       // leaf holds the body's own position
     double size2;     // opening size^2: squared distance from the centre of mass
-                      // to the farthest corner of the light bodies' box
+                      // to the farthest corner of the light bodies' box (+inf for
+                      // a leaf of several bodies: never accepted as a whole)
     float gm;         // G * light mass
-    uint32_t first;   // first child slot (branching) or first body (leaf)
+    uint32_t push;    // what opening the node pushes: its child slots or its bodies (stack_range)
     uint32_t info;    // child or body count | kMLeaf
     float gq;         // G * sum of m |x - com|^2 over the light bodies (quadrupole scale)
 };
 static_assert(sizeof(MNode) == 48, "MNode is 48 bytes");
 constexpr uint32_t kMLeaf = 1u << 31;
+// Stack entry of the mixed walk: first (27 bits) | count - 1 (3 bits) | body
+// range (bit 31).  A leaf of more than 8 bodies has count 1 here; its bodies
+// are not pushed (the walk lists them directly).
+__host__ __device__ inline uint32_t stack_range(uint32_t first, uint32_t count, bool body)
+{
+    return first | ((count <= 8u ? count - 1u : 0u) << 27) | (body ? 0x80000000u : 0u);
+}
 constexpr int kGroupMax = 64;   // bodies per walk group (one wavefront): the largest group limit
 constexpr uint32_t kHeavyChunk = 1024;   // bodies per work item of the heavy direct sums
 
@@ -325,8 +378,11 @@ struct MixedBuffers {
     uint64_t* g_t1;     // N: wall clock when it finished
     uint32_t* g_worker; // N: worker wave that walked the group
     uint32_t* order;    // N: group order of the scheduled walk
-    uint32_t* chunk;    // split schedule: first group of each chunk (n_chunks + 1, <= 65536)
+    uint32_t* chunk;    // split schedule: first group of each chunk (n_chunks + 1, <= 65536);
+                        // otherwise the shared groups of the key order
     float* gcost;       // N: estimated cost of each group
+    uint8_t* gbig;      // N: 1 for a group listed as shared (key order)
+    uint32_t walk_waves;   // wavefronts of the walk's grid
     double* hpart;      // heavy direct sums: 3 partials per work item (system, heavy rank, chunk)
 };
 

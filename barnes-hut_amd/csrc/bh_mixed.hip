@@ -28,10 +28,10 @@
 // lanes test the nodes of their range in FP64.  Accepted nodes and the bodies
 // of reached leaves go into an LDS interaction list as FP32 (x - c, y - c,
 // z - c, G m) with c the group centre (FP64), so the offsets keep FP32
-// precision near the group.  A full list is evaluated by all 64 lanes:
+// precision near the group.  A full list is cut into shares, so that every
+// lane has one whatever the group's size, and evaluated in
 // FP32 FMA over blocks of 32 entries, each block sum added into a
-// Kahan-compensated FP32 accumulator; lanes past a group's bodies take over
-// stretches of the bodies' lists.  A group's own bodies appear in the
+// Kahan-compensated FP32 accumulator.  A group's own bodies appear in the
 // list with offsets bit-identical to the lane's own, so the self term has
 // dx = dy = dz = 0 and adds +0 (r^2 starts from a small positive floor).
 //
@@ -51,7 +51,16 @@ namespace {
 
 constexpr int kNT = 256;
 constexpr int kWaves = kNT / 64;
+// kShare = 0.6.  Walk, ms (cost order, key order), kShare 0.2 / 0.6 / 1.0 /
+// no sharing: 50k bodies 0.128, 0.150 / 0.128, 0.147 / 0.125, 0.149 / 0.197,
+// 0.200; 200k key order 0.436 / 0.330 / 0.424 / 0.416; 300k 0.475, 0.520 /
+// 0.437, 0.493 / 0.440, 0.490 / 0.428, 0.486.  A shared group's round costs a
+// third more wave time than a lone wavefront's (its barriers, and four
+// wavefronts working out the same ranges), so sharing pays only for groups
+// that would end late, and the limit grows with the groups per wave.
+constexpr uint32_t kShareNum = 3, kShareDen = 5;
 constexpr int kListCap = 256;
+constexpr int kListPad = 64;    // zero entries past a flushed list (share_len)
 constexpr int kStackCap = 1024;
 // Up to 64 ranges may be popped while the stack holds at most this many
 // entries: one round pushes at most 8 ranges per popped range, and a
@@ -62,12 +71,6 @@ constexpr uint32_t kNone = 0xffffffffu;
 // (which grows like (b/D)^2 / (1 - b/D)^2) small; above it, up to theta, the
 // relative quadrupole test decides as well
 constexpr double kSafe2 = 0.64;
-
-// stack entry: first (27 bits) | count - 1 (3 bits, ranges hold <= 8) | body range (bit 31)
-__device__ inline uint32_t enc(uint32_t first, uint32_t count, bool body)
-{
-    return first | ((count - 1u) << 27) | (body ? 0x80000000u : 0u);   // count in [1, 8]
-}
 
 // Cell occupancy by depth, per system: sys[s].dcount[d] = number of
 // boundaries u[j] | u[j+1] inside system s that split at depth d, so depth d
@@ -309,10 +312,28 @@ __global__ __launch_bounds__(kNT) void k_group_marks(size_t n, TreeBuffers tb, M
     }
 }
 
-__device__ inline void group_first(size_t i, size_t n, uint32_t gid, const TreeBuffers& tb, const MixedBuffers& mb)
+// A group is shared by a block's wavefronts when its work in the previous
+// walk exceeds this: kShare x (groups per wave) x (an even share of the walk
+// per wave).  See k_walk_mixed for the choice.
+__device__ inline uint64_t share_limit(const StepScalars* sc, uint32_t walk_waves)
+{
+    return sc->work_prev * sc->groups_prev * kShareNum / (static_cast<uint64_t>(walk_waves) * walk_waves * kShareDen);
+}
+
+__device__ inline void group_first(size_t i, size_t n, uint32_t gid, const Bodies& b, const TreeBuffers& tb,
+                                   const MixedBuffers& mb)
 {
     const uint32_t f = tb.gflag[i];
-    if (f) mb.gfirst[gid] = static_cast<uint32_t>(i);
+    if (f) {
+        mb.gfirst[gid] = static_cast<uint32_t>(i);
+        bool big = tb.sc->work_prev != 0u && b.pcost[i] > share_limit(tb.sc, mb.walk_waves);
+        if (big) {
+            const uint32_t k = atomicAdd(&tb.sc->n_big, 1u);
+            big = k < kMaxShared;   // (at most waves^2 / (kShare x groups) exceed the limit)
+            if (big) mb.chunk[k] = gid;
+        }
+        mb.gbig[gid] = big ? 1u : 0u;
+    }
     if (i + 1 == n) {   // the group count G and the end sentinel gfirst[G] = n
         mb.gfirst[gid + f] = static_cast<uint32_t>(n);
         tb.sc->n_groups = gid + f;
@@ -344,7 +365,7 @@ __global__ __launch_bounds__(kNT) void k_mixed_nodes(size_t n, Bodies b, TreeBuf
     const size_t t = static_cast<size_t>(blockIdx.x) * kNT + threadIdx.x;
     if (static_cast<size_t>(blockIdx.x) * kNT < n) {   // block-uniform: the blocks over the bodies
         const uint32_t gid = scan_block_excl(t < n ? tb.gflag[t] : 0u, tb.gtile, n);
-        if (t < n) group_first(t, n, gid, tb, mb);
+        if (t < n) group_first(t, n, gid, b, tb, mb);
     }
     const uint32_t M = tb.sc->n_leaves, B = tb.sc->n_branch;
     if (t >= static_cast<size_t>(M) + B) return;
@@ -393,9 +414,10 @@ __global__ __launch_bounds__(kNT) void k_mixed_nodes(size_t n, Bodies b, TreeBuf
     }
     nd.size2 = s2;
     if (leaf) {
-        nd.first = f0;
+        nd.push = stack_range(f0, f1 - f0, true);
         nd.info = (f1 - f0) | kMLeaf;
-        if (f1 - f0 == 1u) {
+        if (f1 - f0 > 1u) nd.size2 = INFINITY;
+        else {
             // the body itself (its light mass is its mass, or 0 if heavy):
             // the walk appends it from the node alone, with the very offsets
             // a body entry gives, which the self-term test relies on
@@ -408,7 +430,7 @@ __global__ __launch_bounds__(kNT) void k_mixed_nodes(size_t n, Bodies b, TreeBuf
         uint32_t k = 0;
 #pragma unroll
         for (int o = 0; o < 8; ++o) k += c[o] >= 0 ? 1u : 0u;
-        nd.first = tb.n_sys + base;
+        nd.push = stack_range(tb.n_sys + base, k, false);
         nd.info = k;
     }
     mb.node[slot] = nd;
@@ -420,21 +442,36 @@ __device__ inline uint32_t uni(uint32_t v)
     return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
 }
 
+// Cross-lane moves within a row of 16 lanes by DPP (no LDS round trip);
+// kCtrl: 0x120 + k rotates the row right by k, 0x110 + k shifts it right
+template <int kCtrl>
+__device__ inline double dpp_f64(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), kCtrl, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), kCtrl, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+__device__ inline double min2(double v, double t) { return (t < v) ? t : v; }
+__device__ inline double max2(double v, double t) { return (v < t) ? t : v; }
+
 __device__ inline double wave_min(double v)
 {
-    for (int o = 32; o > 0; o >>= 1) {
-        const double t = __shfl_xor(v, o, 64);
-        v = (t < v) ? t : v;
-    }
-    return v;
+    v = min2(v, dpp_f64<0x128>(v));
+    v = min2(v, dpp_f64<0x124>(v));
+    v = min2(v, dpp_f64<0x122>(v));
+    v = min2(v, dpp_f64<0x121>(v));
+    v = min2(v, __shfl_xor(v, 16, 64));
+    return min2(v, __shfl_xor(v, 32, 64));
 }
 __device__ inline double wave_max(double v)
 {
-    for (int o = 32; o > 0; o >>= 1) {
-        const double t = __shfl_xor(v, o, 64);
-        v = (v < t) ? t : v;
-    }
-    return v;
+    v = max2(v, dpp_f64<0x128>(v));
+    v = max2(v, dpp_f64<0x124>(v));
+    v = max2(v, dpp_f64<0x122>(v));
+    v = max2(v, dpp_f64<0x121>(v));
+    v = max2(v, __shfl_xor(v, 16, 64));
+    return max2(v, __shfl_xor(v, 32, 64));
 }
 
 // lane k's value (k wave-uniform)
@@ -458,13 +495,16 @@ __device__ inline uint32_t rank_below(uint64_t mask)
 
 __device__ inline uint32_t wave_incl_scan(uint32_t v)
 {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t t = static_cast<uint32_t>(__shfl_up(static_cast<int>(v), o, 64));
-        if (lane >= o) v += t;
-    }
-    return v;
+    // rows of 16 by row shifts, then row 0 into row 1 and 2 into 3, then the
+    // lower half into the upper (row_bcast); absent lanes add 0
+    int x = static_cast<int>(v);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return static_cast<uint32_t>(x);
 }
 
 struct Acc3 {
@@ -514,153 +554,174 @@ __device__ inline void interact(const float4 q, float ox, float oy, float oz, fl
     bz = fmaf(s, dz, bz);
 }
 
-// Evaluates this lane's share of list[0..ln) for its body (offsets ox, oy,
-// oz): with K lanes per body, the entries sub, sub + K, sub + 2K, ...  FP32
-// FMA inside blocks of 32 such entries, Kahan-compensated across blocks.
-// Returns the flush's cost for the schedules: the wave's steps (entries per
-// lane).
-template <int K>
-__device__ inline uint32_t flush_list_k(const float4* __restrict__ list, uint32_t ln, uint32_t sub, float ox,
-                                        float oy, float oz, float soft2, Acc3& a)
+// ------------------------------------------------- evaluating the list
+// A group of cnt bodies has S partial sums per body (list_shares), and the
+// list of a flush is cut into S shares of len consecutive entries
+// (share_len).  Virtual lane t = s cnt + b takes share s for body b, so 128
+// or 256 virtual lanes hold a group whatever its size; a wavefront (NW = 1)
+// runs them as up to four passes over the list, a block of NW wavefronts as
+// 4 / NW passes each.  Every virtual lane's sum -- FP32 FMA over blocks of 32
+// entries, Kahan-compensated across blocks and flushes -- depends on the
+// group alone, so every NW gives the same bits.  Against idle lanes taking
+// over stretches of other lanes' bodies (which this replaced) the wave steps
+// are 2% fewer (1.085 against 1.106 x the ideal on a 300k belt), with no
+// hand-over.
+__device__ inline uint32_t list_shares(uint32_t cnt)
 {
-    ln = uni(ln);
-    constexpr uint32_t span = 32u * K;
-    uint32_t e0 = 0;
-    for (; e0 + span <= ln; e0 += span) {
-        float bx = 0.f, by = 0.f, bz = 0.f;
-#pragma unroll
-        for (int u = 0; u < 32; u += 8) {
-            float4 q[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) q[k] = list[e0 + static_cast<uint32_t>(u + k) * K + sub];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) interact(q[k], ox, oy, oz, soft2, bx, by, bz);
-        }
-        a.add(bx, by, bz);
-    }
-    if (e0 < ln) {
-        float bx = 0.f, by = 0.f, bz = 0.f;
-        for (uint32_t e = e0 + sub; e < ln; e += K) interact(list[e], ox, oy, oz, soft2, bx, by, bz);
-        a.add(bx, by, bz);
-    }
-    return (ln + K - 1) / K;
+    const uint32_t s = (cnt <= 16u ? 128u : 256u) / cnt;
+    return s > 32u ? 32u : s;
 }
 
-// p[0..R) (R wave-uniform) for one body: FP32 FMA inside blocks of 32
-// entries, each block sum added into a; the last, partial block loads eight
-// entries at a time as well.
-__device__ inline void seg_sum(const float4* __restrict__ p, uint32_t R, float ox, float oy, float oz, float soft2,
-                               Acc3& a)
+// Entries per share: at least ceil(ln / S), and a length whose multiples fall
+// into different LDS banks for the shares that meet in one wavefront (16
+// entries of 16 bytes span all banks): odd for small groups, whose
+// wavefronts mix many shares, else no multiple of 8.  invS = ceil(65536 / S):
+// the quotient is exact for ln < 330 and S <= 32.  S len <= kListCap + kListPad.
+__device__ inline uint32_t share_len(uint32_t ln, uint32_t S, uint32_t invS, uint32_t cnt)
+{
+    const uint32_t len = ((ln + S - 1u) * invS) >> 16;
+    if (cnt <= 16u) return len | 1u;
+    return (cnt < 64u && (len & 7u) == 0u) ? len + 1u : len;
+}
+
+template <int N>
+__device__ inline void interact_n(const float4* __restrict__ p, float ox, float oy, float oz, float r2_0, float& bx,
+                                  float& by, float& bz)
+{
+    float4 q[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) q[k] = p[k];
+#pragma unroll
+    for (int k = 0; k < N; ++k) interact(q[k], ox, oy, oz, r2_0, bx, by, bz);
+}
+
+// p[0..len) (len wave-uniform) for one body: blocks of 32 entries, eight
+// loaded at a time, each block's FP32 sum added into a
+__device__ inline void share_sum(const float4* __restrict__ p, uint32_t len, float ox, float oy, float oz, float r2_0,
+                                 Acc3& a)
 {
     uint32_t j = 0;
-    for (; j + 32u <= R; j += 32u) {
+    while (j < len) {
+        const uint32_t end = min(len, j + 32u);
         float bx = 0.f, by = 0.f, bz = 0.f;
-#pragma unroll
-        for (int u = 0; u < 32; u += 8) {
-            float4 q[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) q[k] = p[j + static_cast<uint32_t>(u + k)];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) interact(q[k], ox, oy, oz, soft2, bx, by, bz);
+        for (; j + 8u <= end; j += 8u) interact_n<8>(p + j, ox, oy, oz, r2_0, bx, by, bz);
+        if (end - j >= 4u) {
+            interact_n<4>(p + j, ox, oy, oz, r2_0, bx, by, bz);
+            j += 4u;
         }
-        a.add(bx, by, bz);
-    }
-    if (j < R) {
-        float bx = 0.f, by = 0.f, bz = 0.f;
-        for (; j + 8u <= R; j += 8u) {
-            float4 q[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) q[k] = p[j + static_cast<uint32_t>(k)];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) interact(q[k], ox, oy, oz, soft2, bx, by, bz);
+        if (end - j >= 2u) {
+            interact_n<2>(p + j, ox, oy, oz, r2_0, bx, by, bz);
+            j += 2u;
         }
-        for (; j < R; ++j) interact(p[j], ox, oy, oz, soft2, bx, by, bz);
+        if (end - j >= 1u) {
+            interact_n<1>(p + j, ox, oy, oz, r2_0, bx, by, bz);
+            j += 1u;
+        }
         a.add(bx, by, bz);
     }
 }
 
-// Shortest share of a list, in entries, that the idle lanes of a group take
-// over: shorter shares cost more in hand-over than they save (measured on the
-// 300k walk: 16 entries +2.5%, 24 -0.5%, 32 -2.5%, 48 -2%).
-constexpr uint32_t kMinShare = 32;
-
-// One lane per body.  In a group of cnt < 64 bodies the E = 64 - cnt idle
-// lanes help: with q = ceil(cnt / E), R = floor(ln / (q + 1)) rounded down to
-// a multiple of 8 (stretches load 8 entries at a time) and T = q R, the
-// body lanes take the entries [0, T) of their body in q stretches of R, while
-// idle lane e takes [T, T + R) of bodies e, e + E, e + 2E, ... in the same
-// stretches; the body lanes then take [T + R, ln).  A helper's stretch is a
-// compensated sum of its own, handed to the body's lane by a cross-lane read
-// (body b of stretch s reads lane cnt + b - sE) and added in FP64 into
-// (rx, ry, rz), in list order.  Every body's sum depends on its group and
-// list alone.  All passes share one loop body, which keeps the kernel's code
-// within the instruction cache.  Returns the flush's cost for the schedules:
-// ln - T, the entries beyond the body lanes' stretches (the wave steps
-// ln - R).  (Chosen by measurement on the 300k learned step: counting the
-// wave's steps ordered the groups 1% worse, the whole list 1.5% worse.)
-__device__ inline uint32_t flush_list_1(const float4* __restrict__ list, uint32_t ln, uint32_t cnt, float ox, float oy,
-                                        float oz, float soft2, Acc3& a, double& rx, double& ry, double& rz)
+// The schedules' cost of a flushed list of ln entries, in wave steps of one
+// wavefront with 4, 2 or 1 lanes per body; for 33..63 bodies only the entries
+// beyond the stretches that idle lanes can take over count.  (Chosen by
+// measurement on the 300k learned step: counting every step ordered the
+// groups 1% worse, the whole list 1.5% worse.)
+constexpr uint32_t kMinShare = 32;   // shortest stretch, in entries, that counts as taken over
+__device__ inline uint32_t list_cost(uint32_t ln, uint32_t cnt)
 {
-    ln = uni(ln);
-    const uint32_t lane = __lane_id();
+    if (cnt <= 16u) return (ln + 3u) >> 2;
+    if (cnt <= 32u) return (ln + 1u) >> 1;
     const uint32_t E = 64u - cnt;
-    uint32_t q = 0, R = 0;
-    if (E > 0u) {
-        q = (cnt + E - 1u) / E;
-        R = (ln / (q + 1u)) & ~7u;
-        if (R < kMinShare) q = 0;   // no helpers: one pass over the list
-    }
-    const uint32_t T = q * R;
-    const bool helper = lane >= cnt;
-    for (uint32_t s = 0; s <= q; ++s) {
-        const bool last = s == q;   // the body lanes' rest of the list
-        const uint32_t hb = lane - cnt + s * E;   // the helper's body in stretch s
-        const bool hv = helper && !last && hb < cnt;
-        const int src = static_cast<int>(hv ? hb : lane);
-        const float px = __shfl(ox, src, 64), py = __shfl(oy, src, 64), pz = __shfl(oz, src, 64);
-        if (helper && !last) a = Acc3();
-        const uint32_t from = last ? T + (q ? R : 0u) : (helper ? T : s * R);
-        seg_sum(list + from, last ? ln - T - (q ? R : 0u) : R, px, py, pz, soft2, a);
-        if (!last) {
-            // bodies sE .. sE + E - 1 take their stretch from lanes cnt .. cnt + E - 1
-            const bool own = !helper && lane >= s * E && lane < s * E + E;
-            const int from_lane = static_cast<int>(own ? cnt + lane - s * E : lane);
-            const double gx = __shfl(static_cast<double>(a.sx) - static_cast<double>(a.cx), from_lane, 64);
-            const double gy = __shfl(static_cast<double>(a.sy) - static_cast<double>(a.cy), from_lane, 64);
-            const double gz = __shfl(static_cast<double>(a.sz) - static_cast<double>(a.cz), from_lane, 64);
-            if (own) {
-                rx += gx;
-                ry += gy;
-                rz += gz;
-            }
-        }
-    }
-    return ln - T;
+    if (E == 0u) return ln;
+    const uint32_t q = (cnt + E - 1u) / E;
+    const uint32_t R = (ln / (q + 1u)) & ~7u;
+    return R < kMinShare ? ln : ln - q * R;
 }
 
-// K (wave-uniform) = lanes per body: 4 for groups of <= 16 bodies, 2 for
-// <= 32, else 1 (then the lanes past the group's bodies help), so small
-// groups keep every lane busy.
-__device__ inline uint32_t flush_list(const float4* __restrict__ list, uint32_t ln, uint32_t K, uint32_t sub,
-                                      uint32_t cnt, float ox, float oy, float oz, float soft2, Acc3& a, double& rx,
-                                      double& ry, double& rz)
+// A round's ranges, one per lane in the order of the pop: range r holds the
+// slots [excl, excl + count) of the round, and its slot s stands for the node
+// (or body) info + s.
+struct Ranges {
+    uint32_t info, excl, count, total;   // total: the round's slots (wave-uniform)
+};
+constexpr int kRoundSlots = 512;   // 64 ranges of at most 8
+
+// A lone wavefront writes out the entries of a whole round at once ...
+__device__ inline void write_slots(const Ranges& r, uint32_t* slots)
 {
-    if (K == 4) return flush_list_k<4>(list, ln, sub, ox, oy, oz, soft2, a);
-    if (K == 2) return flush_list_k<2>(list, ln, sub, ox, oy, oz, soft2, a);
-    return flush_list_1(list, ln, cnt, ox, oy, oz, soft2, a, rx, ry, rz);
+    const uint32_t e = r.info + r.excl;
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; ++k)
+        if (k < r.count) slots[r.excl + k] = e + k;
+    __builtin_amdgcn_wave_barrier();
 }
 
-constexpr int kNodeBuf = 512;    // nodes of one round (<= 64 ranges of <= 8)
-
-// Entry s of a round (ent) and, for a node entry, its node; a zero node (no
-// mass: never used) for body entries and past the round's end.
-__device__ inline MNode fetch_node(const MixedBuffers& mb, const uint32_t* nbuf, uint32_t s, uint32_t total,
-                                   uint32_t& ent)
+// ... wavefronts that share a round find each of their own 64: the entry of
+// slot sb + lane belongs to the last range that starts at or before it, found
+// by marking the starts that fall into the 64 slots (mark: 64 words of the
+// wavefront's own) and a running maximum of their lanes.
+__device__ inline uint32_t slot_entry(const Ranges& r, uint32_t sb, uint32_t* mark)
 {
-    MNode nd{};
-    ent = s < total ? nbuf[s] : 0u;
-    if (s < total && !(ent & 0x80000000u)) nd = mb.node[ent & 0x7fffffffu];
-    return nd;
+    const uint32_t lane = __lane_id();
+    const uint32_t at = r.excl - sb;
+    const uint32_t before = static_cast<uint32_t>(__popcll(__ballot(r.count != 0u && r.excl < sb)));
+    mark[lane] = 0u;
+    __builtin_amdgcn_wave_barrier();
+    if (r.count != 0u && at < 64u) mark[at] = lane + 1u;
+    __builtin_amdgcn_wave_barrier();
+    int x = static_cast<int>(mark[lane]);
+    __builtin_amdgcn_wave_barrier();
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
+    x = max(x, static_cast<int>(before));
+    const uint32_t s = sb + lane;
+    const uint32_t e = static_cast<uint32_t>(__shfl(static_cast<int>(r.info), x - 1, 64)) + s;
+    return s < r.total ? e : 0u;
+}
+
+// Entry of slot sb + lane (0 past the round's end) and its node, a zero node
+// (no mass: never used) for a body entry and past the end.
+template <int NW>
+__device__ inline uint32_t fetch_slot(const Ranges& r, uint32_t sb, uint32_t* slots, const MNode* __restrict__ nodes,
+                                      MNode& nd)
+{
+    const uint32_t s = sb + __lane_id();
+    uint32_t ent = 0u;
+    if (NW == 1) {
+        if (s < r.total) ent = slots[s];
+    } else {
+        ent = slot_entry(r, sb, slots);
+    }
+    nd = MNode{};
+    if (s < r.total && !(ent & 0x80000000u)) nd = nodes[ent];
+    return ent;
+}
+
+// Waits for the block's other wavefronts; a lone wavefront needs no
+// barrier (its LDS accesses stay in order), only that the compiler keeps them
+// in place.
+template <int NW>
+__device__ inline void group_sync()
+{
+    if (NW == 1) __builtin_amdgcn_wave_barrier();
+    else __syncthreads();
+}
+
+// Key order: entry t of part x is group (t / R * P + x) * R + t % R, increasing
+// in t, so the first t past the end closes x.  The part's blocks hold its first
+// part_blocks entries; the queue hands out the rest.
+__device__ inline uint32_t part_group(uint32_t x, uint32_t t)
+{
+    const uint64_t q = (static_cast<uint64_t>(t / kWalkRun) * kWalkParts + x) * kWalkRun + t % kWalkRun;
+    return q < kNone ? static_cast<uint32_t>(q) : kNone;
+}
+__device__ inline uint32_t part_blocks(uint32_t x, uint32_t nblk)
+{
+    return nblk > x ? (nblk - x + kWalkParts - 1) / kWalkParts : 0u;
 }
 
 // Accelerations of the heavy bodies: an FP64 direct sum over every other
@@ -697,21 +758,28 @@ __device__ inline double rsqrt_f64(double x)
 // k_heavy_final adds the chunk partials in chunk order.  A system's heavy
 // accelerations therefore depend on that system alone, not on the launch
 // shape or on the other systems of an ensemble.
-__device__ inline void heavy_item(const Bodies& b, const TreeBuffers& tb, const MixedBuffers& mb, const MixedParams& p,
-                                  uint32_t item, int lane, double (*part)[64])
+struct HeavyArgs {
+    const double *px, *py, *pz, *m;
+    const SysScalars* sys;
+    uint32_t n_sys;
+    double* hpart;
+    double soft2, G;
+};
+
+__device__ inline void heavy_item(const HeavyArgs& ha, uint32_t item, int lane, double (*part)[64])
 {
-    uint32_t lo = 0, hi = tb.n_sys;   // the last system whose first item is <= item
+    uint32_t lo = 0, hi = ha.n_sys;   // the last system whose first item is <= item
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (tb.sys[mid].heavy_item <= item) lo = mid;
+        if (ha.sys[mid].heavy_item <= item) lo = mid;
         else hi = mid;
     }
-    const SysScalars* sy = tb.sys + lo;
+    const SysScalars* sy = ha.sys + lo;
     const uint32_t r = item - sy->heavy_item;
     const uint32_t k = r / sy->heavy_chunks, c = r % sy->heavy_chunks;
     if (k >= sy->n_heavy) return;
     const uint32_t h = sy->heavy_slot[k];
-    const double x = b.px[h], y = b.py[h], z = b.pz[h];
+    const double x = ha.px[h], y = ha.py[h], z = ha.pz[h];
     const size_t j0 = sy->body_lo + static_cast<size_t>(c) * kHeavyChunk;
     const size_t j1 = min(j0 + kHeavyChunk, static_cast<size_t>(sy->body_hi));
     Neumaier ax, ay, az;
@@ -720,10 +788,10 @@ __device__ inline void heavy_item(const Bodies& b, const TreeBuffers& tb, const 
     // square roots and divisions of consecutive bodies overlap
 #pragma unroll 4
     for (size_t j = j0 + lane; j < j1; j += 64) {
-        const double dx = b.px[j] - x, dy = b.py[j] - y, dz = b.pz[j] - z;
-        const double r2 = dx * dx + dy * dy + dz * dz + p.soft2;
+        const double dx = ha.px[j] - x, dy = ha.py[j] - y, dz = ha.pz[j] - z;
+        const double r2 = dx * dx + dy * dy + dz * dz + ha.soft2;
         const double invR = rsqrt_f64(r2);
-        const double s = (j != h && r2 > 0.0) ? p.G * b.m[j] * (invR * invR * invR) : 0.0;
+        const double s = (j != h && r2 > 0.0) ? ha.G * ha.m[j] * (invR * invR * invR) : 0.0;
         ax.add(s * dx);
         ay.add(s * dy);
         az.add(s * dz);
@@ -735,313 +803,555 @@ __device__ inline void heavy_item(const Bodies& b, const TreeBuffers& tb, const 
     if (lane < 3) {
         Neumaier t;
         for (int q = 0; q < 64; ++q) t.add(part[lane][q]);
-        mb.hpart[3 * static_cast<size_t>(item) + lane] = t.value();
+        ha.hpart[3 * static_cast<size_t>(item) + lane] = t.value();
     }
     __builtin_amdgcn_wave_barrier();
 }
 
-// 157 VGPRs: 3 waves per SIMD (held there by amdgpu_waves_per_eu).  Capping
-// at 128 for 4 waves measured 1% slower on the 300k walk and 4% faster at 2M
-// (the list loop needs its registers).
-__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3))) void k_walk_mixed(Bodies b, size_t n, TreeBuffers tb, MixedBuffers mb,
-                                                    MixedParams p)
+// The walk of a group, by one wavefront (NW = 1) or by the four of a block
+// (NW = 4): each round's nodes 64 per wavefront, the list's virtual lanes 64
+// per wavefront.  The order of the nodes, the list and its flushes, and every
+// sum are the same for both, so the results are the same bits.
+//
+// The arguments (some 70 pointers and scalars) are read from the kernel's
+// argument segment where a stage needs them: held in scalar registers across
+// the whole loop they were spilled to vector registers (100 spills).
+struct WalkArgs {
+    Bodies b;
+    TreeBuffers tb;
+    MixedBuffers mb;
+    MixedParams p;
+};
+using WalkArgsP = const __attribute__((address_space(4))) WalkArgs*;
+
+// the arguments, read again after this point (the compiler cannot tell that
+// the address is the same, so it does not keep earlier loads alive)
+__device__ inline WalkArgsP args_here(WalkArgsP a)
 {
-    __shared__ float4 s_list[kWaves][kListCap];
-    __shared__ uint32_t s_stack[kWaves][kStackCap];
-    __shared__ uint32_t s_nodes[kWaves][kNodeBuf];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    float4* list = s_list[w];
-    uint32_t* stk = s_stack[w];
-    uint32_t* nbuf = s_nodes[w];
-    const uint32_t G = tb.sc->n_groups;
-    const uint32_t worker = blockIdx.x * kWaves + w;
-    const float soft2f = static_cast<float>(p.soft2);
-    const double theta2 = p.theta2;
-    uint32_t pos = 0, end = 0;   // the current chunk's groups (sched 2)
+    asm volatile("" : "+s"(a));
+    return a;
+}
+
+// Body j as a list entry of a group centred on (cx, cy, cz); false (q left
+// alone) for a heavy or massless body.
+__device__ inline bool body_entry(WalkArgsP a, uint32_t j, double cx, double cy, double cz, float4& q)
+{
+    const double m = a->b.m[j];
+    if (a->b.hrank[j] >= 0 || m == 0.0) return false;
+    q = make_float4(static_cast<float>(a->b.px[j] - cx), static_cast<float>(a->b.py[j] - cy),
+                    static_cast<float>(a->b.pz[j] - cz), static_cast<float>(a->p.G * m));
+    return true;
+}
+
+// LDS of a block: four wavefronts' own, or one shared group's, over it.
+// The list (with its padding), then the words of write_slots or 64 per
+// wavefront for slot_entry, then the stack; the sums that are exchanged (256
+// doubles, 768 between wavefronts) lie over the first two.
+constexpr int kListBytes = (kListCap + kListPad) * 16;
+constexpr int kWaveLds = kListBytes + kRoundSlots * 4 + kStackCap * 4;
+static_assert(kListBytes + kRoundSlots * 4 >= 768 * 8, "the exchanged sums fit");
+
+// Walks group g by NW wavefronts (1: this one alone; 4: the block's, this one
+// the w-th) and returns its work.  turn_no: exchanges so far (which of the two
+// rows of s_word is next).
+template <int NW>
+__device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, uint32_t g, int w, int lane,
+                                           unsigned char* lds, uint32_t (*s_word)[kWaves], uint32_t& turn_no)
+{
+    constexpr int V = 4 / NW;   // passes over a list: virtual wavefronts w, w + NW, ... of the group's four
+    const uint32_t tid = static_cast<uint32_t>(w * 64 + lane);
+    float4* list = reinterpret_cast<float4*>(lds);
+    uint32_t* slots = reinterpret_cast<uint32_t*>(lds + kListBytes) + w * 64;
+    uint32_t* stk = reinterpret_cast<uint32_t*>(lds + kListBytes + kRoundSlots * 4);
+    double* part_sum = reinterpret_cast<double*>(lds);
+            const uint64_t t_start = wall_clock64();
+            const WalkArgsP ag = args_here(args);
+            const uint32_t b0 = uni(ag->mb.gfirst[g]);
+            const uint32_t cnt = uni(ag->mb.gfirst[g + 1]) - b0;
+            // lane = body for the box, the heavy bodies and the results
+            const bool valid = static_cast<uint32_t>(lane) < cnt;
+            const uint32_t i = b0 + (valid ? static_cast<uint32_t>(lane) : 0u);
+            const double x = ag->b.px[i], y = ag->b.py[i], z = ag->b.pz[i];
+            // virtual lanes: share and body of pass v (share >> 8 | body; a lane
+            // past the last share repeats share 0 and its sum is never read)
+            const uint32_t S = list_shares(cnt), invS = (65535u + S) / S;
+            uint32_t vl[V];
+    #pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const uint32_t t = static_cast<uint32_t>((v * NW + w) * 64 + lane);
+                const uint32_t sh = t / cnt;
+                vl[v] = (t - sh * cnt) | ((sh < S ? sh : 0u) << 8);
+            }
+            const double lox = wave_min(x), loy = wave_min(y), loz = wave_min(z);
+            const double hix = wave_max(x), hiy = wave_max(y), hiz = wave_max(z);
+            const double cx = 0.5 * (lox + hix), cy = 0.5 * (loy + hiy), cz = 0.5 * (loz + hiz);
+            const double hx = 0.5 * (hix - lox), hy = 0.5 * (hiy - loy), hz = 0.5 * (hiz - loz);
+            const float ox = static_cast<float>(x - cx);
+            const float oy = static_cast<float>(y - cy);
+            const float oz = static_cast<float>(z - cz);
+            Acc3 acc[V];
+            uint32_t ln = 0, sp = 1, n_inter = 0, n_visit = 0, n_steps = 0;
+            bool overflow = false;
+            const uint32_t gsys = ag->tb.n_sys == 1 ? 0u : uni(ag->tb.bsys[b0]);
+            const MNode* __restrict__ nodes = ag->mb.node;
+            const float r2_0 = list_r2_floor(nodes[gsys].gm, static_cast<float>(ag->p.soft2));   // the system's root
+            // heavy bodies of the system: FP64 direct sum, the ranks k = q mod 4 in
+            // rank order into partial q (one or more of the four per wavefront),
+            // the partials added in order
+            double hax = 0.0, hay = 0.0, haz = 0.0;
+            {
+                const SysScalars* sy = ag->tb.sys + gsys;
+                const uint32_t nh = sy->n_heavy;
+                const double soft2 = ag->p.soft2, grav = ag->p.G;
+                // lane k loads heavy body k (one load latency for all of them); the
+                // loop reads them back as wave constants
+                uint32_t hj = kNone;
+                double hpx = 0.0, hpy = 0.0, hpz = 0.0, hpm = 0.0;
+                if (static_cast<uint32_t>(lane) < nh) {
+                    hj = sy->heavy_slot[lane];
+                    hpx = ag->b.px[hj];
+                    hpy = ag->b.py[hj];
+                    hpz = ag->b.pz[hj];
+                    hpm = ag->b.m[hj];
+                }
+    #pragma unroll 1
+                for (int v = 0; v < V; ++v) {
+                    double sx = 0.0, sy_ = 0.0, sz = 0.0;
+                    for (uint32_t k = static_cast<uint32_t>(v * NW + w); k < nh; k += 4u) {
+                        const uint32_t j = lane_u32(hj, k);
+                        const double dx = lane_f64(hpx, k) - x, dy = lane_f64(hpy, k) - y, dz = lane_f64(hpz, k) - z;
+                        const double r2 = dx * dx + dy * dy + dz * dz + soft2;
+                        const bool pair = j != i && r2 > 0.0;
+                        const bool in_range = (r2 >= 0x1p-767) & (r2 <= 0x1p+1000);
+                        const double invR = __all(in_range | !pair) ? inv_sqrt_in_range(pair ? r2 : 1.0)
+                                                                    : 1.0 / sqrt(pair ? r2 : 1.0);
+                        const double s = grav * lane_f64(hpm, k) * (invR * invR * invR);
+                        if (pair) {
+                            sx += s * dx;
+                            sy_ += s * dy;
+                            sz += s * dz;
+                        }
+                    }
+                    if (NW == 1) {
+                        hax += sx;
+                        hay += sy_;
+                        haz += sz;
+                    } else {
+                        double* q = part_sum + (v * NW + w) * 192 + lane;
+                        q[0] = sx;
+                        q[64] = sy_;
+                        q[128] = sz;
+                    }
+                }
+            }
+            if (NW > 1) {
+                __syncthreads();
+                for (int q = 0; q < 4; ++q) {
+                    hax += part_sum[q * 192 + lane];
+                    hay += part_sum[q * 192 + 64 + lane];
+                    haz += part_sum[q * 192 + 128 + lane];
+                }
+            }
+            // relative opening test: a node is also opened while its quadrupole
+            // scale G Q / D^4 exceeds alpha x the smallest heavy-body acceleration
+            // of the group (the acceleration every body of these systems is made of)
+            const double ah = valid ? sqrt(hax * hax + hay * hay + haz * haz) : INFINITY;
+            const double aref = wave_min(ah);
+            const double alpha = ag->p.alpha, theta2 = ag->p.theta2;
+            const double qlim = (alpha > 0.0 && aref > 0.0 && aref < INFINITY) ? alpha * aref : INFINITY;
+            // up to theta^2 = kSafe2 (and without a limit) the extent test implies the rest
+            const bool relative = theta2 > kSafe2 && __any(qlim < INFINITY);
+            if (tid == 0) stk[0] = stack_range(gsys, 1, false);   // the root of the group's system
+            group_sync<NW>();   // (also: every wavefront has read the exchanged sums)
+            for (bool last = false; !last;) {
+                // pop up to 64 ranges, one per lane, while the stack cannot
+                // overflow; when it is empty one more turn flushes the rest of the list
+                last = sp == 0u || overflow;
+                Ranges r{0u, 0u, 0u, 0u};
+                if (!last) {
+                    const uint32_t P = (sp <= static_cast<uint32_t>(kBigPopLimit)) ? min(sp, 64u) : 1u;
+                    const bool has = static_cast<uint32_t>(lane) < P;
+                    const uint32_t e = has ? stk[sp - 1 - lane] : 0u;
+                    sp -= P;
+                    r.count = has ? ((e >> 27) & 7u) + 1u : 0u;
+                    const uint32_t incl = wave_incl_scan(r.count);
+                    r.total = lane_u32(incl, 63);
+                    r.excl = incl - r.count;
+                    r.info = (e & 0x87ffffffu) - r.excl;
+                    n_visit += r.total;
+                    if (NW == 1) write_slots(r, slots);
+                }
+                uint32_t ent = 0u;
+                MNode nd{};
+                if (static_cast<uint32_t>(w) * 64u < r.total) ent = fetch_slot<NW>(r, static_cast<uint32_t>(w) * 64u, slots, nodes, nd);
+                uint32_t base = 0;
+                do {
+                    // the opening test; a leaf of one body is always accepted, one
+                    // of several never (its bodies are), and lanes without a node
+                    // have no mass
+                    const double rx = nd.x - cx, ry = nd.y - cy, rz = nd.z - cz;
+                    const double ex = fmax(fabs(rx) - hx, 0.0);
+                    const double ey = fmax(fabs(ry) - hy, 0.0);
+                    const double ez = fmax(fabs(rz) - hz, 0.0);
+                    const double d2 = ex * ex + ey * ey + ez * ez;
+                    bool pass = nd.size2 < theta2 * d2;
+                    if (relative) pass &= nd.size2 <= kSafe2 * d2 || static_cast<double>(nd.gq) <= qlim * (d2 * d2);
+                    const bool live = nd.gm != 0.f;
+                    const uint32_t push = nd.push, info = nd.info;
+                    bool app = live && (pass || info == (kMLeaf | 1u));
+                    const bool open = live && !app;
+                    const bool open_big = open && info > (kMLeaf | 8u);
+                    float4 q = make_float4(static_cast<float>(rx), static_cast<float>(ry), static_cast<float>(rz), nd.gm);
+                    if (static_cast<int32_t>(ent) < 0) app = body_entry(args_here(args), ent & 0x7fffffffu, cx, cy, cz, q);
+                    // the next chunk's nodes are on their way while this chunk is
+                    // listed (without the prefetch: +4% on the 300k walk)
+                    const uint32_t sb_n = base + static_cast<uint32_t>((NW + w) * 64);
+                    ent = 0u;
+                    nd.gm = 0.f;
+                    if (sb_n < r.total) ent = fetch_slot<NW>(r, sb_n, slots, nodes, nd);
+                    // list entries and stack pushes of this chunk (one per lane at
+                    // most), and leaves of more than 8 co-keyed bodies (see below)
+                    uint64_t am = __ballot(app);
+                    const uint64_t pm = __ballot(open && !open_big);
+                    uint64_t big = __ballot(open_big);
+                    // counts: entries | pushes << 10 | chunks with such leaves << 20,
+                    // of all NW chunks and of those before this wavefront's
+                    const uint32_t word = static_cast<uint32_t>(__popcll(am)) |
+                                          static_cast<uint32_t>(__popcll(pm)) << 10 | (big ? 1u << 20 : 0u);
+                    uint32_t all = word, before = 0;
+                    uint32_t* const row = s_word[turn_no & 1u];
+                    if (NW > 1) {
+                        if (lane == 0) row[w] = word;
+                        __syncthreads();
+                        ++turn_no;
+                        all = 0;
+    #pragma unroll
+                        for (int c = 0; c < NW; ++c) {
+                            const uint32_t v = row[c];
+                            before += c < w ? v : 0u;
+                            all += v;
+                        }
+                        all = uni(all);
+                        before = uni(before);
+                    }
+                    const uint32_t need = (all >> 10) & 0x3ffu;
+                    if (sp + need > static_cast<uint32_t>(kStackCap)) {
+                        if (tid == 0) atomicOr(&sc->error, kErrStack);
+                        overflow = true;
+                    } else {
+                        // one range per opened node or leaf of at most 8 bodies
+                        if (open && !open_big) stk[sp + ((before >> 10) & 0x3ffu) + rank_below(pm)] = push;
+                        sp += need;
+                    }
+                    if (!last && all < (1u << 20) && ln + (all & 0x3ffu) <= static_cast<uint32_t>(kListCap)) {
+                        if (app) list[ln + (before & 0x3ffu) + rank_below(am)] = q;
+                        ln += all & 0x3ffu;
+                        n_inter += all & 0x3ffu;
+                    } else {
+                        // The list is flushed before the chunk that does not fit (and
+                        // at the end).  A leaf of more than 8 co-keyed bodies
+                        // (duplicate or nearly coincident positions) puts its bodies
+                        // on the list directly, 64 at a time, so the stack does not
+                        // grow with its size: while a round holds such leaves its
+                        // chunks take turns, wavefront `turn` appending its entries,
+                        // then its leaves' bodies.
+                        const bool turns = all >= (1u << 20);
+                        uint32_t turn = 0, big_k0 = 0;
+                        for (bool more = true, first = true; more; first = false) {
+                            uint32_t words[NW];   // entries of each chunk, | 1 << 20 while its leaves have bodies left
+                            const bool mine = !turns || turn == static_cast<uint32_t>(w);
+                            am = __ballot(app && mine);
+                            if (NW == 1) {
+                                words[0] = static_cast<uint32_t>(__popcll(am)) | (big ? 1u << 20 : 0u);
+                            } else if (first) {
+    #pragma unroll
+                                for (int c = 0; c < NW; ++c)
+                                    words[c] = !turns || c == 0 ? uni(row[c]) & 0x1003ffu : 0u;
+                            } else {
+                                uint32_t* const rw = s_word[turn_no & 1u];
+                                if (lane == 0)
+                                    rw[w] = static_cast<uint32_t>(__popcll(am)) | (mine && big ? 1u << 20 : 0u);
+                                __syncthreads();
+                                ++turn_no;
+    #pragma unroll
+                                for (int c = 0; c < NW; ++c) words[c] = uni(rw[c]);
+                            }
+                            for (int c0 = 0;;) {
+                                uint32_t l1 = ln, at = 0;
+                                int c1 = c0;
+    #pragma unroll
+                                for (int c = 0; c < NW; ++c) {
+                                    if (c >= c0 && c == c1 && l1 + (words[c] & 0x3ffu) <= static_cast<uint32_t>(kListCap)) {
+                                        if (c == w) at = l1;
+                                        l1 += words[c] & 0x3ffu;
+                                        ++c1;
+                                    }
+                                }
+                                if (w >= c0 && w < c1 && ((am >> lane) & 1u)) list[at + rank_below(am)] = q;
+                                n_inter += l1 - ln;
+                                ln = l1;
+                                c0 = c1;
+                                if (c0 == NW && !last) break;
+                                // flush: padded with entries of no mass to S shares
+                                const uint32_t len = share_len(ln, S, invS, cnt);
+                                if (tid < 64 && ln + static_cast<uint32_t>(lane) < S * len)
+                                    list[ln + static_cast<uint32_t>(lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
+                                group_sync<NW>();
+    #pragma unroll
+                                for (int v = 0; v < V; ++v) {
+                                    if (static_cast<uint32_t>((v * NW + w) * 64) < S * cnt) {
+                                        const int src = static_cast<int>(vl[v] & 0xffu);
+                                        share_sum(list + (vl[v] >> 8) * len, len, __shfl(ox, src, 64), __shfl(oy, src, 64),
+                                                  __shfl(oz, src, 64), r2_0, acc[v]);
+                                    }
+                                }
+                                n_steps += list_cost(ln, cnt);
+                                group_sync<NW>();
+                                ln = 0;
+                                if (c0 == NW) break;
+                            }
+                            more = turns;
+                            if (turns) {
+                                // the next 64 bodies of this turn's leaves, or the next turn
+                                if ((words[turn] >> 20) != 0u) {
+                                    if (turn == static_cast<uint32_t>(w)) {
+                                        const uint32_t l = static_cast<uint32_t>(__builtin_ctzll(big));
+                                        const uint32_t j0 = lane_u32(push, l) & 0x07ffffffu, c = lane_u32(info, l) & ~kMLeaf;
+                                        const uint32_t j = j0 + big_k0 + static_cast<uint32_t>(lane);
+                                        app = j < j0 + c && body_entry(args_here(args), j, cx, cy, cz, q);
+                                        big_k0 += 64u;
+                                        if (big_k0 >= c) {
+                                            big_k0 = 0;
+                                            big &= big - 1;
+                                        }
+                                    }
+                                } else {
+                                    more = ++turn < static_cast<uint32_t>(NW);
+                                }
+                            }
+                        }
+                    }
+                    base += NW * 64u;
+                } while (base < r.total && !overflow);
+                group_sync<NW>();   // the next round reads the stack
+            }
+            // the virtual lanes' sums (a Kahan sum's value is s - c: c holds the
+            // negative of the rounding lost), added in FP64 in share order
+            double lacc[3];
+            if (NW == 1) {
+    #pragma unroll
+                for (int a = 0; a < 3; ++a) {
+    #pragma unroll
+                    for (int v = 0; v < V; ++v)
+                        part_sum[v * 64 + lane] = static_cast<double>(a == 0 ? acc[v].sx : (a == 1 ? acc[v].sy : acc[v].sz)) -
+                                                  static_cast<double>(a == 0 ? acc[v].cx : (a == 1 ? acc[v].cy : acc[v].cz));
+                    __builtin_amdgcn_wave_barrier();
+                    double t = 0.0;
+                    for (uint32_t k = 0; k < S; ++k) t += part_sum[k * cnt + (valid ? lane : 0)];
+                    lacc[a] = t;
+                    __builtin_amdgcn_wave_barrier();
+                }
+            } else {
+    #pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    double* q = part_sum + (v * NW + w) * 64 + lane;
+                    q[0] = static_cast<double>(acc[v].sx) - static_cast<double>(acc[v].cx);
+                    q[256] = static_cast<double>(acc[v].sy) - static_cast<double>(acc[v].cy);
+                    q[512] = static_cast<double>(acc[v].sz) - static_cast<double>(acc[v].cz);
+                }
+                __syncthreads();
+    #pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    double t = 0.0;
+                    if (a % NW == w)
+                        for (uint32_t k = 0; k < S; ++k) t += part_sum[a * 256 + k * cnt + (valid ? lane : 0)];
+                    lacc[a] = t;
+                }
+            }
+            // heavy bodies take their accelerations from k_heavy_direct instead;
+            // axis a is written by wavefront a mod NW
+            const WalkArgsP ae = args_here(args);
+            const uint32_t work = n_steps + n_visit / 2u;
+            if (valid && ae->b.hrank[i] < 0) {
+                const bool kick = ae->p.kick != 0;
+                const double half_dt = ae->p.half_dt;
+                const double ax = hax + lacc[0];
+                const double ay = hay + lacc[1];
+                const double az = haz + lacc[2];
+                if (0 % NW == w) {
+                    ae->b.ax[i] = ax;
+                    if (kick) ae->b.vx[i] = ae->b.vx[i] + half_dt * ax;
+                }
+                if (1 % NW == w) {
+                    ae->b.ay[i] = ay;
+                    if (kick) ae->b.vy[i] = ae->b.vy[i] + half_dt * ay;
+                }
+                if (2 % NW == w) {
+                    ae->b.az[i] = az;
+                    if (kick) ae->b.vz[i] = ae->b.vz[i] + half_dt * az;
+                }
+            }
+            // the group's work, the schedules' cost unit: the flushes' costs plus
+            // half the visits (a visit measured half the time of a list step on
+            // the 300k walk)
+            if (valid && w == 0) ae->b.pcost[i] = work;
+            if (tid == 0) {
+                ae->mb.g_inter[g] = n_inter;
+                ae->mb.g_visit[g] = n_visit;
+                ae->mb.g_work[g] = work;
+                ae->mb.g_t0[g] = t_start;
+                ae->mb.g_t1[g] = wall_clock64();
+                ae->mb.g_worker[g] = blockIdx.x * kWaves + static_cast<uint32_t>(w);
+            }
+            group_sync<NW>();   // the next group writes the exchanged sums and the list
+    return work;
+}
+
+__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3))) void k_walk_mixed(WalkArgs)
+{
+    const WalkArgsP args = (WalkArgsP)__builtin_amdgcn_kernarg_segment_ptr();
+    __shared__ __attribute__((aligned(16))) unsigned char s_mem[kWaves * kWaveLds];
+    __shared__ __attribute__((aligned(16))) uint32_t s_word[2][kWaves];
+    __shared__ uint32_t s_take;
+    const int w = static_cast<int>(uni(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    StepScalars* const sc = args->tb.sc;
+    const uint32_t G = sc->n_groups;
+    const uint32_t nblk = gridDim.x, waves = nblk * kWaves;
     // heaviest-first order pays while the tail decides the walk (few groups
     // per worker); with many groups per worker the key order's locality wins
     // (measured crossover between 8 and 33 groups per worker wave)
-    const bool use_order = p.sched == 1 && G <= p.order_max_groups;
-    // this XCD's runs of the queue first, then those of the following parts
-    uint32_t part = blockIdx.x % kWalkParts, parts_left = kWalkParts;
-    for (;;) {
-        uint32_t g;
-        if (p.sched == 2) {
-            // balanced chunks of consecutive groups, served by a dynamic queue;
-            // every take consumes a chunk, so the loop ends after n_chunks takes
-            while (pos >= end) {
-                uint32_t q = 0;
-                if (lane == 0) q = atomicAdd(&tb.sc->group_counter, 1u);
-                q = uni(q);
-                if (q >= p.n_chunks) break;
-                pos = uni(mb.chunk[q]);
-                end = uni(mb.chunk[q + 1]);
-            }
-            if (pos >= end) break;
-            g = pos++;
-        } else if (use_order) {
-            // heaviest first from one queue: dealing the order out per XCD
-            // measured 23% slower on the 300k walk (its span grows)
-            uint32_t q = 0;
-            if (lane == 0) q = atomicAdd(&tb.sc->group_counter, 1u);
-            q = uni(q);
-            if (q >= G) break;
-            g = mb.order[q];
+    const int sched = args->p.sched;
+    const bool use_order = sched == 1 && G <= args->p.order_max_groups;
+    // First the groups that are shared: order[0..C) in the cost order, the
+    // list of k_mixed_nodes in key order; without a previous walk every group
+    // of a small system (2 a block) and none of a larger one.  Every block's
+    // first group is fixed by its place, and blocks ask the queue only after
+    // that, so a system with fewer groups than blocks takes no atomic at all.
+    // (With every take an atomic, 3,072 waves each closing eight queues on
+    // one cache line held up the loads of the 561 waves that had a group for
+    // 100 of the 336 us of a 19k walk.)
+    uint32_t C = 0;
+    bool listed = false;   // the shared groups come from a list, not 0..C-1
+    if (sched != 2) {
+        if (sc->work_prev == 0u) {
+            C = G <= 2u * nblk ? G : 0u;
+            listed = use_order;
         } else {
-            // key order, dealt out per XCD (5% shorter on the 300k walk, 4%
-            // on a 32-system ensemble): the t-th entry of part x is group
-            // (t / R * P + x) * R + t % R, increasing in t, so the first t
-            // past the end closes x
-            uint32_t q = 0;
-            bool got = false;
-            while (parts_left > 0) {
-                uint32_t t = 0;
-                if (lane == 0) t = atomicAdd(&tb.sc->part_counter[part], 1u);
-                t = uni(t);
-                const uint64_t qq = (static_cast<uint64_t>(t / kWalkRun) * kWalkParts + part) * kWalkRun + t % kWalkRun;
-                if (qq < G) {
-                    q = static_cast<uint32_t>(qq);
-                    got = true;
-                    break;
-                }
-                part = (part + 1) % kWalkParts;
-                --parts_left;
-            }
-            if (!got) break;
-            g = q;
-        }
-        g = uni(g);
-        if (g >= G) continue;   // a schedule entry outside the groups of this step
-        const uint64_t t_start = wall_clock64();
-        const uint32_t b0 = mb.gfirst[g];
-        const uint32_t cnt = mb.gfirst[g + 1] - b0;
-        // K lanes per body: lane = sub * (64 / K) + body
-        const uint32_t K = cnt <= 16u ? 4u : (cnt <= 32u ? 2u : 1u);
-        const uint32_t per = 64u / K;
-        const uint32_t bl = static_cast<uint32_t>(lane) % per, sub = static_cast<uint32_t>(lane) / per;
-        const bool valid = bl < cnt;
-        const uint32_t i = b0 + (valid ? bl : 0u);
-        const double x = b.px[i], y = b.py[i], z = b.pz[i];
-        const double lox = wave_min(x), loy = wave_min(y), loz = wave_min(z);
-        const double hix = wave_max(x), hiy = wave_max(y), hiz = wave_max(z);
-        const double cx = 0.5 * (lox + hix), cy = 0.5 * (loy + hiy), cz = 0.5 * (loz + hiz);
-        const double hx = 0.5 * (hix - lox), hy = 0.5 * (hiy - loy), hz = 0.5 * (hiz - loz);
-        const float ox = static_cast<float>(x - cx);
-        const float oy = static_cast<float>(y - cy);
-        const float oz = static_cast<float>(z - cz);
-        Acc3 acc;
-        double rx = 0.0, ry = 0.0, rz = 0.0;   // the helpers' stretches (one lane per body)
-        uint32_t ln = 0, sp = 1, n_inter = 0, n_visit = 0, n_steps = 0;
-        bool overflow = false;
-        const uint32_t gsys = tb.bsys[b0];
-        const float r2_0 = list_r2_floor(mb.node[gsys].gm, soft2f);   // the system's root
-        // heavy bodies of the system: FP64 direct sum in rank order
-        double hax = 0.0, hay = 0.0, haz = 0.0;
-        const SysScalars* sy = tb.sys + gsys;
-        const uint32_t nh = sy->n_heavy;
-        // lane k loads heavy body k (one load latency for all of them); the
-        // loop reads them back as wave constants
-        uint32_t hj = kNone;
-        double hpx = 0.0, hpy = 0.0, hpz = 0.0, hpm = 0.0;
-        if (static_cast<uint32_t>(lane) < nh) {
-            hj = sy->heavy_slot[lane];
-            hpx = b.px[hj];
-            hpy = b.py[hj];
-            hpz = b.pz[hj];
-            hpm = b.m[hj];
-        }
-        for (uint32_t k = 0; k < nh; ++k) {
-            const uint32_t j = lane_u32(hj, k);
-            if (j == i) continue;
-            const double dx = lane_f64(hpx, k) - x, dy = lane_f64(hpy, k) - y, dz = lane_f64(hpz, k) - z;
-            const double r2 = dx * dx + dy * dy + dz * dz + p.soft2;
-            if (!(r2 > 0.0)) continue;
-            const double invR = 1.0 / sqrt(r2);
-            const double s = p.G * lane_f64(hpm, k) * (invR * invR * invR);
-            hax += s * dx;
-            hay += s * dy;
-            haz += s * dz;
-        }
-        // relative opening test: a node is also opened while its quadrupole
-        // scale G Q / D^4 exceeds alpha x the smallest heavy-body acceleration
-        // of the group (the acceleration every body of these systems is made of)
-        const double ah = valid ? sqrt(hax * hax + hay * hay + haz * haz) : INFINITY;
-        const double aref = wave_min(ah);
-        const double qlim = (p.alpha > 0.0 && aref > 0.0 && aref < INFINITY) ? p.alpha * aref : INFINITY;
-        if (lane == 0) stk[0] = enc(gsys, 1, false);   // the root of the group's system
-        __builtin_amdgcn_wave_barrier();
-        while (sp > 0 && !overflow) {
-            // pop up to 64 ranges, one per lane, while the stack cannot overflow
-            const uint32_t P = (sp <= static_cast<uint32_t>(kBigPopLimit)) ? min(sp, 64u) : 1u;
-            const bool has = static_cast<uint32_t>(lane) < P;
-            const uint32_t e = has ? stk[sp - 1 - lane] : 0u;
-            sp -= P;
-            const uint32_t ecount = has ? ((e >> 27) & 7u) + 1u : 0u;
-            const uint32_t incl = wave_incl_scan(ecount);
-            const uint32_t total = uni(static_cast<uint32_t>(__shfl(static_cast<int>(incl), 63, 64)));
-            __builtin_amdgcn_wave_barrier();
-            {
-                const uint32_t kind = e & 0x80000000u;
-                const uint32_t first = e & 0x07ffffffu;
-                for (uint32_t k = 0, o = incl - ecount; k < ecount; ++k) nbuf[o + k] = (first + k) | kind;
-            }
-            __builtin_amdgcn_wave_barrier();
-            n_visit += total;
-            // the nodes of the next 64 entries are loaded before this chunk is
-            // tested, so their latency overlaps its work
-            uint32_t ent_n = 0u;
-            MNode nd_n = fetch_node(mb, nbuf, static_cast<uint32_t>(lane), total, ent_n);
-            for (uint32_t base = 0; base < total; base += 64u) {
-                const uint32_t s = base + static_cast<uint32_t>(lane);
-                const bool act = s < total;
-                const uint32_t ent = ent_n;
-                const MNode nd = nd_n;
-                nd_n = fetch_node(mb, nbuf, s + 64u, total, ent_n);
-                // node entries decide without branches (the opening test runs
-                // for every lane; a wavefront mixes nodes and leaves anyway);
-                // body entries of a multi-body leaf load their body
-                const bool isbody = (ent & 0x80000000u) != 0u;
-                const uint32_t nc = nd.info & ~kMLeaf;
-                const bool leaf = (nd.info & kMLeaf) != 0u;
-                const double ex = fmax(fabs(nd.x - cx) - hx, 0.0);
-                const double ey = fmax(fabs(nd.y - cy) - hy, 0.0);
-                const double ez = fmax(fabs(nd.z - cz) - hz, 0.0);
-                const double d2 = ex * ex + ey * ey + ez * ez;
-                const bool pass = nd.size2 < theta2 * d2 &&
-                                  (nd.size2 <= kSafe2 * d2 || static_cast<double>(nd.gq) <= qlim * (d2 * d2));
-                const bool live = act && !isbody && nd.gm != 0.f;
-                bool app = live && (leaf ? nc == 1u : pass);
-                const bool push_leaf = live && leaf && nc != 1u;
-                const bool push_node = live && !leaf && !pass;
-                uint32_t npush = push_leaf ? (nc + 7u) >> 3 : (push_node ? 1u : 0u);
-                const uint32_t pfirst = nd.first, pcount = nc;
-                const bool pbody = push_leaf;
-                float4 q = make_float4(static_cast<float>(nd.x - cx), static_cast<float>(nd.y - cy),
-                                       static_cast<float>(nd.z - cz), nd.gm);
-                if (act && isbody) {
-                    const uint32_t id = ent & 0x7fffffffu;
-                    const double mb_ = b.m[id];
-                    app = b.hrank[id] < 0 && mb_ != 0.0;
-                    if (app)
-                        q = make_float4(static_cast<float>(b.px[id] - cx), static_cast<float>(b.py[id] - cy),
-                                        static_cast<float>(b.pz[id] - cz), static_cast<float>(p.G * mb_));
-                }
-                // interaction list appends (one per lane at most)
-                const uint64_t am = __ballot(app);
-                const uint32_t na = static_cast<uint32_t>(__popcll(am));
-                if (ln + na > static_cast<uint32_t>(kListCap)) {
-                    __builtin_amdgcn_wave_barrier();
-                    n_steps += flush_list(list, ln, K, sub, cnt, ox, oy, oz, r2_0, acc, rx, ry, rz);
-                    __builtin_amdgcn_wave_barrier();
-                    ln = 0;
-                }
-                if (app) list[ln + rank_below(am)] = q;
-                ln += na;
-                n_inter += na;
-                // stack pushes: one range per opened node or leaf of at most 8
-                // bodies
-                const uint64_t pm = __ballot(npush == 1u);
-                uint64_t big = __ballot(npush > 1u);
-                const uint32_t need = static_cast<uint32_t>(__popcll(pm));
-                if (sp + need > static_cast<uint32_t>(kStackCap)) {
-                    if (lane == 0) atomicOr(&tb.sc->error, kErrStack);
-                    overflow = true;
-                    break;
-                }
-                if (npush == 1u) stk[sp + rank_below(pm)] = enc(pfirst, pcount, pbody);
-                sp += need;
-                // a leaf of more than 8 co-keyed bodies (duplicate or nearly
-                // coincident positions) puts its bodies on the list directly,
-                // 64 at a time, so the stack does not grow with its size
-                for (; big; big &= big - 1) {
-                    const int l = __builtin_ctzll(big);
-                    const uint32_t f = uni(static_cast<uint32_t>(__shfl(static_cast<int>(pfirst), l, 64)));
-                    const uint32_t c = uni(static_cast<uint32_t>(__shfl(static_cast<int>(pcount), l, 64)));
-                    for (uint32_t k0 = 0; k0 < c; k0 += 64u) {
-                        bool appb = false;
-                        float4 qb = make_float4(0.f, 0.f, 0.f, 0.f);
-                        if (k0 + static_cast<uint32_t>(lane) < c) {
-                            const uint32_t j = f + k0 + static_cast<uint32_t>(lane);
-                            const double mj = b.m[j];
-                            if (b.hrank[j] < 0 && mj != 0.0) {
-                                appb = true;
-                                qb = make_float4(static_cast<float>(b.px[j] - cx), static_cast<float>(b.py[j] - cy),
-                                                 static_cast<float>(b.pz[j] - cz), static_cast<float>(p.G * mj));
-                            }
-                        }
-                        const uint64_t bmask = __ballot(appb);
-                        const uint32_t nb = static_cast<uint32_t>(__popcll(bmask));
-                        if (ln + nb > static_cast<uint32_t>(kListCap)) {
-                            __builtin_amdgcn_wave_barrier();
-                            n_steps += flush_list(list, ln, K, sub, cnt, ox, oy, oz, r2_0, acc, rx, ry, rz);
-                            __builtin_amdgcn_wave_barrier();
-                            ln = 0;
-                        }
-                        if (appb) list[ln + rank_below(bmask)] = qb;
-                        ln += nb;
-                        n_inter += nb;
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        n_steps += flush_list(list, ln, K, sub, cnt, ox, oy, oz, r2_0, acc, rx, ry, rz);
-        __builtin_amdgcn_wave_barrier();
-        // the K partial sums of a body, added in FP64 in sub order (a Kahan
-        // sum's value is s - c: c holds the negative of the rounding lost)
-        double lax = static_cast<double>(acc.sx) - static_cast<double>(acc.cx) + rx;
-        double lay = static_cast<double>(acc.sy) - static_cast<double>(acc.cy) + ry;
-        double laz = static_cast<double>(acc.sz) - static_cast<double>(acc.cz) + rz;
-        if (K > 1) {
-            double tx = 0.0, ty = 0.0, tz = 0.0;
-            for (uint32_t k = 0; k < K; ++k) {
-                const int src = static_cast<int>(k * per + bl);
-                tx += __shfl(lax, src, 64);
-                ty += __shfl(lay, src, 64);
-                tz += __shfl(laz, src, 64);
-            }
-            lax = tx;
-            lay = ty;
-            laz = tz;
-        }
-        // heavy bodies take their accelerations from k_heavy_direct instead
-        if (valid && sub == 0 && b.hrank[i] < 0) {
-            const double ax = hax + lax;
-            const double ay = hay + lay;
-            const double az = haz + laz;
-            b.ax[i] = ax;
-            b.ay[i] = ay;
-            b.az[i] = az;
-            if (p.kick) {
-                b.vx[i] = b.vx[i] + p.half_dt * ax;
-                b.vy[i] = b.vy[i] + p.half_dt * ay;
-                b.vz[i] = b.vz[i] + p.half_dt * az;
-            }
-        }
-        // the group's work, the schedules' cost unit: the flushes' costs plus
-        // half the visits (a visit measured half the time of a list step on
-        // the 300k walk)
-        const uint32_t work = n_steps + n_visit / 2u;
-        if (valid && sub == 0) b.pcost[i] = work;
-        if (lane == 0) {
-            mb.g_inter[g] = n_inter;
-            mb.g_visit[g] = n_visit;
-            mb.g_work[g] = work;
-            mb.g_t0[g] = t_start;
-            mb.g_t1[g] = wall_clock64();
-            mb.g_worker[g] = worker;
+            C = min(use_order ? sc->n_coop : sc->n_big, G);
+            listed = true;
         }
     }
+    uint32_t turn_no = 0;
+    uint64_t work_done = 0;
+    for (uint32_t k = blockIdx.x; k < C;) {
+        uint32_t g = k;
+        if (listed) {
+            const WalkArgsP al = args_here(args);
+            g = use_order ? al->mb.order[k] : al->mb.chunk[k];
+        }
+        g = uni(g);
+        if (g < G) {
+            const uint32_t work = walk_group<kWaves>(args, sc, g, w, lane, s_mem, s_word, turn_no);
+            if (w == 0) work_done += work;
+        }
+        if (C <= nblk) break;   // every block had its only one
+        if (threadIdx.x == 0) s_take = atomicAdd(&sc->queue[kQShared][0], 1u);
+        __syncthreads();
+        k = uni(nblk + s_take);
+        __syncthreads();
+    }
+    __syncthreads();   // from here on every wavefront is on its own
+    if (C < G) {
+        unsigned char* const lds = s_mem + w * kWaveLds;
+        uint32_t pos = 0, end = 0;   // the current chunk's groups (sched 2)
+        uint32_t part = blockIdx.x % kWalkParts;   // key order: this XCD's runs first, then the other parts'
+        // With no shared groups a wave's first group is fixed by its place too
+        // (a block's waves take neighbouring places: they sit on the CU's four
+        // SIMDs, so the costliest groups spread over the SIMDs); else the
+        // queues serve the waves as their blocks finish.
+        const uint32_t rank = blockIdx.x * kWaves + static_cast<uint32_t>(w);
+        bool first_take = C == 0u;
+        const uint32_t held = C == 0u ? waves : 0u;   // entries that are fixed
+        auto take = [&](uint32_t row) {
+            uint32_t q = 0;
+            if (lane == 0) q = atomicAdd(&sc->queue[row][0], 1u);
+            return uni(q);
+        };
+        auto held_part = [&](uint32_t x) { return C == 0u ? part_blocks(x, nblk) * kWaves : 0u; };
+        for (;;) {
+            uint32_t g;
+            if (sched == 2) {
+                // balanced chunks of consecutive groups, served by a dynamic queue;
+                // every take consumes a chunk, so the loop ends after n_chunks takes
+                while (pos >= end) {
+                    const uint32_t q = first_take ? rank : held + take(kQOrder);
+                    first_take = false;
+                    const WalkArgsP ac = args_here(args);
+                    if (q >= ac->p.n_chunks) break;
+                    pos = uni(ac->mb.chunk[q]);
+                    end = uni(ac->mb.chunk[q + 1]);
+                }
+                if (pos >= end) break;
+                g = pos++;
+            } else if (use_order) {
+                // heaviest first from one queue: dealing the order out per XCD
+                // measured 23% slower on the 300k walk (its span grows)
+                const uint32_t q = C + (first_take ? rank : held + take(kQOrder));
+                first_take = false;
+                if (q >= G) break;
+                g = args_here(args)->mb.order[q];
+            } else {
+                // key order, dealt out per XCD (5% shorter on the 300k walk, 4%
+                // on a 32-system ensemble)
+                uint32_t q;
+                if (first_take) q = part_group(part, blockIdx.x / kWalkParts * kWaves + static_cast<uint32_t>(w));
+                else q = part_group(part, held_part(part) + take(part));
+                first_take = false;
+                while (q >= G) {
+                    // this part is closed: note it, learn which others are, and
+                    // take from the next that may be open (a part once closed
+                    // stays closed, so the loop ends).  Two atomics for a wave
+                    // that leaves when all are; reading the queues' counters
+                    // instead (relaxed loads, device scope) held up the last
+                    // groups by 130 us at 300k.
+                    uint32_t mask = 0;
+                    if (lane == 0) mask = atomicOr(&sc->queue[kQClosed][0], 1u << part);
+                    const uint32_t open = 0xffu & ~(uni(mask) | 1u << part);
+                    if (open == 0u) break;
+                    const uint32_t turned = ((open >> part) | (open << (kWalkParts - part))) & 0xffu;
+                    part = (part + static_cast<uint32_t>(__builtin_ctz(turned))) % kWalkParts;
+                    q = part_group(part, held_part(part) + take(part));
+                }
+                if (q >= G) break;
+                g = q;
+                if (C > 0u && args_here(args)->mb.gbig[g]) continue;   // walked by a block above
+            }
+            g = uni(g);
+            if (g >= G) continue;   // a schedule entry outside the groups of this step
+            work_done += walk_group<1>(args, sc, g, 0, lane, lds, s_word, turn_no);
+        }
+    }
+    if (lane == 0 && work_done)
+        atomicAdd(reinterpret_cast<unsigned long long*>(&sc->work_sum[blockIdx.x & 7u][0]), static_cast<unsigned long long>(work_done));
     // then the heavy bodies' chunk sums, in the walk's tail: a wave whose
-    // groups are done takes work items while the last groups finish (its LDS
-    // list holds the lane partials)
-    for (;;) {
-        uint32_t q = 0;
-        if (lane == 0) q = atomicAdd(&tb.sc->heavy_counter, 1u);
+    // groups are done takes work items while the last groups finish (its part
+    // of the LDS holds the lane partials).  When the blocks with a group leave
+    // enough waves, the items go to the last waves of the grid without a queue.
+    const WalkArgsP at = args_here(args);
+    const uint32_t items = at->p.heavy_items;
+    const HeavyArgs ha{at->b.px, at->b.py, at->b.pz, at->b.m, at->tb.sys, at->tb.n_sys, at->mb.hpart, at->p.soft2, at->p.G};
+    const bool fixed = C == G && static_cast<uint64_t>(G) * kWaves + items <= waves;
+    for (uint32_t k = 0;; ++k) {
+        uint32_t q;
+        if (fixed) {
+            q = k == 0u ? waves - 1u - (blockIdx.x * kWaves + static_cast<uint32_t>(w)) : items;
+        } else {
+            q = 0;
+            if (lane == 0) q = atomicAdd(&sc->queue[kQHeavy][0], 1u);
+        }
         q = uni(q);
-        if (q >= p.heavy_items) break;
-        heavy_item(b, tb, mb, p, q, lane, reinterpret_cast<double(*)[64]>(list));
+        if (q >= items) break;
+        heavy_item(ha, q, lane, reinterpret_cast<double(*)[64]>(s_mem + w * kWaveLds));
     }
 }
 
@@ -1051,7 +1361,7 @@ __global__ __launch_bounds__(kNT) void k_heavy_partial(Bodies b, TreeBuffers tb,
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t waves = gridDim.x * kWaves;
     for (uint32_t item = blockIdx.x * kWaves + w; item < p.heavy_items; item += waves)
-        heavy_item(b, tb, mb, p, item, lane, part[w]);
+        heavy_item(HeavyArgs{b.px, b.py, b.pz, b.m, tb.sys, tb.n_sys, mb.hpart, p.soft2, p.G}, item, lane, part[w]);
 }
 
 // One wavefront per (system, heavy rank, axis): lane l adds the chunk
@@ -1155,6 +1465,12 @@ __global__ __launch_bounds__(kNT) void k_sched_scatter(size_t n, TreeBuffers tb,
     }
     __syncthreads();
     if (threadIdx.x >= 64 && threadIdx.x < kSchedBuckets) first[threadIdx.x] += wave0_total;
+    if (blockIdx.x == 0) {
+        // the groups of the buckets above the sharing limit come first
+        __syncthreads();
+        if (threadIdx.x == 0 && tb.sc->work_prev != 0u)
+            tb.sc->n_coop = first[cost_bucket(static_cast<float>(share_limit(tb.sc, mb.walk_waves)))];
+    }
     for (uint32_t t0 = blockIdx.x * kNT; t0 < G; t0 += gridDim.x * kNT) {
         if (threadIdx.x < kSchedBuckets) cnt[threadIdx.x] = 0;
         __syncthreads();
@@ -1272,7 +1588,7 @@ void launch_walk_mixed(const Bodies& b, size_t n, const TreeBuffers& tb, const M
                        const MixedParams& p, unsigned blocks, hipStream_t s)
 {
     if (n == 0 || blocks == 0) return;
-    k_walk_mixed<<<blocks, kNT, 0, s>>>(b, n, tb, mb, p);
+    k_walk_mixed<<<blocks, kNT, 0, s>>>(WalkArgs{b, tb, mb, p});
 }
 
 void launch_heavy_direct(const Bodies& b, const TreeBuffers& tb, const MixedBuffers& mb, const MixedParams& p,

@@ -311,11 +311,21 @@ __global__ __launch_bounds__(kNT) void k_keys(Bodies b, size_t n, TreeBuffers tb
         // steps of one call until the host reads and clears them
         StepScalars* sc = tb.sc;
         if (threadIdx.x == 0) {
-            sc->group_counter = 0;
-            sc->heavy_counter = 0;
             sc->n_deep = 0;
+            sc->n_big = 0;
+            sc->n_coop = 0;
+            // the last walk's work, if there was one since
+            uint64_t sum = 0;
+            for (int x = 0; x < 8; ++x) {
+                sum += sc->work_sum[x][0];
+                sc->work_sum[x][0] = 0;
+            }
+            if (sum != 0) {
+                sc->work_prev = sum;
+                sc->groups_prev = sc->n_groups;
+            }
         }
-        if (threadIdx.x < kWalkParts) sc->part_counter[threadIdx.x] = 0;
+        if (threadIdx.x < kQueues) sc->queue[threadIdx.x][0] = 0;
         for (uint32_t k = threadIdx.x; k < 8u * kSchedBuckets; k += kNT) (&sc->sched_hist[0][0])[k] = 0;
         if (threadIdx.x < kSchedBuckets) sc->sched_cursor[threadIdx.x] = 0;
     }

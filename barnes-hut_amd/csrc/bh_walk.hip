@@ -52,35 +52,6 @@ __device__ inline WalkNode load_node(const WalkNode* __restrict__ walk, uint32_t
     return walk[min(k, T - 1)];
 }
 
-// 1.0 / sqrt(x) for x in [2^-767, 2^1000], bit for bit: the instruction
-// sequence the compiler emits for the IEEE FP64 square root (reciprocal
-// square-root estimate refined by Goldschmidt steps) followed by the one for
-// the IEEE division 1 / s (reciprocal estimate, two Newton steps, remainder
-// correction), without their range handling.  In this range the square root
-// needs no exponent scaling and is finite and nonzero, and 1 / s with
-// s in [2^-500, 2^500] needs no scaling and no fix-up, so the range handling
-// leaves every value unchanged there and dropping it saves 12 instructions.
-__device__ inline double inv_sqrt_in_range(double x)
-{
-    const double y = __builtin_amdgcn_rsq(x);
-    double g = x * y;
-    double h = y * 0.5;
-    const double r = __builtin_fma(-h, g, 0.5);
-    g = __builtin_fma(g, r, g);
-    h = __builtin_fma(h, r, h);
-    double d = __builtin_fma(-g, g, x);
-    g = __builtin_fma(d, h, g);
-    d = __builtin_fma(-g, g, x);
-    g = __builtin_fma(d, h, g);   // sqrt(x), correctly rounded
-    double q = __builtin_amdgcn_rcp(g);
-    double e = __builtin_fma(-g, q, 1.0);
-    q = __builtin_fma(q, e, q);
-    e = __builtin_fma(-g, q, 1.0);
-    q = __builtin_fma(q, e, q);
-    e = __builtin_fma(-g, q, 1.0);
-    return __builtin_fma(e, q, q);   // 1 / sqrt(x), correctly rounded
-}
-
 // Block b of the grid (XCD b mod 8) -> the block of bodies it walks: XCD x
 // takes blocks [x * per, (x + 1) * per) of the Morton order, per = ceil(g / 8)
 // (a short last XCD range simply has fewer blocks).
