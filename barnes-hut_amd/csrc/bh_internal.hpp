@@ -208,6 +208,28 @@ __device__ inline double inv_sqrt_in_range(double x)
     return __builtin_fma(e, q, q);   // 1 / sqrt(x), correctly rounded
 }
 
+// Whether inv_sqrt_in_range takes x, from its exponent alone (one subtraction
+// and one compare): x in [2^-767, 2^1000)
+__device__ inline bool inv_sqrt_takes(double x)
+{
+    return static_cast<uint32_t>(__double2hiint(x)) - 0x10000000u < 0x7e700000u - 0x10000000u;
+}
+
+// Compensated sum: c gathers the rounding error of every addition, exactly
+// (the error of s + x in six additions, no comparison; the same value as
+// Neumaier's branch on the larger operand).
+struct ExactSum {
+    double s = 0.0, c = 0.0;
+    __device__ void add(double x)
+    {
+        const double t = s + x;
+        const double xr = t - s;
+        c += (s - (t - xr)) + (x - xr);
+        s = t;
+    }
+    __device__ double value() const { return s + c; }
+};
+
 // ----------------------------------------------------------------- sort
 // Stable LSD radix sort of (key, idx) pairs by the low `bits` key bits.
 // Input in (k0, v0); result in (k0, v0) after the call (ping-pong through
