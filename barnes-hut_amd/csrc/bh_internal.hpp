@@ -517,6 +517,24 @@ void launch_model_train(const ModelBuffers& md, const float* x, const float* t, 
                         hipStream_t s, float hist_drop = 0.f);
 void launch_refresh_bf16(const ModelBuffers& md, hipStream_t s);
 
+// ------------------------------------------------------ host transfers
+struct PackedBodies {   // regions of the staging area, null where not wanted
+    double *pos, *vel, *acc, *mass;
+    uint64_t* ids;
+};
+void launch_split3(const double* v, size_t n, double* x, double* y, double* z, hipStream_t s);
+void launch_pack(const Bodies& b, size_t n, const PackedBodies& out, hipStream_t s);
+// no previous walk work, zero accelerations, ids = rows if own_ids
+void launch_new_bodies(const Bodies& b, size_t n, bool own_ids, hipStream_t s);
+// The systems of the rows (bsys) and the heavy set of every system (hrank;
+// n_heavy is given): runs of kHeavyRun rows of one system, run r = rows
+// run_sys[2 r + 1] * kHeavyRun .. of system run_sys[2 r], system s's runs
+// sys_run[s] .. sys_run[s + 1] - 1.  scratch: heavy_scratch_bytes(n_runs).
+constexpr uint32_t kHeavyRun = 4096;
+size_t heavy_scratch_bytes(uint32_t n_runs);
+void launch_heavy_set(const Bodies& b, const TreeBuffers& tb, const uint32_t* run_sys, uint32_t n_runs,
+                      const uint32_t* sys_run, uint8_t* bsys, void* scratch, hipStream_t s);
+
 // FP64 direct sum for m sample bodies over the bodies of each sample's system
 // (Neumaier-compensated).
 void launch_direct_sum(const Bodies& b, const TreeBuffers& tb, const int64_t* idx, size_t m, double G, double soft2,
