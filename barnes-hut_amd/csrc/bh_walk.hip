@@ -73,9 +73,10 @@ __global__ __launch_bounds__(kNT) void k_walk_plain(Bodies b, size_t n, uint32_t
 {
     const uint32_t vb = xcd_block(blockIdx.x, grid_blocks);
     const size_t i = static_cast<size_t>(vb) * kNT + threadIdx.x;
-    if (i >= n) return;
     // M + B <= 2n - 1 by construction; the clamp keeps a corrupted count in bounds
     const uint32_t T = min(sc->n_nodes, static_cast<uint32_t>(2 * n));
+    if (T * sizeof(WalkNode) <= kWarmBytes) warm_l2(walk, T * sizeof(WalkNode));
+    if (i >= n) return;
     const double px = b.px[i];
     const double py = b.py[i];
     const double pz = b.pz[i];
