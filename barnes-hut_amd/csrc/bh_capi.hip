@@ -243,6 +243,9 @@ int run_force(bh_ctx* c, int form, double theta, double G, double soft2, bool ki
         tb.lraw = nullptr;
         tb.gflag = nullptr;
         tb.gtile = nullptr;
+        // an eager step's launches, and a small tree's in a graph too
+        if (c->moment_cut < 0 && (c->n <= bh::kDeepWhole || tb.deep_from == bh::kMaxDepth))
+            tb.deep_from = bh::moments_cutoff(c->n);
     } else {
         tb.deep_from = bh::kMaxDepth;   // the light-moment pyramid needs no list of deep nodes
     }
@@ -660,6 +663,8 @@ int choose_deep_from(bh_ctx* c)
         c->tb.deep_from = c->moment_cut;
         return BH_OK;
     }
+    // run_force sums a small tree in one workgroup; the mixed forms sum no depths
+    if (c->n <= bh::kDeepWhole || c->cfg.form != BH_FORM_PLAIN) return BH_OK;
     StepScalars sc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     HIP_TRY(c, hipMemcpy(&sc, c->tb.sc, sizeof sc, hipMemcpyDeviceToHost));

@@ -273,6 +273,9 @@ void radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, si
 // the rest is not in order.  Buffers (k1, v1) and (k2, v2) hold n entries.
 void sort_near_sorted(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint64_t* k2, uint32_t* v2, size_t n,
                       int bits, const uint8_t* sysd, uint32_t* tmp, size_t cap, hipStream_t s);
+// The same order for keys in any order, n <= 2^16, by the merge sort alone;
+// result in (k0, v0).  Uses no words of a sort's tmp.
+void sort_small(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n, hipStream_t s);
 // device address of its control words: [0] 1 if the last call took the
 // near-sorted path, [3] the keys it radix sorted there
 uint32_t* sort_near_ctl(uint32_t* sort_tmp, size_t cap);
@@ -371,6 +374,15 @@ void launch_permute(const Bodies& src, const Bodies& dst, const TreeBuffers& tb,
 // (one launch per populated depth, the plain form's order).
 void launch_build_tree(const Bodies& b, size_t n, TreeBuffers& tb, bool moments, hipStream_t s);
 void launch_tree_moments(size_t n, TreeBuffers& tb, hipStream_t s);
+// TreeBuffers::deep_from of the plain form when nothing is known of the tree.
+// Up to kDeepWhole bodies one workgroup sums all of it (a level takes it about
+// 0.9 us, a launch of a graph 1.3, of a stream 3: a step at 3,000 bodies takes
+// 248 us with cutoff 0, 252 with 10, 267 with 21; at 6,000 321, 315, 327).  Up
+// to 2^16 bodies few nodes lie at depth 10 and below (19,054: 487, 436, 447 us;
+// 60,000: 1061, 554, 567); larger trees get a launch per depth until a graph
+// capture has looked at one (choose_deep_from).
+constexpr size_t kDeepWhole = 4096;
+inline int moments_cutoff(size_t n) { return n <= kDeepWhole ? 0 : n <= 65536 ? 10 : kMaxDepth; }
 // the mixed forms' light moments and boxes of the branching nodes, from the
 // pyramid of their leaves (four launches at every size)
 void launch_light_moments(size_t n, TreeBuffers& tb, hipStream_t s);

@@ -819,7 +819,7 @@ constexpr int kMsNT = 1024;   // threads of the tile sort: two elements each
 constexpr int kMsWays = 16;
 static_assert(kMsTile == 2 * kMsNT, "the tile sort holds two elements per thread");
 
-__device__ inline uint32_t merge_rounds(uint32_t m)
+__host__ __device__ inline uint32_t merge_rounds(uint32_t m)
 {
     uint32_t r = 0;
     for (uint64_t L = kMsTile; L < m; L *= kMsWays) ++r;
@@ -868,8 +868,8 @@ __device__ inline uint64_t shfl_xor_u64(uint64_t x, int mask)
 }
 
 template <bool kSys>
-__device__ inline void tile_sort(const uint64_t* __restrict__ ik, const uint32_t* __restrict__ iv,
-                                 uint64_t* __restrict__ k1, uint32_t* __restrict__ v1, const uint8_t* __restrict__ sysd,
+__device__ inline void tile_sort(const uint64_t* ik, const uint32_t* iv,
+                                 uint64_t* k1, uint32_t* v1, const uint8_t* __restrict__ sysd,
                                  uint32_t m, size_t t0, uint64_t* sk, uint32_t* sv, uint8_t* ss)
 {
     const uint32_t e0 = 2u * threadIdx.x;
@@ -962,20 +962,27 @@ __device__ inline void tile_sort(const uint64_t* __restrict__ ik, const uint32_t
     }
 }
 
-__global__ __launch_bounds__(kMsNT) void k_ns_tile_sort(const uint64_t* __restrict__ k0, const uint32_t* __restrict__ v0,
-                                                        const uint64_t* __restrict__ k2, const uint32_t* __restrict__ v2,
-                                                        uint64_t* __restrict__ k1, uint32_t* __restrict__ v1,
-                                                        const uint8_t* __restrict__ sysd, uint32_t* tmp, size_t cap)
+// (the output may be the input: a block reads its tile before it writes it)
+__global__ __launch_bounds__(kMsNT) void k_ns_tile_sort(const uint64_t* k0, const uint32_t* v0,
+                                                        const uint64_t* k2, const uint32_t* v2,
+                                                        uint64_t* k1, uint32_t* v1,
+                                                        const uint8_t* __restrict__ sysd, uint32_t* tmp, size_t cap,
+                                                        uint32_t m_given)
 {
     __shared__ uint64_t sk[kMsTile];
     __shared__ uint32_t sv[kMsTile];
     __shared__ uint8_t ss[kMsTile];
-    const NsTmp nt = ns_tmp_at(tmp, cap);
-    const uint32_t m = nt.ctl[1];
+    // a given count sorts (k0, v0) itself; else the control words say what is sorted
+    uint32_t m = m_given, near = 0;
+    if (!m_given) {
+        const NsTmp nt = ns_tmp_at(tmp, cap);
+        m = nt.ctl[1];
+        near = nt.ctl[0];
+    }
     const size_t t0 = static_cast<size_t>(blockIdx.x) * kMsTile;
     if (t0 >= m) return;
-    const uint64_t* ik = nt.ctl[0] == 1u ? k2 : k0;
-    const uint32_t* iv = nt.ctl[0] == 1u ? v2 : v0;
+    const uint64_t* ik = near == 1u ? k2 : k0;
+    const uint32_t* iv = near == 1u ? v2 : v0;
     if (sysd) tile_sort<true>(ik, iv, k1, v1, sysd, m, t0, sk, sv, ss);
     else tile_sort<false>(ik, iv, k1, v1, sysd, m, t0, sk, sv, ss);
 }
@@ -1081,12 +1088,11 @@ __device__ inline void merge_one(const uint64_t* __restrict__ ik, const uint32_t
 __global__ __launch_bounds__(kNT) void k_ns_merge_round(const uint64_t* __restrict__ ik, const uint32_t* __restrict__ iv,
                                                         uint64_t* __restrict__ ok, uint32_t* __restrict__ ov,
                                                         const uint8_t* __restrict__ sysd, uint32_t* tmp, size_t cap,
-                                                        uint32_t L)
+                                                        uint32_t L, uint32_t m_given)
 {
     __shared__ uint64_t sk[kMsWays][kMsSamples];
     __shared__ uint32_t sv[kMsWays][kMsSamples];
     __shared__ uint8_t ss[kMsWays][kMsSamples];
-    const NsTmp nt = ns_tmp_at(tmp, cap);
     size_t i = static_cast<size_t>(blockIdx.x) * kNT + threadIdx.x;
     uint64_t k = 0;
     uint32_t v = 0;
@@ -1094,7 +1100,7 @@ __global__ __launch_bounds__(kNT) void k_ns_merge_round(const uint64_t* __restri
         k = ik[i];
         v = iv[i];
     }
-    const uint32_t m = nt.ctl[1];
+    const uint32_t m = m_given ? m_given : ns_tmp_at(tmp, cap).ctl[1];
     if (L >= m) return;
     const uint32_t S = L / kMsSamples;
     const size_t span = static_cast<size_t>(L) * kMsWays;
@@ -1290,19 +1296,37 @@ void sort_near_sorted(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, ui
     (void)bits;   // the merge sort compares whole keys
     // tile sort into (k1, v1), then rounds ping-ponging k1 -> k2 -> k1 ...
     k_ns_tile_sort<<<static_cast<unsigned>((n + kMsTile - 1) / kMsTile), kMsNT, 0, s>>>(k0, v0, k2, v2, k1, v1, sysd,
-                                                                                     tmp, cap);
+                                                                                     tmp, cap, 0u);
     uint64_t* ka = k1;
     uint32_t* va = v1;
     uint64_t* kb = k2;
     uint32_t* vb = v2;
     for (size_t L = kMsTile; L < n; L *= kMsWays) {
         k_ns_merge_round<<<static_cast<unsigned>((n + kNT - 1) / kNT), kNT, 0, s>>>(ka, va, kb, vb, sysd, tmp, cap,
-                                                                                  static_cast<uint32_t>(L));
+                                                                                  static_cast<uint32_t>(L), 0u);
         std::swap(ka, kb);
         std::swap(va, vb);
     }
     k_ns_merge<<<static_cast<unsigned>((n + kMpTile - 1) / kMpTile), kNT, 0, s>>>(k0, v0, n, k1, v1, k2, v2, sysd, tmp,
                                                                                 cap);
+}
+
+void sort_small(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n, hipStream_t s)
+{
+    if (n == 0) return;
+    const uint32_t m = static_cast<uint32_t>(n);
+    // the tiles go where an even number of rounds is left to bring them to (k0, v0)
+    const bool odd = merge_rounds(m) & 1u;
+    uint64_t *ka = odd ? k1 : k0, *kb = odd ? k0 : k1;
+    uint32_t *va = odd ? v1 : v0, *vb = odd ? v0 : v1;
+    k_ns_tile_sort<<<static_cast<unsigned>((n + kMsTile - 1) / kMsTile), kMsNT, 0, s>>>(k0, v0, nullptr, nullptr, ka, va,
+                                                                                     nullptr, nullptr, n, m);
+    for (size_t L = kMsTile; L < n; L *= kMsWays) {
+        k_ns_merge_round<<<static_cast<unsigned>((n + kNT - 1) / kNT), kNT, 0, s>>>(ka, va, kb, vb, nullptr, nullptr, n,
+                                                                                  static_cast<uint32_t>(L), m);
+        std::swap(ka, kb);
+        std::swap(va, vb);
+    }
 }
 
 uint32_t* sort_error_word(uint32_t* sort_tmp) { return sort_tmp_at(sort_tmp).chain + 3; }

@@ -41,7 +41,7 @@ struct StaticLayout {
     Bodies cur{}, alt{};
     TreeBuffers tb{};
     double* partials = nullptr;
-    size_t sort_words = 0, scan_words = 0;
+    size_t scan_words = 0;
     size_t bytes = 0;
 };
 
@@ -100,25 +100,22 @@ StaticLayout carve(unsigned char* base, size_t cap)
     t.walk = static_cast<WalkNode*>(take(sizeof(WalkNode) * N2));
     t.deep = static_cast<uint32_t*>(take(4 * N));
     L.scan_words = scan_tmp_words(N2);
-    L.sort_words = sort_tmp_words(N);
     t.scan_tmp = static_cast<uint32_t*>(take(4 * L.scan_words));
-    t.sort_tmp = static_cast<uint32_t*>(take(4 * L.sort_words));
     t.sc = static_cast<StepScalars*>(take(sizeof(StepScalars)));
     t.sys = static_cast<SysScalars*>(take(sizeof(SysScalars)));
     uint8_t* bsys = static_cast<uint8_t*>(take(N));
     t.bsys = bsys;
     L.partials = static_cast<double*>(take(8 * 6 * kBoxBlocks));
-    // the plain form: no light moments, no walk-group flags, one system,
-    // one moment launch per depth
+    // the plain form: no light moments, no walk-group flags, one system
     t.lraw = nullptr;
     t.lbox = nullptr;
     t.lsec = nullptr;
     t.gflag = nullptr;
     t.gtile = nullptr;
+    t.sort_tmp = nullptr;
     t.key_alt2 = nullptr;
     t.perm_alt2 = nullptr;
     t.n_sys = 1;
-    t.deep_from = kMaxDepth;
     L.bytes = off;
     return L;
 }
@@ -128,7 +125,7 @@ StaticLayout carve(unsigned char* base, size_t cap)
 // system's fixed scalars set.  Grid-stride over max(n, words to clear).
 __global__ __launch_bounds__(kNT) void k_static_init(size_t n, const bh_vec3* __restrict__ pos,
                                                      const double* __restrict__ mass, Bodies b, TreeBuffers tb,
-                                                     size_t sort_words, size_t scan_words)
+                                                     size_t scan_words)
 {
     const size_t stride = static_cast<size_t>(gridDim.x) * kNT;
     const size_t t0 = static_cast<size_t>(blockIdx.x) * kNT + threadIdx.x;
@@ -146,7 +143,6 @@ __global__ __launch_bounds__(kNT) void k_static_init(size_t n, const bh_vec3* __
         b.pcost[i] = 0u;
         const_cast<uint8_t*>(tb.bsys)[i] = 0;
     }
-    for (size_t k = t0; k < sort_words; k += stride) tb.sort_tmp[k] = 0u;
     for (size_t k = t0; k < scan_words; k += stride) tb.scan_tmp[k] = 0u;
     const size_t sc_words = sizeof(StepScalars) / sizeof(uint32_t);
     for (size_t k = t0; k < sc_words; k += stride) reinterpret_cast<uint32_t*>(tb.sc)[k] = 0u;
@@ -223,14 +219,17 @@ int bh_compute_accelerations_static(int64_t n, const bh_vec3* pos, const double*
     const uint32_t box_blocks =
         static_cast<uint32_t>(std::max<size_t>(1, (N + kBoxBodiesPerBlock - 1) / kBoxBodiesPerBlock));
     L.tb.box_blocks = box_blocks;
-    const size_t clear = std::max<size_t>({N, L.sort_words, L.scan_words});
+    const size_t clear = std::max<size_t>(N, L.scan_words);
     const unsigned init_blocks = static_cast<unsigned>(std::min<size_t>((clear + kNT - 1) / kNT, 1024));
     static_assert(sizeof(SysScalars) / sizeof(uint32_t) <= kNT, "block 0 clears all of SysScalars");
-    k_static_init<<<init_blocks, kNT, 0, s>>>(N, pos, mass, L.cur, L.tb, L.sort_words, L.scan_words);
+    k_static_init<<<init_blocks, kNT, 0, s>>>(N, pos, mass, L.cur, L.tb, L.scan_words);
     launch_kick_drift_box(L.cur, N, false, 0.0, false, 0.0, L.tb, L.partials, s);
     launch_keys(L.cur, N, L.tb, L.partials, s);
-    radix_sort_pairs(L.tb.key, L.tb.perm, L.tb.key_alt, L.tb.perm_alt, N, 63, nullptr, L.tb.sort_tmp,
-                     kStaticMaxBodies, s);
+    // (the radix sort's histogram and eight passes, mostly waits between tiles,
+    // took 109 us at 3,000 bodies; with the merge sort's two launches and the
+    // moments in one launch the evaluation went from 0.406 to 0.308 ms)
+    sort_small(L.tb.key, L.tb.perm, L.tb.key_alt, L.tb.perm_alt, N, s);
+    L.tb.deep_from = moments_cutoff(N);
     launch_permute(L.cur, L.alt, L.tb, N, s);
     launch_build_tree(L.alt, N, L.tb, true, s);
     launch_walk_order(N, L.tb, s);

@@ -560,11 +560,19 @@ __global__ __launch_bounds__(kNT) void k_link(size_t n, TreeBuffers tb)
 // Every child's values are loaded before the first sum (an empty octant loads
 // the node's first child again and is then skipped), so one node costs two
 // dependent memory round trips, not one per child.
-__device__ inline void node_moments(const TreeBuffers& tb, uint32_t M, size_t bi)
+struct ChildSet {
+    int4 a, b;
+};
+
+__device__ inline ChildSet child_set(const TreeBuffers& tb, size_t bi)
 {
     const int4* c4 = reinterpret_cast<const int4*>(tb.child + 8 * bi);
-    const int4 ca = c4[0], cb = c4[1];
-    const int32_t c[8] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
+    return {c4[0], c4[1]};
+}
+
+__device__ inline void node_moments(const TreeBuffers& tb, uint32_t M, size_t bi, const ChildSet& cs)
+{
+    const int32_t c[8] = {cs.a.x, cs.a.y, cs.a.z, cs.a.w, cs.b.x, cs.b.y, cs.b.z, cs.b.w};
     int32_t any = c[0];
 #pragma unroll
     for (int k = 1; k < 8; ++k) any = (any < 0) ? c[k] : any;
@@ -593,50 +601,89 @@ __global__ __launch_bounds__(kNT) void k_moments_level(TreeBuffers tb, int depth
     const size_t bi = static_cast<size_t>(blockIdx.x) * kNT + threadIdx.x;
     const uint32_t M = tb.sc->n_leaves, B = tb.sc->n_branch;
     if (bi >= B || tb.bdepth[bi] != depth) return;
-    node_moments(tb, M, bi);
+    node_moments(tb, M, bi, child_set(tb, bi));
 }
 
 // The listed nodes tb.deep[0, n_deep), bottom-up by depth in one workgroup:
 // a barrier between depths makes a level's moments visible to the next, so
-// each node sees final children, as with one launch per depth.  The list is
-// in LDS when it fits, else read from memory on every level; only the
-// depths between the list's shallowest and deepest are visited.
+// each node sees final children, as with one launch per depth.  A list that
+// fits is put into LDS in the order of its depths, deepest first, and each
+// thread reads its next node's children (the topology is final) before the
+// barrier, so that a level costs one memory trip; a longer list is read from
+// memory on every level.
 constexpr int kDeepNT = 1024;
-constexpr uint32_t kDeepLds = 4096;
+constexpr uint32_t kDeepLds = 12288;
 
 __device__ inline void moments_listed(const TreeBuffers& tb)
 {
     __shared__ uint32_t sn[kDeepLds];
-    __shared__ uint8_t sd[kDeepLds];
-    __shared__ int s_top, s_bot;
+    __shared__ uint32_t s_end[kMaxDepth + 1];   // list positions where each depth's nodes end
     const uint32_t M = tb.sc->n_leaves, nd = tb.sc->n_deep;
     if (nd == 0) return;
-    const bool lds = nd <= kDeepLds;
+    if (nd > kDeepLds) {
+        for (int d = kMaxDepth; d >= 0; --d) {
+            for (uint32_t k = threadIdx.x; k < nd; k += kDeepNT) {
+                const uint32_t bi = tb.deep[k];
+                if (tb.bdepth[bi] == d) node_moments(tb, M, bi, child_set(tb, bi));
+            }
+            __syncthreads();
+        }
+        return;
+    }
+    if (threadIdx.x <= kMaxDepth) s_end[threadIdx.x] = 0;
+    __syncthreads();
+    constexpr int kPer = static_cast<int>(kDeepLds / kDeepNT);
+    uint32_t node[kPer], at[kPer];   // this thread's nodes, their depths and ranks within them
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const uint32_t k = threadIdx.x + static_cast<uint32_t>(q) * kDeepNT;
+        node[q] = k < nd ? tb.deep[k] : kNone;
+    }
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        at[q] = 0;
+        if (node[q] == kNone) continue;
+        const uint32_t d = tb.bdepth[node[q]];
+        at[q] = d << 16 | atomicAdd(&s_end[d], 1u);
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        s_top = 0;
-        s_bot = kMaxDepth;
-    }
-    __syncthreads();
-    int top = 0, bot = kMaxDepth;
-    for (uint32_t k = threadIdx.x; k < nd; k += kDeepNT) {
-        const uint32_t bi = tb.deep[k];
-        const int d = tb.bdepth[bi];
-        top = max(top, d);
-        bot = min(bot, d);
-        if (lds) {
-            sn[k] = bi;
-            sd[k] = static_cast<uint8_t>(d);
+        uint32_t e = 0;
+        for (int d = kMaxDepth; d >= 0; --d) {
+            e += s_end[d];
+            s_end[d] = e;
         }
     }
-    atomicMax(&s_top, top);
-    atomicMin(&s_bot, bot);
     __syncthreads();
-    for (int d = s_top; d >= s_bot; --d) {
-        for (uint32_t k = threadIdx.x; k < nd; k += kDeepNT) {
-            const uint32_t bi = lds ? sn[k] : tb.deep[k];
-            const int dk = lds ? sd[k] : tb.bdepth[bi];
-            if (dk == d) node_moments(tb, M, bi);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const uint32_t d = at[q] >> 16;
+        if (node[q] != kNone) sn[(d < kMaxDepth ? s_end[d + 1] : 0u) + (at[q] & 0xffffu)] = node[q];
+    }
+    __syncthreads();
+    uint32_t lo = 0, bi = kNone;
+    ChildSet cs{};
+    for (int d = kMaxDepth; d >= 0; --d) {
+        const uint32_t hi = s_end[d];
+        if (hi == lo) continue;   // (block-uniform)
+        if (bi != kNone) node_moments(tb, M, bi, cs);   // the node read ahead
+        else if (lo == 0 && threadIdx.x < hi) {
+            bi = sn[threadIdx.x];
+            node_moments(tb, M, bi, child_set(tb, bi));
         }
+        for (uint32_t k = lo + threadIdx.x + kDeepNT; k < hi; k += kDeepNT) {
+            bi = sn[k];
+            node_moments(tb, M, bi, child_set(tb, bi));
+        }
+        // the first node of the next depth that has any
+        int d1 = d - 1;
+        while (d1 >= 0 && s_end[d1] == hi) --d1;
+        bi = kNone;
+        if (d1 >= 0 && hi + threadIdx.x < s_end[d1]) {
+            bi = sn[hi + threadIdx.x];
+            cs = child_set(tb, bi);
+        }
+        lo = hi;
         __syncthreads();
     }
 }
@@ -844,13 +891,14 @@ __global__ __launch_bounds__(kPyrNT) void k_pyr_nodes(TreeBuffers tb)
     for (int q = 0; q < 6; ++q) tb.lbox[6 * t + q] = acc[6 + q];
 }
 
-// reversed per-leaf node counts for the suffix scan
+// reversed per-leaf node counts for the suffix scan, and their block sums
 __global__ __launch_bounds__(kNT) void k_suffix_input(size_t n, TreeBuffers tb, uint32_t* __restrict__ out)
 {
     const size_t k = static_cast<size_t>(blockIdx.x) * kNT + threadIdx.x;
-    if (k >= n) return;
     const uint32_t M = tb.sc->n_leaves;
-    out[k] = k < M ? 1u + tb.cnt_hi[M - 1 - k] : 0u;
+    const uint32_t v = k < M ? 1u + tb.cnt_hi[M - 1 - k] : 0u;   // (M <= n)
+    if (k < n) out[k] = v;
+    scan_block_sum(v, tb.scan_tmp);
 }
 
 // S(i): number of nodes whose key range ends at or after leaf i
@@ -987,7 +1035,8 @@ void launch_build_tree(const Bodies& b, size_t n, TreeBuffers& tb, bool moments,
 void launch_walk_order(size_t n, TreeBuffers& tb, hipStream_t s)
 {
     k_suffix_input<<<nblk(n), kNT, 0, s>>>(n, tb, tb.is_rep);
-    scan_exclusive_u32(tb.is_rep, tb.suffix, &tb.sc->n_nodes, n, tb.scan_tmp, s);
+    scan_tile_offsets(tb.scan_tmp, n, s);
+    scan_tile_apply(tb.is_rep, n, tb.scan_tmp, tb.suffix, &tb.sc->n_nodes, s);
     k_walk_records<<<nblk(2 * n), kNT, 0, s>>>(n, tb);
 }
 

@@ -197,10 +197,11 @@ int bh_get_sort_stats(bh_ctx *ctx, int *near_path, int64_t *sorted_keys);
 /* Tree moments (no counterpart in the reference, whose octree sums them in
  * one recursive pass, src/linear_octree.cpp): one launch per depth, bottom
  * up, except that the branching nodes at depth >= cutoff are summed by a
- * single workgroup, depth by depth, in one launch.  cutoff -1 (default):
- * chosen from the current tree whenever a step graph is captured, one below
- * its deepest branching node (so the empty depths cost one launch, not one
- * each); 0..21 fixes it (21: one launch per depth throughout).  Every cutoff
+ * single workgroup, depth by depth, in one launch.  cutoff -1 (default): the
+ * whole tree up to 4,096 bodies; else chosen from the current tree whenever a
+ * step graph is captured, one below its deepest branching node (so the empty
+ * depths cost one launch, not one each), and 10 up to 65,536 bodies or 21
+ * until then; 0..21 fixes it (21: one launch per depth throughout).  Every cutoff
  * gives the same bits. */
 int bh_set_moment_cutoff(bh_ctx *ctx, int cutoff);
 
