@@ -45,6 +45,13 @@ constexpr uint32_t kMetaDepthMask = 31u;      // test (bottom) depth
 constexpr uint32_t kMetaTopShift = 5;         // chain top depth (5 bits)
 constexpr uint32_t kMetaLeaf = 1u << 10;      // distinct-key leaf (depth 21)
 constexpr uint32_t kMetaChain = 1u << 11;     // leaf chain starts above depth 21
+// Up to kWaveMax bodies the plain walk may visit a node's children in two
+// chains, from the first child and from the middle one: kMetaMore is set on a
+// node whose chain goes on with the sibling at `skip`, and the middle child's
+// walk index stands above kMetaMidShift.
+constexpr uint32_t kMetaMore = 1u << 12;
+constexpr uint32_t kMetaMidShift = 16;
+constexpr size_t kWaveMax = 20480;            // (at most 2 n - 1 walk indices: 16 bits)
 
 constexpr int kMaxHeavy = 16;     // bodies per system summed directly in FP64 by the mixed forms
 constexpr int kMaxSystems = 256;  // systems per context (the sort's system pass uses 8-bit digits)
@@ -214,17 +221,18 @@ __device__ inline double inv_sqrt_in_range(double x)
 // written by other XCDs, so every line's first touch goes to memory, and a
 // walk meets its lines one dependent load after the other.  (Plain walk of
 // 3,000 bodies 0.172 -> 0.148 ms, 19,054 0.355 -> 0.320, 50,021 0.534 ->
-// 0.489.)  blockDim 256; bytes a multiple of 16.
+// 0.489.)  Blocks of kThreads; bytes a multiple of 16.
 constexpr size_t kWarmBytes = size_t{4} << 20;
 
+template <uint32_t kThreads = 256>
 __device__ inline void warm_l2(const void* base, size_t bytes)
 {
     const uint4* p = static_cast<const uint4*>(base);
     const uint32_t total = static_cast<uint32_t>(bytes / sizeof(uint4));
     const uint32_t xcd_blocks = (gridDim.x - (blockIdx.x & 7u) + 7u) / 8u;   // of this XCD
-    const uint32_t stride = xcd_blocks * 256u;
+    const uint32_t stride = xcd_blocks * kThreads;
     constexpr uint32_t kU = 8;
-    for (uint32_t i = blockIdx.x / 8u * 256u + threadIdx.x; i < total; i += kU * stride) {
+    for (uint32_t i = blockIdx.x / 8u * kThreads + threadIdx.x; i < total; i += kU * stride) {
         uint4 v[kU];
 #pragma unroll
         for (uint32_t u = 0; u < kU; ++u) v[u] = p[min(i + u * stride, total - 1u)];

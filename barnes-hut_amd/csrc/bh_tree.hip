@@ -915,6 +915,42 @@ __device__ inline double finish_com(double raw, double m)
     return (z * z + m * c) / (z + m);
 }
 
+// kMetaMore and the middle child of node t (see kMetaMore).  Children are in
+// walk order from octant 7 down; the second half of c of them, from the
+// (c + 1) / 2-th, is a chain of its own.
+__device__ inline uint32_t child_chains(const TreeBuffers& tb, uint32_t M, uint32_t t, uint32_t par)
+{
+    uint32_t meta = 0;
+    if (par != kNone) {
+        const ChildSet cs = child_set(tb, par - M);
+        const int32_t c[8] = {cs.b.w, cs.b.z, cs.b.y, cs.b.x, cs.a.w, cs.a.z, cs.a.y, cs.a.x};
+        uint32_t all = 0, before = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (c[k] == static_cast<int32_t>(t)) before = all;
+            all += c[k] >= 0;
+        }
+        if (before + 1 < all && before + 1 != (all + 1) / 2) meta |= kMetaMore;
+    }
+    if (t >= M) {
+        const ChildSet cs = child_set(tb, t - M);
+        const int32_t c[8] = {cs.b.w, cs.b.z, cs.b.y, cs.b.x, cs.a.w, cs.a.z, cs.a.y, cs.a.x};
+        uint32_t all = 0, at = 0, mid = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) all += c[k] >= 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (c[k] < 0) continue;
+            if (at == (all + 1) / 2) mid = static_cast<uint32_t>(c[k]);
+            ++at;
+        }
+        // (not the first child, so no ancestor ends with it)
+        const uint32_t w = mid < M ? suffix_count(tb, M, mid) - 1 : suffix_count(tb, M, tb.bhi[mid - M] + 1);
+        meta |= (w & 0xffffu) << kMetaMidShift;
+    }
+    return meta;
+}
+
 __global__ __launch_bounds__(kNT) void k_walk_records(size_t n, TreeBuffers tb)
 {
     const size_t t = static_cast<size_t>(blockIdx.x) * kNT + threadIdx.x;
@@ -965,6 +1001,7 @@ __global__ __launch_bounds__(kNT) void k_walk_records(size_t n, TreeBuffers tb)
     nd.side2 = leaf ? (chain_leaf ? tb.sys[0].side2[kMaxDepth - 1] : INFINITY) : tb.sys[0].side2[test_depth];
     nd.skip = skip;
     uint32_t meta = test_depth | (top << kMetaTopShift);
+    if (n <= kWaveMax) meta |= child_chains(tb, M, static_cast<uint32_t>(t), par);
     if (leaf) {
         meta |= kMetaLeaf;
         if (top <= kMaxDepth - 1) meta |= kMetaChain;

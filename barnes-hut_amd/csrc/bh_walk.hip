@@ -62,6 +62,58 @@ __device__ inline uint32_t xcd_block(uint32_t b, uint32_t g)
     return x * per + k;
 }
 
+// set bits of m below this lane
+__device__ inline uint32_t rank_below(uint64_t m)
+{
+    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
+}
+
+__device__ inline uint64_t read_lane(uint64_t v, int from)
+{
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), from));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), from));
+    return static_cast<uint64_t>(hi) << 32 | lo;
+}
+
+struct Decision {
+    double dx, dy, dz, r2, t2r2;
+    bool live, is_self, accept, open;
+};
+
+// The decision at a node (src/traversal.cpp:67-77): zero-mass nodes and the
+// body's own leaf are skipped, a leaf is always accepted, a cell when side^2 <
+// theta^2 r^2.  (A leaf is accepted always except by its own bodies: their
+// leaf's side^2 is +inf unless its chain starts above depth 21, so `pass` is
+// the reference's self-chain test.  Bitwise, so the decision is a few mask
+// operations and no branch.)
+__device__ inline Decision decide(const WalkNode& nd, double px, double py, double pz, bool is_self,
+                                  const WalkParams& p)
+{
+    Decision d;
+    d.dx = nd.x - px;
+    d.dy = nd.y - py;
+    d.dz = nd.z - pz;
+    d.r2 = d.dx * d.dx + d.dy * d.dy + d.dz * d.dz + p.soft2;
+    d.t2r2 = p.theta2 * d.r2;
+    d.live = nd.m != 0.0;
+    d.is_self = is_self;
+    const bool pass = nd.side2 < d.t2r2;
+    const bool leaf = (nd.meta & kMetaLeaf) != 0u;
+    d.accept = d.live & (pass | (leaf & !is_self));
+    d.open = d.live & !d.accept & !is_self;
+    return d;
+}
+
+// G m / r^3.  inv_sqrt_in_range gives the bits of 1.0 / sqrt(r2) in its
+// range; a wave with a lane outside it takes the library path.
+__device__ inline double pull(double r2, double m, double G)
+{
+    const bool in_range = (r2 >= 0x1p-767) & (r2 <= 0x1p+1000);
+    const double invR = __all(in_range) ? inv_sqrt_in_range(r2) : 1.0 / sqrt(r2);
+    const double invR3 = invR * invR * invR;
+    return G * m * invR3;
+}
+
 template <bool kCount>
 __global__ __launch_bounds__(kNT) void k_walk_plain(Bodies b, size_t n, uint32_t grid_blocks,
                                                     const WalkNode* __restrict__ walk,
@@ -86,51 +138,31 @@ __global__ __launch_bounds__(kNT) void k_walk_plain(Bodies b, size_t n, uint32_t
     uint32_t cur = 0;
     WalkNode nd = load_node(walk, 0, T);
     while (cur < T) {
-        // the decision first (src/traversal.cpp:67-77): zero-mass nodes and
-        // the body's own leaf are skipped, a leaf is always accepted, a cell
-        // when side^2 < theta^2 r^2
-        const double dx = nd.x - px;
-        const double dy = nd.y - py;
-        const double dz = nd.z - pz;
-        const double r2 = dx * dx + dy * dy + dz * dz + p.soft2;
-        const double t2r2 = p.theta2 * r2;
-        const bool live = nd.m != 0.0;
-        const bool is_self = cur == self;
-        const bool pass = nd.side2 < t2r2;
-        const bool leaf = (nd.meta & kMetaLeaf) != 0u;
-        // a cell is accepted when it passes; a leaf always, except by its own
-        // bodies: their leaf's side^2 is +inf unless its chain starts above
-        // depth 21, so `pass` is the reference's self-chain test
-        // (bitwise, so the decision is a few mask operations and no branch)
-        const bool accept = live & (pass | (leaf & !is_self));
-        const bool open = live & !accept & !is_self;
+        // the decision first
+        const Decision d = decide(nd, px, py, pz, cur == self, p);
         // then the fetch of the next record, whose latency the FP64
         // arithmetic of the accepted node covers; a subtree's skip index
         // always lies beyond it, and max() keeps the walk moving forward even
         // for a corrupted record
-        const uint32_t next = open ? cur + 1 : max(nd.skip, cur + 1);
+        const uint32_t next = d.open ? cur + 1 : max(nd.skip, cur + 1);
         const WalkNode nn = load_node(walk, next, T);
-        if (accept) {
-            // inv_sqrt_in_range gives the bits of 1.0 / sqrt(r2) in its range;
-            // a wave with an accepting lane outside it takes the library path
-            const bool in_range = (r2 >= 0x1p-767) & (r2 <= 0x1p+1000);
-            const double invR = __all(in_range) ? inv_sqrt_in_range(r2) : 1.0 / sqrt(r2);
-            const double invR3 = invR * invR * invR;
-            const double s = p.G * nd.m * invR3;
-            ax += s * dx;
-            ay += s * dy;
-            az += s * dz;
+        if (d.accept) {
+            const double s = pull(d.r2, nd.m, p.G);
+            ax += s * d.dx;
+            ay += s * d.dy;
+            az += s * d.dz;
         }
-        if (kCount && live) {
+        if (kCount && d.live) {
             ++nt;
             const uint32_t top = (nd.meta >> kMetaTopShift) & 31u;
             const uint32_t bottom = nd.meta & kMetaDepthMask;
-            if (accept) {
+            if (d.accept) {
                 ++na;
                 // the reference opens the chain cells above the first passing depth
-                const uint32_t last = leaf ? (is_self ? kMaxDepth - 1 : kMaxDepth) : bottom;
-                no += first_pass_depth(sy, top, last, t2r2) - top;
-            } else if (is_self) {
+                const bool leaf = (nd.meta & kMetaLeaf) != 0u;
+                const uint32_t last = leaf ? (d.is_self ? kMaxDepth - 1 : kMaxDepth) : bottom;
+                no += first_pass_depth(sy, top, last, d.t2r2) - top;
+            } else if (d.is_self) {
                 no += kMaxDepth - top;
             } else {
                 no += bottom - top + 1;
@@ -155,6 +187,274 @@ __global__ __launch_bounds__(kNT) void k_walk_plain(Bodies b, size_t n, uint32_t
     }
 }
 
+// ----------------------------------------------------- a small system's walk
+// One wavefront walks one body.  The per-lane walk above is one chain of
+// dependent visits per body, and a small system has too few bodies to fill the
+// chip with such chains; here the nodes still to be visited lie on a stack in
+// LDS, up to 128 are visited at once, and a visit pushes the first and the
+// middle child of an opened node and the next sibling of its chain.  The
+// visits come in no order, so an accepted node is also a bit in a bitmap over
+// the walk indices: the bits below it are its rank in the reference's order.
+// The contributions are then evaluated 64 at a time in that order, and three
+// lanes add them up one by one, while the next 64 records are on their way: the
+// bits of the per-lane walk.
+// LDS: 2 n bits for the bitmap; the stack, whose place the counts before each
+// word of the bitmap take, and then the contributions; and the accepted nodes
+// as they were found, whose place the ordered ones take.  More than kFound are
+// read off the bitmap in pieces instead.  A full stack, or more visits than
+// the tree has nodes, sends the body to the walk by one lane.
+// Walk of 3,000 bodies (theta 1.05) 0.140 -> 0.028 ms, 8,000 0.206 -> 0.080,
+// 19,054 0.297 -> 0.197, the last bound by vector instructions and by the
+// latency of a wavefront's rounds (16 wavefronts a CU, by their LDS).
+constexpr uint32_t kStack = 1024;       // (950 the deepest seen with no limit, at theta 0.1)
+constexpr uint32_t kFound = 1536;
+constexpr uint32_t kWaves = 4;          // bodies of a block, independent of each other
+constexpr uint32_t kConRow = 66;        // contributions of one component: 64 and a pad for the banks
+
+struct alignas(16) WaveLds {
+    union {
+        uint16_t stack[kStack];
+        uint16_t before[2 * kWaveMax / 64];
+        double con[3][kConRow];
+    };
+    uint16_t list[kFound];
+};
+
+template <int kCtrl, int kRows>
+__device__ inline uint32_t dpp_add(uint32_t v)
+{
+    return v + static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRows, 0xf, false));
+}
+
+__device__ inline uint32_t wave_scan(uint32_t v)   // inclusive prefix sum
+{
+    v = dpp_add<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);   // row_bcast 15, 31
+    return dpp_add<0x143, 0xc>(v);
+}
+
+__device__ inline void store_acc(const Bodies& b, size_t i, uint32_t c, double a, const WalkParams& p)
+{
+    (c == 0 ? b.ax : c == 1 ? b.ay : b.az)[i] = a;
+    if (!p.kick) return;
+    double* v = (c == 0 ? b.vx : c == 1 ? b.vy : b.vz) + i;
+    *v = *v + p.half_dt * a;   // src/main.cpp:278-280
+}
+
+struct Vec3 {
+    double x, y, z;
+};
+
+__device__ inline Vec3 contribution(const WalkNode& nd, double px, double py, double pz, const WalkParams& p)
+{
+    const double dx = nd.x - px;
+    const double dy = nd.y - py;
+    const double dz = nd.z - pz;
+    const double r2 = dx * dx + dy * dy + dz * dz + p.soft2;
+    const double s = pull(r2, nd.m, p.G);
+    return {s * dx, s * dy, s * dz};
+}
+
+// Orders this wavefront's LDS accesses for its lanes (the LDS serves one
+// wavefront's instructions in order, so nothing is waited for).
+__device__ inline void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__global__ __launch_bounds__(64 * kWaves) void k_walk_wave(Bodies b, size_t n, uint32_t grid_blocks,
+                                                           const WalkNode* __restrict__ walk,
+                                                           const uint32_t* __restrict__ self_w,
+                                                           const StepScalars* __restrict__ sc, WalkParams p,
+                                                           uint32_t words)
+{
+    extern __shared__ unsigned long long all_bits[];
+    __shared__ WaveLds ls[kWaves];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    unsigned long long* const bits = all_bits + wave * words;
+    WaveLds& l = ls[wave];
+    const uint32_t T = min(sc->n_nodes, static_cast<uint32_t>(2 * n));
+    warm_l2<64 * kWaves>(walk, T * sizeof(WalkNode));
+    const size_t i = static_cast<size_t>(xcd_block(blockIdx.x, grid_blocks)) * kWaves + wave;
+    if (i >= n || T == 0) return;
+    const double px = b.px[i];
+    const double py = b.py[i];
+    const double pz = b.pz[i];
+    const uint32_t self = self_w[i];
+    for (uint32_t k = lane; k < words; k += 64) bits[k] = 0;
+    if (lane == 0) l.stack[0] = 0;
+    wave_sync();
+
+    uint32_t size = 1, visits = 0, total = 0;   // total: accepted nodes
+    // the visit of node k by the lanes with act: at most three pushes each
+    const auto visit = [&](bool act, uint32_t k, const WalkNode& nd) {
+        const Decision d = decide(nd, px, py, pz, k == self, p);
+        const bool take = act & d.accept;
+        const uint64_t mt = __ballot(take);
+        const uint32_t at = total + rank_below(mt);
+        if (take) atomicOr(bits + (k >> 6), 1ull << (k & 63u));
+        if (take & (at < kFound)) l.list[at] = static_cast<uint16_t>(k);
+        total += static_cast<uint32_t>(__popcll(mt));
+        const uint32_t mid = nd.meta >> kMetaMidShift;
+        const bool more = act & ((nd.meta & kMetaMore) != 0u) & (nd.skip > k) & (nd.skip < T);
+        const bool open = act & d.open & (k + 1 < T);
+        const bool open2 = open & (mid > k) & (mid < T);
+        const uint64_t mm = __ballot(more), mo = __ballot(open), m2 = __ballot(open2);
+        const uint32_t s2 = size + static_cast<uint32_t>(__popcll(mm));
+        const uint32_t s3 = s2 + static_cast<uint32_t>(__popcll(m2));
+        const uint32_t s4 = s3 + static_cast<uint32_t>(__popcll(mo));
+        if (more) l.stack[size + rank_below(mm)] = static_cast<uint16_t>(nd.skip);
+        if (open2) l.stack[s2 + rank_below(m2)] = static_cast<uint16_t>(mid);
+        if (open) l.stack[s3 + rank_below(mo)] = static_cast<uint16_t>(k + 1);
+        size = s4;
+    };
+    bool ok = true;
+    while (ok && size > 0) {
+        // near a full stack fewer are visited at once: t leave it, at most 3 t come
+        const uint32_t t = min(min(size, 128u), (kStack - size) / 2);
+        if (t == 0) {
+            ok = false;
+            break;
+        }
+        size -= t;
+        visits += t;
+        const bool a0 = lane < t, a1 = lane + 64 < t;
+        const uint32_t k0 = l.stack[size + (a0 ? lane : 0u)];
+        const WalkNode n0 = load_node(walk, k0, T);
+        if (t > 64) {
+            const uint32_t k1 = l.stack[size + (a1 ? lane + 64 : 0u)];
+            const WalkNode n1 = load_node(walk, k1, T);
+            wave_sync();
+            visit(true, k0, n0);
+            visit(a1, k1, n1);
+        } else {
+            wave_sync();
+            visit(a0, k0, n0);
+        }
+        if (visits > T) ok = false;
+        wave_sync();
+    }
+    wave_sync();
+
+    if (!ok) {
+        if (lane) return;
+        double ax = 0.0, ay = 0.0, az = 0.0;
+        for (uint32_t cur = 0; cur < T;) {
+            const WalkNode nd = load_node(walk, cur, T);
+            const Decision d = decide(nd, px, py, pz, cur == self, p);
+            if (d.accept) {
+                const Vec3 c = contribution(nd, px, py, pz, p);
+                ax += c.x;
+                ay += c.y;
+                az += c.z;
+            }
+            cur = d.open ? cur + 1 : max(nd.skip, cur + 1);
+        }
+        store_acc(b, i, 0, ax, p);
+        store_acc(b, i, 1, ay, p);
+        store_acc(b, i, 2, az, p);
+        return;
+    }
+
+    uint32_t cnt = 0;                 // ordered indices in l.list
+    uint32_t next = 0;                // where they are read off: the bitmap's next 64 words,
+    uint64_t word = 0, left = 0;      // the lane's of the last 64, those not yet read
+    if (total <= kFound) {
+        uint32_t f[kFound / 64];
+#pragma unroll
+        for (uint32_t q = 0; q < kFound / 64; ++q)
+            if (q * 64 < total) f[q] = l.list[min(q * 64 + lane, total - 1)];
+        for (uint32_t w0 = 0; w0 < words; w0 += 64) {
+            const uint32_t w = w0 + lane;
+            const uint32_t c = w < words ? static_cast<uint32_t>(__popcll(bits[w])) : 0u;
+            const uint32_t inc = wave_scan(c);
+            if (w < words) l.before[w] = static_cast<uint16_t>(cnt + inc - c);
+            cnt += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(inc), 63));
+        }
+        wave_sync();
+        // (the nodes visited are distinct, and so are their ranks; the lanes
+        // past the end write the last one's again)
+        cnt = min(cnt, kFound);
+#pragma unroll
+        for (uint32_t q = 0; q < kFound / 64; ++q)
+            if (q * 64 < total) {
+                const uint64_t below = bits[f[q] >> 6] & ((1ull << (f[q] & 63u)) - 1ull);
+                const uint32_t r = l.before[f[q] >> 6] + static_cast<uint32_t>(__popcll(below));
+                l.list[min(r, kFound - 1)] = static_cast<uint16_t>(f[q]);
+            }
+        next = words;
+    }
+    double acc = 0.0;   // lane c: component c
+    const uint32_t row = min(lane, 2u);
+    const auto put = [&](uint32_t j, const Vec3& c) {
+        // (a sum that starts at 0.0 is never -0.0, so adding 0.0 keeps its bits)
+        const bool in = j + lane < cnt;
+        l.con[0][lane] = in ? c.x : 0.0;
+        l.con[1][lane] = in ? c.y : 0.0;
+        l.con[2][lane] = in ? c.z : 0.0;
+    };
+    const auto add_up = [&]() {
+        const double2* v = reinterpret_cast<const double2*>(l.con[row]);
+#pragma unroll 1
+        for (uint32_t g = 0; g < 32; g += 8) {   // (all of it at once would take 128 registers)
+            double2 c[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) c[u] = v[g + u];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) {
+                acc += c[u].x;
+                acc += c[u].y;
+            }
+        }
+    };
+    do {
+        if (left != 0 || next < words) {
+            cnt = 0;
+            while (cnt <= kFound - 64) {
+                if (left == 0) {
+                    if (next >= words) break;
+                    word = next + lane < words ? bits[next + lane] : 0;
+                    left = __ballot(word != 0);
+                    next += 64;
+                    continue;
+                }
+                const int from = __ffsll(static_cast<unsigned long long>(left)) - 1;
+                left &= left - 1;
+                const uint64_t w = read_lane(word, from);
+                const uint32_t k0 = (next - 64 + static_cast<uint32_t>(from)) * 64;
+                if (w >> lane & 1) l.list[cnt + rank_below(w)] = static_cast<uint16_t>(k0 + lane);
+                cnt += static_cast<uint32_t>(__popcll(w));
+            }
+        }
+        wave_sync();
+        if (cnt == 0) continue;
+        put(0, contribution(load_node(walk, l.list[min(lane, cnt - 1)], T), px, py, pz, p));
+        wave_sync();
+        for (uint32_t j = 64; j < cnt; j += 64) {
+            const WalkNode nd = load_node(walk, l.list[min(j + lane, cnt - 1)], T);
+            add_up();
+            wave_sync();
+            put(j, contribution(nd, px, py, pz, p));
+            wave_sync();
+        }
+        add_up();
+        wave_sync();
+    } while (left != 0 || next < words);
+    if (lane < 3) store_acc(b, i, lane, acc, p);
+}
+
+// A wavefront per body up to 16,384 bodies, and to kWaveMax where the list is
+// not very short (theta <= 1.2): the work grows with n, the per-lane chains
+// hardly do.  Walk in ms, per-lane and by wavefronts (belt): 16,384 bodies
+// 0.273 and 0.170 (theta 1.05), 0.099 and 0.099 (theta 2); 20,000 bodies 0.300
+// and 0.203 (1.05), 0.797 and 0.741 (0.5), 0.104 and 0.117 (2); 24,000 bodies
+// 0.313 and 0.305 (1.05), 0.87 and 1.2 (0.5).
+bool by_wavefronts(size_t n, double theta2) { return n <= 16384 || (n <= kWaveMax && theta2 <= 1.44); }
+
 }  // namespace
 
 void launch_walk_plain(const Bodies& b, size_t n, const TreeBuffers& tb, const WalkParams& p,
@@ -168,7 +468,12 @@ void launch_walk_plain(const Bodies& b, size_t n, const TreeBuffers& tb, const W
     if (cnt_accept && cnt_open && cnt_test)
         k_walk_plain<true><<<grid, kNT, 0, s>>>(b, n, g, tb.walk, tb.self_w, tb.sc, tb.sys, p, cnt_accept, cnt_open,
                                                 cnt_test);
-    else
+    else if (by_wavefronts(n, p.theta2)) {
+        const uint32_t words = static_cast<uint32_t>((2 * n + 63) / 64);
+        const uint32_t gw = static_cast<uint32_t>((n + kWaves - 1) / kWaves);
+        k_walk_wave<<<(gw + kXcds - 1) / kXcds * kXcds, 64 * kWaves, kWaves * words * sizeof(uint64_t), s>>>(
+            b, n, gw, tb.walk, tb.self_w, tb.sc, p, words);
+    } else
         k_walk_plain<false><<<grid, kNT, 0, s>>>(b, n, g, tb.walk, tb.self_w, tb.sc, tb.sys, p, nullptr, nullptr,
                                                  nullptr);
 }

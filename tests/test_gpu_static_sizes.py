@@ -3,11 +3,12 @@ the merge sort alone, whose rounds end in one or the other buffer (one tile to
 2,048 keys, one round to 32,768, two above), and sums a small tree's moments in
 one workgroup.  Bits equal a context's evaluation with the radix sort and one
 moment launch per depth, whatever the input order and with equal keys."""
-import ctypes as C
 import sys
 
 import numpy as np
 import pytest
+
+from test_zz_no_alloc import Hip
 
 pytestmark = pytest.mark.gpu
 
@@ -18,8 +19,6 @@ def say(*a):
 
 @pytest.mark.parametrize("n", [1, 2, 65, 2047, 2048, 2049, 4096, 4097, 32767, 32768, 32769, 65535, 65536])
 def test_static_sizes_match_full_sort_and_levels(bh, n):
-    import torch
-
     say("static evaluation", n, "bodies")
     rng = np.random.default_rng(n)
     pos, vel, m = (a[:n] for a in bh.generate(bh.GEN_TROJAN, 7, max(n, 65)))
@@ -36,13 +35,13 @@ def test_static_sizes_match_full_sort_and_levels(bh, n):
         st = e.get_bodies()
     want = np.empty_like(pos)
     want[st["ids"].astype(np.int64)] = st["acc"]
-    dpos, dm = torch.from_numpy(pos).cuda(), torch.from_numpy(m).cuda()
-    dacc = torch.full((n, 3), np.nan, dtype=torch.float64, device="cuda")
-    torch.cuda.synchronize()
-    lib = bh.load()
-    rc = lib.bh_compute_accelerations_static(n, C.c_void_p(dpos.data_ptr()), C.c_void_p(dm.data_ptr()), 0.9, bh.G,
-                                             0.0, C.c_void_p(dacc.data_ptr()), None)
-    assert rc == 0, lib.bh_static_last_error()
-    torch.cuda.synchronize()
-    got = dacc.cpu().numpy()
+    hip = Hip(bh)
+    try:
+        dpos, dm, dacc = hip.put(pos), hip.put(m), hip.put(np.full((n, 3), np.nan))
+        rc = bh.load().bh_compute_accelerations_static(n, dpos, dm, 0.9, bh.G, 0.0, dacc, None)
+        assert rc == 0, bh.load().bh_static_last_error()
+        hip.sync()
+        got = hip.get(dacc, (n, 3))
+    finally:
+        hip.free()
     assert np.array_equal(got.view(np.uint64), want.view(np.uint64))
