@@ -293,7 +293,7 @@ int run_force(bh_ctx* c, int form, double theta, double G, double soft2, bool ki
         MARK(3);
         bh::MixedParams mp{theta * theta, G, soft2, half_dt, c->mac_alpha, kick_after ? 1 : 0,
                            sched == BH_SCHED_KEY_ORDER ? 0 : (split ? 2 : 1), n_chunks, order_max,
-                           c->heavy_items};
+                           c->heavy_items, training ? 1 : 0};
         // the heavy bodies' chunk sums: at most 2 per walk wave run in the
         // walk's tail (waves whose groups are done take them: -14 us at 300k);
         // more (+6% walk at 2M, where the tail is short) get their own launch.
@@ -1307,6 +1307,13 @@ int bh_autotune(bh_ctx* c, int form, int reps, bh_tune_result* out)
             best_pick_ms = k.ms;
             have = true;
         }
+    }
+    // Where all candidates are within noise of each other the rule may pick one
+    // that timed slower than the default shape: the default is kept then.
+    if (have && best_pick_ms > def_ms && def_ms > 0.0) {
+        best = def;
+        best_blocks = c->mixed_blocks_max;
+        best_pick_ms = def_ms;
     }
     if (have) best_ms = best_pick_ms;
     c->sched = saved_sched;
