@@ -488,6 +488,7 @@ struct MixedParams {
     uint32_t n_chunks;    // chunks of the split schedule
     uint32_t order_max_groups;   // sched 1 falls back to key order above this many groups
     uint32_t heavy_items; // work items of the heavy direct sums over all systems
+    int count_narrow;     // a training walk: the groups' work in the narrow order (pop_count)
 };
 
 // Walk-group shape, the tunables of the mixed walk: at most gmax (<= 64)

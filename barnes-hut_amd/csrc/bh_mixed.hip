@@ -62,10 +62,26 @@ constexpr uint32_t kShareNum = 3, kShareDen = 5;
 constexpr int kListCap = 256;
 constexpr int kListPad = 64;    // zero entries past a flushed list (share_len)
 constexpr int kStackCap = 1024;
-// Up to 64 ranges may be popped while the stack holds at most this many
-// entries: one round pushes at most 8 ranges per popped range, and a
-// single-range round (pure depth first) grows the stack by at most 7 per level.
-constexpr int kBigPopLimit = kStackCap - 7 * 64 - 8 * 22;   // see the pop rule in k_walk_mixed
+// One round pushes at most 8 ranges per popped range, and a single-range round
+// (pure depth first) grows the stack by at most 7 per level: P ranges may be
+// popped while 7 P more fit below the room of one descent.  (Popping 64 or,
+// near the limit, one at a time: a group of four far-apart planets, which opens
+// 33,000 nodes of a 300k belt, walked 5.7 nodes a round, 3.9 ms of a walk of
+// 3.8; with this rule it takes 0.4 ms and the walk 0.52.  A 64-system belt
+// ensemble of 3.8M bodies 18.7 -> 5.6 ms.  Groups that do not fill their stack
+// are walked as before.)
+// narrow: 64 or one at a time.  The work of a group, the target of the learned
+// form's training, depends on where the list is flushed and so on the order of
+// its entries: a training walk counts it in the narrow order, by a second pass
+// without forces over the groups for which the two differ.
+constexpr uint32_t kStackRoom = kStackCap - 8 * 22;
+constexpr uint32_t kNarrowRoom = kStackRoom - 7 * 64;   // both rules are the same up to here
+__device__ inline uint32_t pop_count(uint32_t sp, bool narrow)
+{
+    if (narrow) return sp <= kNarrowRoom ? min(sp, 64u) : 1u;
+    const uint32_t fit = sp < kStackRoom ? (kStackRoom - sp) / 7u : 0u;
+    return min(min(sp, 64u), max(fit, 1u));
+}
 constexpr uint32_t kNone = 0xffffffffu;
 // b/D at or below 0.8 keeps the monopole error bound of an accepted node
 // (which grows like (b/D)^2 / (1 - b/D)^2) small; above it, up to theta, the
@@ -312,12 +328,18 @@ __global__ __launch_bounds__(kNT) void k_group_marks(size_t n, TreeBuffers tb, M
     }
 }
 
-// A group is shared by a block's wavefronts when its work in the previous
-// walk exceeds this: kShare x (groups per wave) x (an even share of the walk
-// per wave).  See k_walk_mixed for the choice.
+// A group is shared by a block's wavefronts, and walked first, when its work in
+// the previous walk exceeds this: kShare x (groups per wave) x (an even share of
+// the walk per wave), see kShareNum; with many groups per wave an eighth of an
+// even share and four times the mean, which only the groups of far-apart heavy
+// bodies exceed.  (One that starts late ends late: the 64-system ensemble's walk
+// 5.6 -> 4.25 ms with two such groups.)
 __device__ inline uint64_t share_limit(const StepScalars* sc, uint32_t walk_waves)
 {
-    return sc->work_prev * sc->groups_prev * kShareNum / (static_cast<uint64_t>(walk_waves) * walk_waves * kShareDen);
+    const uint64_t even = sc->work_prev / walk_waves;
+    const uint64_t many = sc->work_prev * sc->groups_prev * kShareNum / (static_cast<uint64_t>(walk_waves) * walk_waves * kShareDen);
+    const uint64_t mean = sc->work_prev / max(sc->groups_prev, 1u);
+    return min(many, max(even / 8u, 4u * mean));
 }
 
 __device__ inline void group_first(size_t i, size_t n, uint32_t gid, const Bodies& b, const TreeBuffers& tb,
@@ -329,7 +351,7 @@ __device__ inline void group_first(size_t i, size_t n, uint32_t gid, const Bodie
         bool big = tb.sc->work_prev != 0u && b.pcost[i] > share_limit(tb.sc, mb.walk_waves);
         if (big) {
             const uint32_t k = atomicAdd(&tb.sc->n_big, 1u);
-            big = k < kMaxShared;   // (at most waves^2 / (kShare x groups) exceed the limit)
+            big = k < kMaxShared;   // (at most waves^2 / (kShare x groups) or 8 x waves exceed the limit)
             if (big) mb.chunk[k] = gid;
         }
         mb.gbig[gid] = big ? 1u : 0u;
@@ -961,6 +983,8 @@ __device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, 
             const double qlim = (alpha > 0.0 && aref > 0.0 && aref < INFINITY) ? alpha * aref : INFINITY;
             // up to theta^2 = kSafe2 (and without a limit) the extent test implies the rest
             const bool relative = theta2 > kSafe2 && __any(qlim < INFINITY);
+            bool deep = false;      // the stack was over kNarrowRoom
+            bool recount = false;   // the second pass of a training walk
             if (tid == 0) stk[0] = stack_range(gsys, 1, false);   // the root of the group's system
             group_sync<NW>();   // (also: every wavefront has read the exchanged sums)
             for (bool last = false; !last;) {
@@ -969,7 +993,8 @@ __device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, 
                 last = sp == 0u || overflow;
                 Ranges r{0u, 0u, 0u, 0u};
                 if (!last) {
-                    const uint32_t P = (sp <= static_cast<uint32_t>(kBigPopLimit)) ? min(sp, 64u) : 1u;
+                    deep |= sp > kNarrowRoom;
+                    const uint32_t P = pop_count(sp, recount);
                     const bool has = static_cast<uint32_t>(lane) < P;
                     const uint32_t e = has ? stk[sp - 1 - lane] : 0u;
                     sp -= P;
@@ -1099,7 +1124,7 @@ __device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, 
                                 group_sync<NW>();
     #pragma unroll
                                 for (int v = 0; v < V; ++v) {
-                                    if (static_cast<uint32_t>((v * NW + w) * 64) < S * cnt) {
+                                    if (!recount && static_cast<uint32_t>((v * NW + w) * 64) < S * cnt) {
                                         const int src = static_cast<int>(vl[v] & 0xffu);
                                         share_sum(list + (vl[v] >> 8) * len, len, __shfl(ox, src, 64), __shfl(oy, src, 64),
                                                   __shfl(oz, src, 64), r2_0, acc[v]);
@@ -1133,6 +1158,13 @@ __device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, 
                     }
                     base += NW * 64u;
                 } while (base < r.total && !overflow);
+                if (last && deep && !recount && !overflow && args_here(args)->p.count_narrow != 0) {
+                    last = false;
+                    recount = true;
+                    sp = 1u;
+                    n_inter = n_visit = n_steps = 0u;
+                    if (tid == 0) stk[0] = stack_range(gsys, 1, false);
+                }
                 group_sync<NW>();   // the next round reads the stack
             }
             // the virtual lanes' sums (a Kahan sum's value is s - c: c holds the

@@ -273,7 +273,9 @@ int bh_get_group_timeline(bh_ctx *ctx, int64_t capacity, uint64_t *t_start, uint
  * model's target.  The list cost is its list entries per lane; in a group of
  * 33-63 bodies, whose idle lanes take over stretches of the list, only the
  * entries beyond the body lanes' stretches count (the ordering this gives
- * measured best).  Array sized by the group count of bh_get_groups. */
+ * measured best).  The list's entries are counted flush by flush; a LEARNED
+ * evaluation that trains counts a group with a full stack in the order of the
+ * depth-first walk.  Array sized by the group count of bh_get_groups. */
 int bh_get_group_work(bh_ctx *ctx, int64_t capacity, uint32_t *work);
 
 /* Estimated cost of each group of the last mixed walk, as its heaviest-first
