@@ -138,13 +138,13 @@ void scan_exclusive_u32(const uint32_t* in, uint32_t* out, uint32_t* total, size
 // its block's offset to the block-local scan (scan_block_excl).  Up to
 // kDirectTiles tiles the consumer's blocks add the sums of the tiles before
 // them themselves (at most 16 loads a thread, from L2), so no launch runs in
-// between; above that, scan_tile_offsets turns the sums into exclusive
-// offsets in place first (one block).  Either way the consumer writes the
+// between; above that, scan_tile_offsets first puts the exclusive offsets
+// behind the sums.  Either way the consumer writes the
 // total (its thread n - 1 holds it).  Every thread of the block calls the
 // block helpers.  tmp holds tile_sum_words(n) u32.
-inline size_t tile_sum_words(size_t n) { return (n + 255) / 256 + 1; }
 constexpr size_t kDirectTiles = 4096;
 __host__ __device__ inline bool scan_direct(size_t n) { return (n + 255) / 256 <= kDirectTiles; }
+inline size_t tile_sum_words(size_t n) { return (n + 255) / 256 * (scan_direct(n) ? 1 : 2) + 1; }
 // launches nothing when scan_direct(n)
 void scan_tile_offsets(uint32_t* tsum, size_t n, hipStream_t s);
 // out[i] = exclusive prefix of in[i] (blocks of 256); *total = the sum
@@ -181,7 +181,7 @@ __device__ inline uint32_t scan_block_excl(uint32_t v, const uint32_t* tsum, siz
     }
     if (lane == 63) w4[w] = inc;
     __syncthreads();
-    uint32_t off = direct ? p4[0] + p4[1] + p4[2] + p4[3] : tsum[blockIdx.x];
+    uint32_t off = direct ? p4[0] + p4[1] + p4[2] + p4[3] : tsum[(n + 255) / 256 + blockIdx.x];
     for (int q = 0; q < w; ++q) off += w4[q];
     return off + inc - v;
 }

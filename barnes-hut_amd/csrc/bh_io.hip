@@ -97,11 +97,67 @@ __device__ inline Pick block_heaviest(Pick p)
     return p;
 }
 
-// Candidates of one run of kHeavyRun rows: its kMaxHeavy heaviest, in order.
-// A thread holds its rows' masses in registers; each round it offers its
-// heaviest row that was not taken (rows are taken at most once).
-constexpr uint32_t kPerThread = kHeavyRun / kNT;
+// The `want` (<= kMaxHeavy) heaviest of the block's rows, in order, into
+// out[0, want) (kNoRow past the last): each thread has a share of the rows,
+// which rows(f) shows to f.  The heaviest rows of the block's kMaxHeavy sets of
+// 16 threads are kMaxHeavy rows, so a row less heavy than all of them is not
+// wanted; the others, some fifty of rows in no order, are gathered in LDS and
+// ranked by counting.  (Taking the heaviest row 16 times, with a reduction over
+// the block each, the two kernels below took 46 and 40 us at 19,054 bodies, now
+// 21 each.)  Only if more than kGather are left are they taken one by one.
+constexpr uint32_t kGather = 1024;
+static_assert(kNT == 16 * kMaxHeavy, "kMaxHeavy sets of 16 threads");
 
+template <typename Rows>
+__device__ inline void block_top(uint32_t want, Rows rows, Pick* out)
+{
+    __shared__ Pick top[kMaxHeavy], some[kGather];
+    __shared__ uint32_t n_some;
+    Pick p{0.0, kNoRow};
+    rows([&](const Pick& q) {
+        if (heavier(q, p)) p = q;
+    });
+    for (int o = 8; o > 0; o >>= 1) {
+        const Pick q{__shfl_xor(p.m, o, 64), static_cast<uint32_t>(__shfl_xor(static_cast<int>(p.i), o, 64))};
+        if (heavier(q, p)) p = q;
+    }
+    if (threadIdx.x % 16 == 0) top[threadIdx.x / 16] = p;
+    if (threadIdx.x == 0) n_some = 0;
+    __syncthreads();
+    Pick limit = top[0];   // (no row: a set without rows, then every row is gathered)
+#pragma unroll
+    for (int k = 1; k < kMaxHeavy; ++k)
+        if (heavier(limit, top[k])) limit = top[k];
+    rows([&](const Pick& q) {
+        if (q.i == kNoRow || heavier(limit, q)) return;
+        const uint32_t at = atomicAdd(&n_some, 1u);
+        if (at < kGather) some[at] = q;
+    });
+    __syncthreads();
+    const uint32_t n = n_some;
+    if (n <= kGather) {
+        for (uint32_t k = threadIdx.x; k < n; k += kNT) {
+            const Pick q = some[k];
+            uint32_t rank = 0;
+#pragma unroll 4
+            for (uint32_t t = 0; t < n; ++t) rank += heavier(some[t], q) ? 1u : 0u;
+            if (rank < want) out[rank] = q;
+        }
+        if (threadIdx.x >= n && threadIdx.x < want) out[threadIdx.x] = Pick{0.0, kNoRow};
+        return;
+    }
+    Pick last{0.0, kNoRow};
+    for (uint32_t r = 0; r < want; ++r) {
+        p = Pick{0.0, kNoRow};
+        rows([&](const Pick& q) {
+            if ((r == 0 || heavier(last, q)) && heavier(q, p)) p = q;
+        });
+        last = block_heaviest(p);
+        if (threadIdx.x == 0) out[r] = last;
+    }
+}
+
+// Candidates of one run of kHeavyRun rows: its kMaxHeavy heaviest, in order.
 __global__ __launch_bounds__(kNT) void k_heavy_candidates(const double* __restrict__ m, TreeBuffers tb,
                                                           const uint32_t* __restrict__ run_sys,
                                                           Pick* __restrict__ cand)
@@ -109,55 +165,38 @@ __global__ __launch_bounds__(kNT) void k_heavy_candidates(const double* __restri
     const SysScalars* sy = tb.sys + run_sys[2 * blockIdx.x];
     const uint32_t lo = sy->body_lo + run_sys[2 * blockIdx.x + 1] * kHeavyRun;
     const uint32_t hi = min(sy->body_hi, lo + kHeavyRun);
-    double v[kPerThread];
-    uint32_t free_rows = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kPerThread; ++k) {
-        const uint32_t i = lo + k * kNT + threadIdx.x;
-        v[k] = i < hi ? m[i] : 0.0;
-        if (i < hi) free_rows |= 1u << k;
-    }
-    for (int r = 0; r < kMaxHeavy; ++r) {
-        Pick p{0.0, kNoRow};
-#pragma unroll
-        for (uint32_t k = 0; k < kPerThread; ++k) {
-            const Pick q{v[k], (free_rows >> k) & 1u ? lo + k * kNT + threadIdx.x : kNoRow};
-            if (heavier(q, p)) p = q;
-        }
-        const Pick best = block_heaviest(p);
-        if (best.i != kNoRow && (best.i - lo) % kNT == threadIdx.x) free_rows &= ~(1u << ((best.i - lo) / kNT));
-        if (threadIdx.x == 0) cand[static_cast<size_t>(blockIdx.x) * kMaxHeavy + r] = best;
-    }
+    block_top(
+        kMaxHeavy,
+        [&](auto f) {
+#pragma unroll 8
+            for (uint32_t i = lo + threadIdx.x; i < hi; i += kNT) f(Pick{m[i], i});
+        },
+        cand + static_cast<size_t>(blockIdx.x) * kMaxHeavy);
 }
 
-// One block per system: the heaviest of its runs' candidates (each run's are
-// in order, so a run offers its first that was not taken), ranked by row.
+// One block per system: the heaviest of its runs' candidates, ranked by row.
 __global__ __launch_bounds__(kNT) void k_heavy_pick(Bodies b, TreeBuffers tb, const uint32_t* __restrict__ sys_run,
                                                     const Pick* __restrict__ cand)
 {
-    __shared__ uint32_t rows[kMaxHeavy];
+    __shared__ Pick best[kMaxHeavy];
     const uint32_t s = blockIdx.x, r0 = sys_run[s], r1 = sys_run[s + 1];
     const uint32_t nh = tb.sys[s].n_heavy;
-    Pick last{0.0, kNoRow};
-    for (uint32_t r = 0; r < nh; ++r) {
-        Pick p{0.0, kNoRow};
-        for (uint32_t run = r0 + threadIdx.x; run < r1; run += kNT) {
-            const Pick* c = cand + static_cast<size_t>(run) * kMaxHeavy;
-            for (int k = 0; k < kMaxHeavy; ++k) {   // its first after the last one taken
-                const Pick q = c[k];
-                if (r > 0 && !heavier(last, q)) continue;
-                if (heavier(q, p)) p = q;
-                break;
-            }
-        }
-        last = block_heaviest(p);
-        if (threadIdx.x == 0) rows[r] = last.i;
-    }
+    if (nh == 0) return;
+    // (consecutive runs go to different sets of 16 threads)
+    const uint32_t first = r0 + threadIdx.x % 16 * 16 + threadIdx.x / 16;
+    block_top(
+        nh,
+        [&](auto f) {
+            for (uint32_t run = first; run < r1; run += kNT)
+#pragma unroll 4
+                for (int k = 0; k < kMaxHeavy; ++k) f(cand[static_cast<size_t>(run) * kMaxHeavy + k]);
+        },
+        best);
     __syncthreads();
-    if (threadIdx.x < nh && rows[threadIdx.x] != kNoRow) {
+    if (threadIdx.x < nh && best[threadIdx.x].i != kNoRow) {
         uint32_t rank = 0;
-        for (uint32_t k = 0; k < nh; ++k) rank += rows[k] < rows[threadIdx.x] ? 1u : 0u;
-        b.hrank[rows[threadIdx.x]] = static_cast<int8_t>(rank);
+        for (uint32_t k = 0; k < nh; ++k) rank += best[k].i < best[threadIdx.x].i ? 1u : 0u;
+        b.hrank[best[threadIdx.x].i] = static_cast<int8_t>(rank);
     }
 }
 

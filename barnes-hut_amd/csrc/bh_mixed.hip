@@ -747,20 +747,9 @@ __device__ inline uint32_t part_blocks(uint32_t x, uint32_t nblk)
 }
 
 // Accelerations of the heavy bodies: an FP64 direct sum over every other
-// body (Neumaier-compensated per thread, partials combined in thread order).
+// body (compensated per thread, partials combined in thread order).
 // The heavy bodies are few and their net accelerations are small next to the
 // forces that cancel in them, so no tree truncation is taken for them.
-struct Neumaier {
-    double s = 0.0, c = 0.0;
-    __device__ void add(double x)
-    {
-        const double t = s + x;
-        if (fabs(s) >= fabs(x)) c += (s - t) + x;
-        else c += (x - t) + s;
-        s = t;
-    }
-    __device__ double value() const { return s + c; }
-};
 
 // 1 / sqrt(x) for x > 0: the hardware estimate refined by two Newton steps
 // y <- y (3/2 - x/2 y^2), each of which squares the relative error, instead
@@ -774,12 +763,20 @@ __device__ inline double rsqrt_f64(double x)
     return y;
 }
 
-// Work item w = (system s, heavy rank k, chunk c): heavy body k of system s
+// A partial sum (system s, heavy rank k, chunk c) is heavy body k of system s
 // summed over the c-th run of 1024 bodies of s by one wavefront -- each lane
-// a Neumaier sum over its stride, lane partials added in lane order -- and
+// a compensated sum over its stride, lane partials added in lane order -- and
 // k_heavy_final adds the chunk partials in chunk order.  A system's heavy
 // accelerations therefore depend on that system alone, not on the launch
 // shape or on the other systems of an ensemble.
+// A work item is kHeavyTogether ranks of a chunk: a body is loaded once for
+// all of them (one rank at a time read every body 16 times a step, 2.1 GB at
+// 4M bodies), and items in a row are the ranks of one chunk.  (In a launch of
+// their own: 4M bodies 0.307 -> 0.141 ms, 1M 0.068 -> 0.040; the FP64 work of
+// the pairs is 0.09 ms at 4M.)
+constexpr uint32_t kHeavyTogether = 4;
+static_assert(kMaxHeavy % kHeavyTogether == 0, "whole items");
+constexpr uint32_t kHeavyRow = 65;   // lane partials of a sum, padded for the banks
 struct HeavyArgs {
     const double *px, *py, *pz, *m;
     const SysScalars* sys;
@@ -788,44 +785,58 @@ struct HeavyArgs {
     double soft2, G;
 };
 
-__device__ inline void heavy_item(const HeavyArgs& ha, uint32_t item, int lane, double (*part)[64])
+__device__ inline void heavy_item(const HeavyArgs& ha, uint32_t item, int lane, double (*part)[kHeavyRow])
 {
     uint32_t lo = 0, hi = ha.n_sys;   // the last system whose first item is <= item
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (ha.sys[mid].heavy_item <= item) lo = mid;
+        if (ha.sys[mid].heavy_item / kHeavyTogether <= item) lo = mid;
         else hi = mid;
     }
     const SysScalars* sy = ha.sys + lo;
-    const uint32_t r = item - sy->heavy_item;
-    const uint32_t k = r / sy->heavy_chunks, c = r % sy->heavy_chunks;
-    if (k >= sy->n_heavy) return;
-    const uint32_t h = sy->heavy_slot[k];
-    const double x = ha.px[h], y = ha.py[h], z = ha.pz[h];
+    const uint32_t r = item - sy->heavy_item / kHeavyTogether;
+    constexpr uint32_t kSets = kMaxHeavy / kHeavyTogether;
+    const uint32_t k0 = r % kSets * kHeavyTogether, c = r / kSets, nh = sy->n_heavy;
+    if (k0 >= nh) return;
+    uint32_t h[kHeavyTogether];
+    double x[kHeavyTogether], y[kHeavyTogether], z[kHeavyTogether];
+    ExactSum a[kHeavyTogether][3];
+#pragma unroll
+    for (uint32_t q = 0; q < kHeavyTogether; ++q) {
+        h[q] = sy->heavy_slot[min(k0 + q, nh - 1)];
+        x[q] = ha.px[h[q]];
+        y[q] = ha.py[h[q]];
+        z[q] = ha.pz[h[q]];
+    }
     const size_t j0 = sy->body_lo + static_cast<size_t>(c) * kHeavyChunk;
     const size_t j1 = min(j0 + kHeavyChunk, static_cast<size_t>(sy->body_hi));
-    Neumaier ax, ay, az;
     // the heavy body itself and co-located bodies add an exact zero (a no-op
     // for the sums) instead of being skipped, so the loop unrolls and the
-    // square roots and divisions of consecutive bodies overlap
-#pragma unroll 4
+    // square roots of consecutive bodies overlap
+#pragma unroll 2
     for (size_t j = j0 + lane; j < j1; j += 64) {
-        const double dx = ha.px[j] - x, dy = ha.py[j] - y, dz = ha.pz[j] - z;
-        const double r2 = dx * dx + dy * dy + dz * dz + ha.soft2;
-        const double invR = rsqrt_f64(r2);
-        const double s = (j != h && r2 > 0.0) ? ha.G * ha.m[j] * (invR * invR * invR) : 0.0;
-        ax.add(s * dx);
-        ay.add(s * dy);
-        az.add(s * dz);
+        const double bx = ha.px[j], by = ha.py[j], bz = ha.pz[j], gm = ha.G * ha.m[j];
+#pragma unroll
+        for (uint32_t q = 0; q < kHeavyTogether; ++q) {
+            const double dx = bx - x[q], dy = by - y[q], dz = bz - z[q];
+            const double r2 = dx * dx + dy * dy + dz * dz + ha.soft2;
+            const double invR = rsqrt_f64(r2);
+            const double s = (j != h[q] && r2 > 0.0) ? gm * (invR * invR * invR) : 0.0;
+            a[q][0].add(s * dx);
+            a[q][1].add(s * dy);
+            a[q][2].add(s * dz);
+        }
     }
-    part[0][lane] = ax.value();
-    part[1][lane] = ay.value();
-    part[2][lane] = az.value();
+#pragma unroll
+    for (uint32_t q = 0; q < kHeavyTogether; ++q)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) part[3 * q + d][lane] = a[q][d].value();
     __builtin_amdgcn_wave_barrier();
-    if (lane < 3) {
-        Neumaier t;
+    const uint32_t k = k0 + static_cast<uint32_t>(lane) / 3u;
+    if (lane < 3 * static_cast<int>(kHeavyTogether) && k < nh) {
+        ExactSum t;
         for (int q = 0; q < 64; ++q) t.add(part[lane][q]);
-        ha.hpart[3 * static_cast<size_t>(item) + lane] = t.value();
+        ha.hpart[3 * (sy->heavy_item + static_cast<size_t>(k) * sy->heavy_chunks + c) + lane % 3] = t.value();
     }
     __builtin_amdgcn_wave_barrier();
 }
@@ -872,6 +883,7 @@ __device__ inline bool body_entry(WalkArgsP a, uint32_t j, double cx, double cy,
 constexpr int kListBytes = (kListCap + kListPad) * 16;
 constexpr int kWaveLds = kListBytes + kRoundSlots * 4 + kStackCap * 4;
 static_assert(kListBytes + kRoundSlots * 4 >= 768 * 8, "the exchanged sums fit");
+static_assert(kWaveLds >= 3 * kHeavyTogether * kHeavyRow * 8, "a heavy item's lane partials fit");
 
 // Walks group g by NW wavefronts (1: this one alone; 4: the block's, this one
 // the w-th) and returns its work.  turn_no: exchanges so far (which of the two
@@ -1374,7 +1386,7 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3))) void k
     // of the LDS holds the lane partials).  When the blocks with a group leave
     // enough waves, the items go to the last waves of the grid without a queue.
     const WalkArgsP at = args_here(args);
-    const uint32_t items = at->p.heavy_items;
+    const uint32_t items = at->p.heavy_items / kHeavyTogether;
     const HeavyArgs ha{at->b.px, at->b.py, at->b.pz, at->b.m, at->tb.sys, at->tb.n_sys, at->mb.hpart, at->p.soft2, at->p.G};
     const bool fixed = C == G && static_cast<uint64_t>(G) * kWaves + items <= waves;
     for (uint32_t k = 0;; ++k) {
@@ -1387,21 +1399,21 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3))) void k
         }
         q = uni(q);
         if (q >= items) break;
-        heavy_item(ha, q, lane, reinterpret_cast<double(*)[64]>(s_mem + w * kWaveLds));
+        heavy_item(ha, q, lane, reinterpret_cast<double(*)[kHeavyRow]>(s_mem + w * kWaveLds));
     }
 }
 
 __global__ __launch_bounds__(kNT) void k_heavy_partial(Bodies b, TreeBuffers tb, MixedBuffers mb, MixedParams p)
 {
-    __shared__ double part[kWaves][3][64];
+    __shared__ double part[kWaves][3 * kHeavyTogether][kHeavyRow];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t waves = gridDim.x * kWaves;
-    for (uint32_t item = blockIdx.x * kWaves + w; item < p.heavy_items; item += waves)
+    for (uint32_t item = blockIdx.x * kWaves + w; item < p.heavy_items / kHeavyTogether; item += waves)
         heavy_item(HeavyArgs{b.px, b.py, b.pz, b.m, tb.sys, tb.n_sys, mb.hpart, p.soft2, p.G}, item, lane, part[w]);
 }
 
 // One wavefront per (system, heavy rank, axis): lane l adds the chunk
-// partials l, l + 64, ... (Neumaier), then the 64 lane sums are added in lane
+// partials l, l + 64, ... (compensated), then the 64 lane sums are added in lane
 // order -- a fixed order for a given system.
 __global__ __launch_bounds__(kNT) void k_heavy_final(Bodies b, TreeBuffers tb, MixedBuffers mb, MixedParams p)
 {
@@ -1417,7 +1429,7 @@ __global__ __launch_bounds__(kNT) void k_heavy_final(Bodies b, TreeBuffers tb, M
     double* accel = a == 0 ? b.ax : (a == 1 ? b.ay : b.az);
     double* vel = a == 0 ? b.vx : (a == 1 ? b.vy : b.vz);
     const double v_old = (p.kick && lane == 0) ? vel[h] : 0.0;   // loaded beside the partials
-    Neumaier acc;
+    ExactSum acc;
     const size_t first = item0 + static_cast<size_t>(k) * nc;
     // eight partials loaded per round before they are added (in chunk order)
     for (uint32_t c0 = static_cast<uint32_t>(lane); c0 < nc; c0 += 64 * 8) {
@@ -1434,7 +1446,7 @@ __global__ __launch_bounds__(kNT) void k_heavy_final(Bodies b, TreeBuffers tb, M
     lanes[w][lane] = acc.value();
     __builtin_amdgcn_wave_barrier();
     if (lane != 0) return;
-    Neumaier tot;
+    ExactSum tot;
     for (int l = 0; l < 64; ++l) tot.add(lanes[w][l]);
     const double v = tot.value();
     accel[h] = v;
@@ -1631,7 +1643,7 @@ void launch_heavy_direct(const Bodies& b, const TreeBuffers& tb, const MixedBuff
                          bool in_walk, hipStream_t s)
 {
     if (p.heavy_items == 0) return;
-    const unsigned hb = std::min<unsigned>((p.heavy_items + kWaves - 1) / kWaves, 4096u);
+    const unsigned hb = std::min<unsigned>((p.heavy_items / kHeavyTogether + kWaves - 1) / kWaves, 4096u);
     if (!in_walk) k_heavy_partial<<<hb, kNT, 0, s>>>(b, tb, mb, p);
     k_heavy_final<<<(tb.n_sys * 3 * kMaxHeavy + kWaves - 1) / kWaves, kNT, 0, s>>>(b, tb, mb, p);
 }

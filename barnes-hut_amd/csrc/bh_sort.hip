@@ -260,6 +260,31 @@ __global__ __launch_bounds__(kWideNT) void k_scan_sums_wide(uint32_t* __restrict
     if (threadIdx.x == 0 && total_out) *total_out = carry;
 }
 
+// Exclusive offsets of nt tile sums into off: a block adds up the sums before
+// its own 1,024 itself, so that no block waits for another (16,384 sums: one
+// block scanning them all in place 33 us, 16 blocks 18).
+__global__ __launch_bounds__(kWideNT) void k_tile_offsets(const uint32_t* __restrict__ sums, size_t nt,
+                                                          uint32_t* __restrict__ off)
+{
+    __shared__ uint32_t before[kWideNT / 64], own[kWideNT / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t b0 = static_cast<size_t>(blockIdx.x) * kWideNT, i = b0 + threadIdx.x;
+    const uint32_t v = i < nt ? sums[i] : 0u;
+    uint32_t pre = 0;
+#pragma unroll 8
+    for (size_t k = threadIdx.x; k < b0; k += kWideNT) pre += sums[k];
+    for (int o = 32; o > 0; o >>= 1) pre += static_cast<uint32_t>(__shfl_xor(static_cast<int>(pre), o, 64));
+    const uint32_t inc = wave_inclusive_scan(v);
+    if (lane == 63) {
+        before[w] = pre;
+        own[w] = inc;
+    }
+    __syncthreads();
+    uint32_t e = inc - v;
+    for (int k = 0; k < kWideNT / 64; ++k) e += before[k] + (k < w ? own[k] : 0u);
+    if (i < nt) off[i] = e;
+}
+
 __global__ __launch_bounds__(256) void k_tile_apply256(const uint32_t* __restrict__ in, size_t n,
                                                        const uint32_t* __restrict__ tsum, uint32_t* __restrict__ out,
                                                        uint32_t* __restrict__ total)
@@ -843,28 +868,102 @@ __device__ inline bool ms_less(uint32_t sa, uint64_t ka, uint32_t va, uint32_t s
     return ka < kb || (ka == kb && va < vb);
 }
 
-// v of lane (lane ^ mask), for a mask that is a compile-time constant once
-// the caller's loops unroll: distances 1 and 2 by DPP quad permutations,
-// 4 to 16 by swizzles inside each half-wave (bitmask mode: lane ^ mask),
-// 32 by a permute.
-__device__ inline uint32_t lane_xor(uint32_t v, int mask)
+// v of lane (lane ^ kMask): distances 1 and 2 by DPP quad permutations, 4 to
+// 16 by swizzles inside each half-wave (bitmask mode: lane ^ mask), 32 by a
+// permute.
+template <int kMask>
+__device__ inline uint32_t lane_xor(uint32_t v)
 {
     const int x = static_cast<int>(v);
-    switch (mask) {
-    case 1: return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false));   // [1,0,3,2]
-    case 2: return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false));   // [2,3,0,1]
-    case 4: return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(x, 0x1F | (4 << 10)));
-    case 8: return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(x, 0x1F | (8 << 10)));
-    case 16: return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(x, 0x1F | (16 << 10)));
-    default: return static_cast<uint32_t>(__shfl_xor(x, mask, 64));
+    if constexpr (kMask == 1) return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false));   // [1,0,3,2]
+    else if constexpr (kMask == 2) return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false));   // [2,3,0,1]
+    else if constexpr (kMask < 32) return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(x, 0x1F | (kMask << 10)));
+    else return static_cast<uint32_t>(__shfl_xor(x, kMask, 64));
+}
+
+// A thread's two elements of the tile sort.
+struct TilePair {
+    uint64_t k[2];
+    uint32_t v[2], s[2];
+};
+
+// element e keeps the smaller of (e, e ^ j) when e is the lower index of an
+// ascending pair or the upper of a descending one
+template <bool kSys>
+__device__ inline void keep(TilePair& t, const TilePair& p, bool keep_min)
+{
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (keep_min == ms_less<kSys>(p.s[i], p.k[i], p.v[i], t.s[i], t.k[i], t.v[i])) {
+            t.k[i] = p.k[i];
+            t.v[i] = p.v[i];
+            t.s[i] = p.s[i];
+        }
     }
 }
 
-__device__ inline uint64_t shfl_xor_u64(uint64_t x, int mask)
+// the phase of partner distance 2 kMask: lane ^ kMask
+template <bool kSys, int kMask>
+__device__ inline void lane_phase(TilePair& t, uint32_t k, uint32_t e0, bool asc)
 {
-    const uint32_t lo = lane_xor(static_cast<uint32_t>(x), mask);
-    const uint32_t hi = lane_xor(static_cast<uint32_t>(x >> 32), mask);
-    return (static_cast<uint64_t>(hi) << 32) | lo;
+    if (2u * kMask >= k) return;
+    TilePair p;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        p.k[i] = static_cast<uint64_t>(lane_xor<kMask>(static_cast<uint32_t>(t.k[i] >> 32))) << 32 |
+                 lane_xor<kMask>(static_cast<uint32_t>(t.k[i]));
+        p.v[i] = lane_xor<kMask>(t.v[i]);
+        p.s[i] = kSys ? lane_xor<kMask>(t.s[i]) : 0u;
+    }
+    keep<kSys>(t, p, ((e0 & (2u * kMask)) == 0) == asc);
+}
+
+// The stages from k on, up to the tile's count: what lies above is padding (366
+// keys: 11.8 -> 9.0 us).  Unrolled, every partner distance a constant (as loops
+// a full tile takes 14.7 us instead of 12.4).
+template <bool kSys, uint32_t k>
+__device__ inline void tile_stages(TilePair& t, uint32_t cnt, uint32_t e0, uint64_t* sk, uint32_t* sv, uint8_t* ss)
+{
+    if (k >= 2u * cnt) return;
+    const bool asc = (e0 & k) == 0;   // the same for both elements: k >= 2
+#pragma unroll
+    for (uint32_t j = k >> 1; j >= 128; j >>= 1) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            sk[e0 + i] = t.k[i];
+            sv[e0 + i] = t.v[i];
+            if (kSys) ss[e0 + i] = static_cast<uint8_t>(t.s[i]);
+        }
+        __syncthreads();
+        TilePair p;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t q = (e0 + i) ^ j;
+            p.k[i] = sk[q];
+            p.v[i] = sv[q];
+            p.s[i] = kSys ? ss[q] : 0u;
+        }
+        __syncthreads();
+        keep<kSys>(t, p, ((e0 & j) == 0) == asc);
+    }
+    lane_phase<kSys, 32>(t, k, e0, asc);
+    lane_phase<kSys, 16>(t, k, e0, asc);
+    lane_phase<kSys, 8>(t, k, e0, asc);
+    lane_phase<kSys, 4>(t, k, e0, asc);
+    lane_phase<kSys, 2>(t, k, e0, asc);
+    lane_phase<kSys, 1>(t, k, e0, asc);
+    const bool sw = asc ? ms_less<kSys>(t.s[1], t.k[1], t.v[1], t.s[0], t.k[0], t.v[0])
+                        : ms_less<kSys>(t.s[0], t.k[0], t.v[0], t.s[1], t.k[1], t.v[1]);
+    if (sw) {
+        const TilePair u = t;
+        t.k[0] = u.k[1];
+        t.v[0] = u.v[1];
+        t.s[0] = u.s[1];
+        t.k[1] = u.k[0];
+        t.v[1] = u.v[0];
+        t.s[1] = u.s[0];
+    }
+    if constexpr (2u * k <= kMsTile) tile_stages<kSys, 2u * k>(t, cnt, e0, sk, sv, ss);
 }
 
 template <bool kSys>
@@ -873,91 +972,27 @@ __device__ inline void tile_sort(const uint64_t* ik, const uint32_t* iv,
                                  uint32_t m, size_t t0, uint64_t* sk, uint32_t* sv, uint8_t* ss)
 {
     const uint32_t e0 = 2u * threadIdx.x;
-    uint64_t kk[2];
-    uint32_t vv[2], sy[2];
+    TilePair t;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const size_t x = t0 + e0 + i;
         if (x < m) {
-            kk[i] = ik[x];
-            vv[i] = iv[x];
-            sy[i] = kSys ? sysd[vv[i]] : 0u;
+            t.k[i] = ik[x];
+            t.v[i] = iv[x];
+            t.s[i] = kSys ? sysd[t.v[i]] : 0u;
         } else {   // padding above every real entry
-            kk[i] = ~0ull;
-            vv[i] = ~0u;
-            sy[i] = 0xffu;
+            t.k[i] = ~0ull;
+            t.v[i] = ~0u;
+            t.s[i] = 0xffu;
         }
     }
-    // fully unrolled: every partner distance is a constant, so the lane
-    // exchanges compile to swizzles and the phase branches disappear
-#pragma unroll
-    for (uint32_t k = 2; k <= kMsTile; k <<= 1) {
-        const bool asc = (e0 & k) == 0;   // the same for both elements: k >= 2
-#pragma unroll
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            if (j == 1) {
-                const bool sw = asc ? ms_less<kSys>(sy[1], kk[1], vv[1], sy[0], kk[0], vv[0])
-                                    : ms_less<kSys>(sy[0], kk[0], vv[0], sy[1], kk[1], vv[1]);
-                if (sw) {
-                    const uint64_t tk = kk[0];
-                    kk[0] = kk[1];
-                    kk[1] = tk;
-                    const uint32_t tv = vv[0];
-                    vv[0] = vv[1];
-                    vv[1] = tv;
-                    const uint32_t ts = sy[0];
-                    sy[0] = sy[1];
-                    sy[1] = ts;
-                }
-                continue;
-            }
-            // element e keeps the smaller of (e, e ^ j) when e is the lower
-            // index of an ascending pair or the upper of a descending one
-            const bool keep_min = ((e0 & j) == 0) == asc;
-            uint64_t pk[2];
-            uint32_t pv[2], ps[2];
-            if (j < 128) {
-                const int mask = static_cast<int>(j >> 1);   // partner lane: lane ^ j / 2
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    pk[i] = shfl_xor_u64(kk[i], mask);
-                    pv[i] = lane_xor(vv[i], mask);
-                    ps[i] = kSys ? lane_xor(sy[i], mask) : 0u;
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    sk[e0 + i] = kk[i];
-                    sv[e0 + i] = vv[i];
-                    if (kSys) ss[e0 + i] = static_cast<uint8_t>(sy[i]);
-                }
-                __syncthreads();
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const uint32_t q = (e0 + i) ^ j;
-                    pk[i] = sk[q];
-                    pv[i] = sv[q];
-                    ps[i] = kSys ? ss[q] : 0u;
-                }
-                __syncthreads();
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const bool p_less = ms_less<kSys>(ps[i], pk[i], pv[i], sy[i], kk[i], vv[i]);
-                if (keep_min == p_less) {
-                    kk[i] = pk[i];
-                    vv[i] = pv[i];
-                    sy[i] = ps[i];
-                }
-            }
-        }
-    }
+    tile_stages<kSys, 2>(t, static_cast<uint32_t>(min(static_cast<size_t>(kMsTile), m - t0)), e0, sk, sv, ss);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const size_t x = t0 + e0 + i;
         if (x < m) {
-            k1[x] = kk[i];
-            v1[x] = vv[i];
+            k1[x] = t.k[i];
+            v1[x] = t.v[i];
         }
     }
 }
@@ -994,7 +1029,9 @@ __global__ __launch_bounds__(kMsNT) void k_ns_tile_sort(const uint64_t* k0, cons
 // q lies within S - 1 entries after the last sample below it, found by
 // lockstep binary searches in LDS, and the last log2(S) steps search those
 // entries in memory (the loads of one step issued together).  Three
-// dependent memory rounds for L = 2048 instead of twelve.
+// dependent memory rounds for L = 2048 instead of twelve.  (The LDS steps are
+// a loop: unrolled they made 35 KB of code and 20% more registers; 274,000
+// removed keys of 4M: 92 -> 57 us a round.)
 constexpr uint32_t kMsSamples = 256;
 constexpr int kMsSampleSteps = 9;   // floor(log2(kMsSamples)) + 1
 
@@ -1016,7 +1053,7 @@ __device__ inline void merge_one(const uint64_t* __restrict__ ik, const uint32_t
         slo[q] = 0;
         slen[q] = (static_cast<uint32_t>(q) == r || gstart + static_cast<size_t>(q) * L >= m) ? 0u : kMsSamples;
     }
-#pragma unroll
+#pragma unroll 1
     for (int it = 0; it < kMsSampleSteps; ++it) {
 #pragma unroll
         for (int q = 0; q < kMsWays; ++q) {
@@ -1252,8 +1289,7 @@ void scan_tile_offsets(uint32_t* tsum, size_t n, hipStream_t s)
 {
     if (scan_direct(n)) return;
     const size_t nt = (n + 255) / 256;
-    if (nt <= static_cast<size_t>(kTile)) k_scan_sums<<<1, kNT, 0, s>>>(tsum, nt, nullptr);
-    else k_scan_sums_wide<<<1, kWideNT, 0, s>>>(tsum, nt, nullptr);
+    k_tile_offsets<<<static_cast<unsigned>((nt + kWideNT - 1) / kWideNT), kWideNT, 0, s>>>(tsum, nt, tsum + nt);
 }
 
 void scan_tile_apply(const uint32_t* in, size_t n, const uint32_t* tsum, uint32_t* out, uint32_t* total,

@@ -557,8 +557,7 @@ __global__ __launch_bounds__(kNT) void k_link(size_t n, TreeBuffers tb)
 // Moments of branching node bi from its existing children, summed in octant
 // order 0..7 from 0.0 (src/linear_octree.cpp:69-87): the plain form's raw
 // moments (the mixed forms take their light moments from the pyramid below).
-// Every child's values are loaded before the first sum (an empty octant loads
-// the node's first child again and is then skipped), so one node costs two
+// Every child's values are loaded before the first sum, so one node costs two
 // dependent memory round trips, not one per child.
 struct ChildSet {
     int4 a, b;
@@ -573,15 +572,10 @@ __device__ inline ChildSet child_set(const TreeBuffers& tb, size_t bi)
 __device__ inline void node_moments(const TreeBuffers& tb, uint32_t M, size_t bi, const ChildSet& cs)
 {
     const int32_t c[8] = {cs.a.x, cs.a.y, cs.a.z, cs.a.w, cs.b.x, cs.b.y, cs.b.z, cs.b.w};
-    int32_t any = c[0];
-#pragma unroll
-    for (int k = 1; k < 8; ++k) any = (any < 0) ? c[k] : any;
-    size_t ix[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) ix[k] = static_cast<size_t>(c[k] < 0 ? any : c[k]);
     double4 r[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) r[k] = reinterpret_cast<const double4*>(tb.raw)[ix[k]];
+    for (int k = 0; k < 8; ++k)
+        if (c[k] >= 0) r[k] = reinterpret_cast<const double4*>(tb.raw)[c[k]];
     double sm = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -618,6 +612,7 @@ __device__ inline void moments_listed(const TreeBuffers& tb)
 {
     __shared__ uint32_t sn[kDeepLds];
     __shared__ uint32_t s_end[kMaxDepth + 1];   // list positions where each depth's nodes end
+    __shared__ uint32_t s_put[kMaxDepth + 1];
     const uint32_t M = tb.sc->n_leaves, nd = tb.sc->n_deep;
     if (nd == 0) return;
     if (nd > kDeepLds) {
@@ -632,33 +627,20 @@ __device__ inline void moments_listed(const TreeBuffers& tb)
     }
     if (threadIdx.x <= kMaxDepth) s_end[threadIdx.x] = 0;
     __syncthreads();
-    constexpr int kPer = static_cast<int>(kDeepLds / kDeepNT);
-    uint32_t node[kPer], at[kPer];   // this thread's nodes, their depths and ranks within them
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const uint32_t k = threadIdx.x + static_cast<uint32_t>(q) * kDeepNT;
-        node[q] = k < nd ? tb.deep[k] : kNone;
-    }
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        at[q] = 0;
-        if (node[q] == kNone) continue;
-        const uint32_t d = tb.bdepth[node[q]];
-        at[q] = d << 16 | atomicAdd(&s_end[d], 1u);
-    }
+    for (uint32_t k = threadIdx.x; k < nd; k += kDeepNT) atomicAdd(&s_end[tb.bdepth[tb.deep[k]]], 1u);
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t e = 0;
         for (int d = kMaxDepth; d >= 0; --d) {
+            s_put[d] = e;
             e += s_end[d];
             s_end[d] = e;
         }
     }
     __syncthreads();
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const uint32_t d = at[q] >> 16;
-        if (node[q] != kNone) sn[(d < kMaxDepth ? s_end[d + 1] : 0u) + (at[q] & 0xffffu)] = node[q];
+    for (uint32_t k = threadIdx.x; k < nd; k += kDeepNT) {
+        const uint32_t b = tb.deep[k];
+        sn[atomicAdd(&s_put[tb.bdepth[b]], 1u)] = b;
     }
     __syncthreads();
     uint32_t lo = 0, bi = kNone;
