@@ -85,6 +85,7 @@ struct bh_ctx {
     bool have_counts = false;
     bool have_groups = false;
     bool prev_counts = false;         // the bodies carry the walk work of an earlier mixed walk
+    bool sorted_whole = false;        // the last sort was sort_small
     bool evaluated = false;           // a force evaluation has permuted the bodies since bh_set_bodies
     hipEvent_t ev[5] = {};
     // per-step phase events of bh_step: ring of kRing sets of 5
@@ -227,7 +228,11 @@ int run_force(bh_ctx* c, int form, double theta, double G, double soft2, bool ki
     bh::launch_kick_drift_box(c->cur, c->n, kick_before, half_dt, drift, dt, c->tb, c->partials, s);
     bh::launch_keys(c->cur, c->n, c->tb, c->partials, s);
     MARK(1);
-    if (c->sort_near)
+    c->sorted_whole = c->sort_near && ev && !c->evaluated && c->n <= bh::kSortSmall;   // (no graph is captured)
+    if (c->sorted_whole)
+        bh::sort_small(c->tb.key, c->tb.perm, c->tb.key_alt, c->tb.perm_alt, c->n,
+                       c->n_sys > 1 ? c->tb.bsys : nullptr, s);
+    else if (c->sort_near)
         bh::sort_near_sorted(c->tb.key, c->tb.perm, c->tb.key_alt, c->tb.perm_alt, c->tb.key_alt2, c->tb.perm_alt2,
                              c->n, 63, c->n_sys > 1 ? c->tb.bsys : nullptr, c->tb.sort_tmp, c->cap, s);
     else
@@ -709,6 +714,7 @@ int graph_step(bh_ctx* c, double dt)
         c->gkey[p] = key;
     }
     HIP_TRY(c, hipGraphLaunch(c->gexec[p], c->stream));
+    c->sorted_whole = false;
     std::swap(c->cur, c->alt);
     c->parity ^= 1;
     c->have_tree = c->cfg.form == BH_FORM_PLAIN;
@@ -1366,8 +1372,9 @@ int bh_get_sort_stats(bh_ctx* c, int* near_path, int64_t* sorted_keys)
     uint32_t ctl[4] = {0, 0, 0, 0};
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     HIP_TRY(c, hipMemcpy(ctl, bh::sort_near_ctl(c->tb.sort_tmp, c->cap), sizeof(ctl), hipMemcpyDeviceToHost));
-    if (near_path) *near_path = c->sort_near ? static_cast<int>(ctl[0]) : 0;
-    if (sorted_keys) *sorted_keys = c->sort_near ? (ctl[0] ? ctl[3] : static_cast<int64_t>(c->n)) : static_cast<int64_t>(c->n);
+    const bool near = c->sort_near && !c->sorted_whole;
+    if (near_path) *near_path = near ? static_cast<int>(ctl[0]) : 0;
+    if (sorted_keys) *sorted_keys = near ? (ctl[0] ? ctl[3] : static_cast<int64_t>(c->n)) : static_cast<int64_t>(c->n);
     return BH_OK;
 }
 

@@ -281,9 +281,13 @@ void radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, si
 // the rest is not in order.  Buffers (k1, v1) and (k2, v2) hold n entries.
 void sort_near_sorted(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint64_t* k2, uint32_t* v2, size_t n,
                       int bits, const uint8_t* sysd, uint32_t* tmp, size_t cap, hipStream_t s);
-// The same order for keys in any order, n <= 2^16, by the merge sort alone;
-// result in (k0, v0).  Uses no words of a sort's tmp.
-void sort_small(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n, hipStream_t s);
+// The same order by the merge sort alone, for keys in any order; result in
+// (k0, v0).  Uses no words of a sort's tmp.
+void sort_small(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n, const uint8_t* sysd, hipStream_t s);
+// Up to here (one merge round) bodies just handed over are sorted by it: 36 us
+// at 19,054 bodies in no order, where the look for keys in order finds none and
+// makes it 67; in order, 36 against 35.
+constexpr size_t kSortSmall = 32768;
 // device address of its control words: [0] 1 if the last call took the
 // near-sorted path, [3] the keys it radix sorted there
 uint32_t* sort_near_ctl(uint32_t* sort_tmp, size_t cap);

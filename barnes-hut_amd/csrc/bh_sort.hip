@@ -1347,7 +1347,7 @@ void sort_near_sorted(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, ui
                                                                                 cap);
 }
 
-void sort_small(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n, hipStream_t s)
+void sort_small(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n, const uint8_t* sysd, hipStream_t s)
 {
     if (n == 0) return;
     const uint32_t m = static_cast<uint32_t>(n);
@@ -1356,9 +1356,9 @@ void sort_small(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n
     uint64_t *ka = odd ? k1 : k0, *kb = odd ? k0 : k1;
     uint32_t *va = odd ? v1 : v0, *vb = odd ? v0 : v1;
     k_ns_tile_sort<<<static_cast<unsigned>((n + kMsTile - 1) / kMsTile), kMsNT, 0, s>>>(k0, v0, nullptr, nullptr, ka, va,
-                                                                                     nullptr, nullptr, n, m);
+                                                                                     sysd, nullptr, n, m);
     for (size_t L = kMsTile; L < n; L *= kMsWays) {
-        k_ns_merge_round<<<static_cast<unsigned>((n + kNT - 1) / kNT), kNT, 0, s>>>(ka, va, kb, vb, nullptr, nullptr, n,
+        k_ns_merge_round<<<static_cast<unsigned>((n + kNT - 1) / kNT), kNT, 0, s>>>(ka, va, kb, vb, sysd, nullptr, n,
                                                                                   static_cast<uint32_t>(L), m);
         std::swap(ka, kb);
         std::swap(va, vb);

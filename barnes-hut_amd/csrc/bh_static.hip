@@ -228,7 +228,7 @@ int bh_compute_accelerations_static(int64_t n, const bh_vec3* pos, const double*
     // (the radix sort's histogram and eight passes, mostly waits between tiles,
     // took 109 us at 3,000 bodies; with the merge sort's two launches and the
     // moments in one launch the evaluation went from 0.406 to 0.308 ms)
-    sort_small(L.tb.key, L.tb.perm, L.tb.key_alt, L.tb.perm_alt, N, s);
+    sort_small(L.tb.key, L.tb.perm, L.tb.key_alt, L.tb.perm_alt, N, nullptr, s);
     L.tb.deep_from = moments_cutoff(N);
     launch_permute(L.cur, L.alt, L.tb, N, s);
     launch_build_tree(L.alt, N, L.tb, true, s);
