@@ -103,6 +103,27 @@ __device__ inline uint32_t lower_bound_in(const uint64_t* __restrict__ u, uint32
     return lo + lower_bound_u64(u + lo, hi - lo, x);
 }
 
+// the same for two values at once: one memory trip a step for both
+__device__ inline void lower_bounds_in(const uint64_t* __restrict__ u, uint32_t lo, uint32_t hi, uint64_t x, uint64_t y,
+                                       uint32_t& at_x, uint32_t& at_y)
+{
+    uint32_t a = lo, b = lo;
+    for (uint32_t len = hi - lo; len > 1;) {
+        const uint32_t half = len >> 1;
+        const uint64_t ua = u[a + half - 1], ub = u[b + half - 1];
+        a += ua < x ? half : 0u;
+        b += ub < y ? half : 0u;
+        len -= half;
+    }
+    if (hi > lo) {
+        const uint64_t ua = u[a], ub = u[b];
+        a += ua < x ? 1u : 0u;
+        b += ub < y ? 1u : 0u;
+    }
+    at_x = a;
+    at_y = b;
+}
+
 // ------------------------------------------------------ kick/drift/box
 // System s owns blocks [box_block(s), box_block(s + 1)) of the grid (about
 // one per 1024 of its bodies), which stride over its bodies; each block
@@ -469,7 +490,13 @@ __device__ inline uint32_t leaf_moments_bounds(const Bodies& b, const TreeBuffer
             const uint64_t a = tb.ukey[j];
             const int d = split_depth(a, tb.ukey[j + 1]);
             tb.delta[j] = static_cast<uint8_t>(d);
-            const uint32_t lo = lower_bound_in(tb.ukey, L0, L1, prefix_at(a, d));
+            // the node's first leaf and the one after its last, for k_branch_init
+            // (in flag and suffix, which are free here)
+            const uint64_t p = prefix_at(a, d);
+            uint32_t lo, hi;
+            lower_bounds_in(tb.ukey, L0, L1, p, p + stride_at(d), lo, hi);
+            tb.flag[j] = lo;
+            tb.suffix[j] = hi;
             const uint64_t first_child = prefix_at(tb.ukey[lo], d + 1);
             const uint32_t rep = lower_bound_in(tb.ukey, L0, L1, first_child + stride_at(d + 1)) - 1;
             tb.rep[j] = rep;
@@ -500,14 +527,11 @@ __global__ __launch_bounds__(kNT) void k_branch_init(size_t n, TreeBuffers tb)
     const bool is_rep = (rep == j);
     tb.rep[j] = tb.bidx[rep];   // from here on: branching index of j's node
     if (!is_rep) return;
-    uint32_t L0, L1;
-    sys_leaves(tb, M, leaf_sys(tb, static_cast<uint32_t>(j)), L0, L1);
     const uint32_t bi = tb.bidx[j];
     const int d = tb.delta[j];
-    const uint64_t p = prefix_at(tb.ukey[j], d);
     tb.bdepth[bi] = static_cast<uint8_t>(d);
-    tb.blo[bi] = lower_bound_in(tb.ukey, L0, L1, p);
-    tb.bhi[bi] = lower_bound_in(tb.ukey, L0, L1, p + stride_at(d)) - 1;
+    tb.blo[bi] = tb.flag[j];
+    tb.bhi[bi] = tb.suffix[j] - 1;
     int32_t* c = tb.child + 8 * static_cast<size_t>(bi);
 #pragma unroll
     for (int k = 0; k < 8; ++k) c[k] = -1;
