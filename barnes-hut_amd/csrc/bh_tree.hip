@@ -498,7 +498,9 @@ __device__ inline uint32_t leaf_moments_bounds(const Bodies& b, const TreeBuffer
             tb.flag[j] = lo;
             tb.suffix[j] = hi;
             const uint64_t first_child = prefix_at(tb.ukey[lo], d + 1);
-            const uint32_t rep = lower_bound_in(tb.ukey, L0, L1, first_child + stride_at(d + 1)) - 1;
+            // (the first child ends at j or before)
+            const uint32_t rep =
+                lower_bound_in(tb.ukey, lo, static_cast<uint32_t>(j) + 1u, first_child + stride_at(d + 1)) - 1;
             tb.rep[j] = rep;
             isrep = (rep == j) ? 1u : 0u;
         }
