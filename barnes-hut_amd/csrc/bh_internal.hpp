@@ -43,14 +43,14 @@ static_assert(sizeof(WalkNode) == 48, "WalkNode is 48 bytes");
 
 constexpr uint32_t kMetaDepthMask = 31u;      // test (bottom) depth
 constexpr uint32_t kMetaTopShift = 5;         // chain top depth (5 bits)
-constexpr uint32_t kMetaLeaf = 1u << 10;      // distinct-key leaf (depth 21)
+constexpr uint32_t kMetaLeaf = 1u << 31;      // distinct-key leaf (depth 21); the sign, which one compare tests
 constexpr uint32_t kMetaChain = 1u << 11;     // leaf chain starts above depth 21
 // Up to kWaveMax bodies the plain walk may visit a node's children in two
 // chains, from the first child and from the middle one: kMetaMore is set on a
 // node whose chain goes on with the sibling at `skip`, and the middle child's
-// walk index stands above kMetaMidShift.
+// walk index stands in the 16 bits from kMetaMidShift.
 constexpr uint32_t kMetaMore = 1u << 12;
-constexpr uint32_t kMetaMidShift = 16;
+constexpr uint32_t kMetaMidShift = 15;
 constexpr size_t kWaveMax = 20480;            // (at most 2 n - 1 walk indices: 16 bits)
 
 constexpr int kMaxHeavy = 16;     // bodies per system summed directly in FP64 by the mixed forms
@@ -186,14 +186,14 @@ __device__ inline uint32_t scan_block_excl(uint32_t v, const uint32_t* tsum, siz
     return off + inc - v;
 }
 
-// 1.0 / sqrt(x) for x in [2^-767, 2^1000], bit for bit: the instruction
-// sequence the compiler emits for the IEEE FP64 square root (reciprocal
-// square-root estimate refined by Goldschmidt steps) followed by the one for
-// the IEEE division 1 / s (reciprocal estimate, two Newton steps, remainder
-// correction), without their range handling.  In this range the square root
-// needs no exponent scaling and is finite and nonzero, and 1 / s with
-// s in [2^-500, 2^500] needs no scaling and no fix-up, so the range handling
-// leaves every value unchanged there and dropping it saves 12 instructions.
+// 1.0 / sqrt(x), bit for bit, for the x that inv_sqrt_takes: the hardware's
+// reciprocal square root estimate refined to sqrt(x), correctly rounded, by
+// Goldschmidt steps (as the IEEE square root is computed), then its reciprocal.
+// The steps also leave h = 1 / (2 sqrt(x)) to 2^-45; one Newton step from 2 h is
+// within an ulp of 1 / g, and from there the remainder step rounds correctly
+// (Markstein) unless g's significand is all ones, which only an x with a low
+// word of at least 0xfffffffe gives.  (With the hardware's reciprocal estimate
+// and two Newton steps instead: 24 clocks a call more.)
 __device__ inline double inv_sqrt_in_range(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
@@ -206,10 +206,8 @@ __device__ inline double inv_sqrt_in_range(double x)
     g = __builtin_fma(d, h, g);
     d = __builtin_fma(-g, g, x);
     g = __builtin_fma(d, h, g);   // sqrt(x), correctly rounded
-    double q = __builtin_amdgcn_rcp(g);
+    double q = h + h;
     double e = __builtin_fma(-g, q, 1.0);
-    q = __builtin_fma(q, e, q);
-    e = __builtin_fma(-g, q, 1.0);
     q = __builtin_fma(q, e, q);
     e = __builtin_fma(-g, q, 1.0);
     return __builtin_fma(e, q, q);   // 1 / sqrt(x), correctly rounded
@@ -241,11 +239,13 @@ __device__ inline void warm_l2(const void* base, size_t bytes)
     }
 }
 
-// Whether inv_sqrt_in_range takes x, from its exponent alone (one subtraction
-// and one compare): x in [2^-767, 2^1000)
+// Whether inv_sqrt_in_range takes x: x in [2^-767, 2^1000), where the square
+// root needs no scaling and is finite and nonzero, and 1 / sqrt(x) needs none
+// either; and not one of the two significands whose root's is all ones.
 __device__ inline bool inv_sqrt_takes(double x)
 {
-    return static_cast<uint32_t>(__double2hiint(x)) - 0x10000000u < 0x7e700000u - 0x10000000u;
+    const uint32_t hi = static_cast<uint32_t>(__double2hiint(x)), lo = static_cast<uint32_t>(__double2loint(x));
+    return (hi - 0x10000000u < 0x7e700000u - 0x10000000u) & (lo < 0xfffffffeu);
 }
 
 // Compensated sum: c gathers the rounding error of every addition, exactly

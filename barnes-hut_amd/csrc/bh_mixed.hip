@@ -956,9 +956,8 @@ __device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, 
                         const double dx = lane_f64(hpx, k) - x, dy = lane_f64(hpy, k) - y, dz = lane_f64(hpz, k) - z;
                         const double r2 = dx * dx + dy * dy + dz * dz + soft2;
                         const bool pair = j != i && r2 > 0.0;
-                        const bool in_range = (r2 >= 0x1p-767) & (r2 <= 0x1p+1000);
-                        const double invR = __all(in_range | !pair) ? inv_sqrt_in_range(pair ? r2 : 1.0)
-                                                                    : 1.0 / sqrt(pair ? r2 : 1.0);
+                        const double invR = __all(inv_sqrt_takes(r2) | !pair) ? inv_sqrt_in_range(pair ? r2 : 1.0)
+                                                                              : 1.0 / sqrt(pair ? r2 : 1.0);
                         const double s = grav * lane_f64(hpm, k) * (invR * invR * invR);
                         if (pair) {
                             sx += s * dx;

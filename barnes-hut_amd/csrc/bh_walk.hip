@@ -104,12 +104,11 @@ __device__ inline Decision decide(const WalkNode& nd, double px, double py, doub
     return d;
 }
 
-// G m / r^3.  inv_sqrt_in_range gives the bits of 1.0 / sqrt(r2) in its
-// range; a wave with a lane outside it takes the library path.
+// G m / r^3.  inv_sqrt_in_range gives the bits of 1.0 / sqrt(r2) where it takes
+// r2; a wave with a lane whose r2 it does not takes the library path.
 __device__ inline double pull(double r2, double m, double G)
 {
-    const bool in_range = (r2 >= 0x1p-767) & (r2 <= 0x1p+1000);
-    const double invR = __all(in_range) ? inv_sqrt_in_range(r2) : 1.0 / sqrt(r2);
+    const double invR = __ballot(!inv_sqrt_takes(r2)) == 0ull ? inv_sqrt_in_range(r2) : 1.0 / sqrt(r2);
     const double invR3 = invR * invR * invR;
     return G * m * invR3;
 }
@@ -299,7 +298,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_walk_wave(Bodies b, size_t n, u
         if (take) atomicOr(bits + (k >> 6), 1ull << (k & 63u));
         if (take & (at < kFound)) l.list[at] = static_cast<uint16_t>(k);
         total += static_cast<uint32_t>(__popcll(mt));
-        const uint32_t mid = nd.meta >> kMetaMidShift;
+        const uint32_t mid = nd.meta >> kMetaMidShift & 0xffffu;
         const bool more = act & ((nd.meta & kMetaMore) != 0u) & (nd.skip > k) & (nd.skip < T);
         const bool open = act & d.open & (k + 1 < T);
         const bool open2 = open & (mid > k) & (mid < T);
