@@ -18,9 +18,10 @@
 // it chooses next is fetched right away, so the fetch overlaps the FP64
 // square root, division and accumulation of an accepted node instead of
 // following them.  Node records are per-lane vector loads; Morton-consecutive
-// lanes walk nearly the same nodes, so most of them are cache hits.  The
-// blocks are dealt out so that each XCD walks one contiguous eighth of the
-// Morton order (its L2 then holds the near field of that eighth).
+// lanes walk nearly the same nodes, at nearly the same time where their lead is
+// limited (walk_lead), so most of them are cache hits.  The blocks are dealt
+// out so that each XCD walks one contiguous eighth of the Morton order (its L2
+// then holds the near field of that eighth).
 // Roofline: FP64 vector (78.6 TF/s); work per body 9 flops per tested node
 // + 12 per accepted node.
 #include <hip/hip_runtime.h>
@@ -113,12 +114,35 @@ __device__ inline double pull(double r2, double m, double G)
     return G * m * invR3;
 }
 
-template <bool kCount>
+// the smallest v of the wavefront (all lanes active), in a scalar
+template <int kCtrl, int kRows>
+__device__ inline uint32_t dpp_min(uint32_t v)
+{
+    return min(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), kCtrl, kRows,
+                                                                  0xf, false)));
+}
+
+__device__ inline uint32_t wave_min(uint32_t v)
+{
+    v = dpp_min<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+    v = dpp_min<0x112, 0xf>(v);
+    v = dpp_min<0x114, 0xf>(v);
+    v = dpp_min<0x118, 0xf>(v);
+    v = dpp_min<0x142, 0xa>(v);   // row_bcast 15, 31
+    v = dpp_min<0x143, 0xc>(v);
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+
+// Visits between two looks at where the last lane is (kLead; 4 and 16 measured
+// the same).
+constexpr int kVisits = 8;
+
+template <bool kCount, bool kLead>
 __global__ __launch_bounds__(kNT) void k_walk_plain(Bodies b, size_t n, uint32_t grid_blocks,
                                                     const WalkNode* __restrict__ walk,
                                                     const uint32_t* __restrict__ self_w,
                                                     const StepScalars* __restrict__ sc,
-                                                    const SysScalars* __restrict__ sy, WalkParams p,
+                                                    const SysScalars* __restrict__ sy, WalkParams p, uint32_t lead,
                                                     int64_t* __restrict__ cnt_accept, int64_t* __restrict__ cnt_open,
                                                     int64_t* __restrict__ cnt_test)
 {
@@ -127,16 +151,17 @@ __global__ __launch_bounds__(kNT) void k_walk_plain(Bodies b, size_t n, uint32_t
     // M + B <= 2n - 1 by construction; the clamp keeps a corrupted count in bounds
     const uint32_t T = min(sc->n_nodes, static_cast<uint32_t>(2 * n));
     if (T * sizeof(WalkNode) <= kWarmBytes) warm_l2(walk, T * sizeof(WalkNode));
-    if (i >= n) return;
-    const double px = b.px[i];
-    const double py = b.py[i];
-    const double pz = b.pz[i];
-    const uint32_t self = self_w[i];
+    // (a lane without a body has arrived; it takes part in the wavefront's minima)
+    const size_t ib = min(i, n - 1);
+    const double px = b.px[ib];
+    const double py = b.py[ib];
+    const double pz = b.pz[ib];
+    const uint32_t self = self_w[ib];
     double ax = 0.0, ay = 0.0, az = 0.0;
     int64_t na = 0, no = 0, nt = 0;
-    uint32_t cur = 0;
+    uint32_t cur = i < n ? 0u : T;
     WalkNode nd = load_node(walk, 0, T);
-    while (cur < T) {
+    const auto visit = [&]() {
         // the decision first
         const Decision d = decide(nd, px, py, pz, cur == self, p);
         // then the fetch of the next record, whose latency the FP64
@@ -169,7 +194,19 @@ __global__ __launch_bounds__(kNT) void k_walk_plain(Bodies b, size_t n, uint32_t
         }
         cur = next;
         nd = nn;
+    };
+    if constexpr (kLead) {
+        for (;;) {
+            const uint32_t last = wave_min(cur);
+            if (last >= T) break;
+            const uint32_t ahead = lead < T - last ? last + lead : T - 1;
+            for (int r = 0; r < kVisits; ++r)
+                if (cur <= ahead) visit();
+        }
+    } else {
+        while (cur < T) visit();
     }
+    if (i >= n) return;
     b.ax[i] = ax;
     b.ay[i] = ay;
     b.az[i] = az;
@@ -454,6 +491,26 @@ __global__ __launch_bounds__(64 * kWaves) void k_walk_wave(Bodies b, size_t n, u
 // 0.313 and 0.305 (1.05), 0.87 and 1.2 (0.5).
 bool by_wavefronts(size_t n, double theta2) { return n <= 16384 || (n <= kWaveMax && theta2 <= 1.44); }
 
+// How many walk indices a lane may be ahead of its wavefront's last one (0: no
+// limit).  The lanes of a wavefront drift apart, and then every lane's record
+// is a line of its own: 44 lines a visit at 300k bodies, one L1 lookup each for
+// each of the record's three loads, and at one lookup a clock these are what
+// bounds a full chip (vector instructions 37% busy).  Lanes that wait for the
+// last one make the visits share lines; their steps are more (simulated at
+// 300k, theta 1.05, limit 5,000: 23 lines a visit, 19% more steps), which a chip
+// with few wavefronts pays for.  Walks in ms, no limit and 30,000 / 10,000 /
+// 4,000 / 1,000: belt 50,000 theta 1.05 0.48, 0.52 / 0.56 / 0.68 / 0.83; 130,000
+// 0.94, 0.89 / 1.03 / 1.12 / 1.25; 300k 2.12, 2.06 / 2.04 / 2.08 / 2.20, theta
+// 0.5 11.6, 11.0 / 10.7 / 10.4 / 10.1; Trojan 300k theta 0.7 5.4, 5.1 / 4.9 /
+// 4.6 / 4.3; Kuiper 300k theta 0.7 1.35, 1.24 / 1.20 / 1.20 / 1.28; Trojan 1M
+// 7.8, 6.7 / 6.1 / 5.9 / 5.8.
+uint32_t walk_lead(size_t n, double theta2)
+{
+    if (n < 100000) return 0u;
+    if (n < 160000) return 30000u;
+    return theta2 < 0.64 ? 4000u : 10000u;
+}
+
 }  // namespace
 
 void launch_walk_plain(const Bodies& b, size_t n, const TreeBuffers& tb, const WalkParams& p,
@@ -464,16 +521,20 @@ void launch_walk_plain(const Bodies& b, size_t n, const TreeBuffers& tb, const W
     // the XCD-contiguous mapping covers blocks [0, 8 * ceil(g / 8)); blocks
     // mapped past g return at once
     const uint32_t grid = ((g + kXcds - 1) / kXcds) * kXcds;
+    const uint32_t lead = walk_lead(n, p.theta2);
     if (cnt_accept && cnt_open && cnt_test)
-        k_walk_plain<true><<<grid, kNT, 0, s>>>(b, n, g, tb.walk, tb.self_w, tb.sc, tb.sys, p, cnt_accept, cnt_open,
+        k_walk_plain<true, false><<<grid, kNT, 0, s>>>(b, n, g, tb.walk, tb.self_w, tb.sc, tb.sys, p, 0u, cnt_accept, cnt_open,
                                                 cnt_test);
     else if (by_wavefronts(n, p.theta2)) {
         const uint32_t words = static_cast<uint32_t>((2 * n + 63) / 64);
         const uint32_t gw = static_cast<uint32_t>((n + kWaves - 1) / kWaves);
         k_walk_wave<<<(gw + kXcds - 1) / kXcds * kXcds, 64 * kWaves, kWaves * words * sizeof(uint64_t), s>>>(
             b, n, gw, tb.walk, tb.self_w, tb.sc, p, words);
-    } else
-        k_walk_plain<false><<<grid, kNT, 0, s>>>(b, n, g, tb.walk, tb.self_w, tb.sc, tb.sys, p, nullptr, nullptr,
+    } else if (lead != 0u)
+        k_walk_plain<false, true><<<grid, kNT, 0, s>>>(b, n, g, tb.walk, tb.self_w, tb.sc, tb.sys, p, lead, nullptr, nullptr,
+                                                 nullptr);
+    else
+        k_walk_plain<false, false><<<grid, kNT, 0, s>>>(b, n, g, tb.walk, tb.self_w, tb.sc, tb.sys, p, 0u, nullptr, nullptr,
                                                  nullptr);
 }
 
