@@ -66,9 +66,9 @@ constexpr int kStackCap = 1024;
 // (pure depth first) grows the stack by at most 7 per level: P ranges may be
 // popped while 7 P more fit below the room of one descent.  (Popping 64 or,
 // near the limit, one at a time: a group of four far-apart planets, which opens
-// 33,000 nodes of a 300k belt, walked 5.7 nodes a round, 3.9 ms of a walk of
-// 3.8; with this rule it takes 0.4 ms and the walk 0.52.  A 64-system belt
-// ensemble of 3.8M bodies 18.7 -> 5.6 ms.  Groups that do not fill their stack
+// 33,000 nodes of a 300k belt, walked 5.7 nodes a round; the belt's walk 3.78 ->
+// 0.52 ms with this rule.  A 64-system belt ensemble of 3.8M bodies 18.7 ->
+// 5.6 ms.  Groups that do not fill their stack
 // are walked as before.)
 // narrow: 64 or one at a time.  The work of a group, the target of the learned
 // form's training, depends on where the list is flushed and so on the order of
