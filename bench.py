@@ -441,8 +441,9 @@ def main():
     walk_ms = head["phase_ms"]["walk_kick"]
     achieved = work["flops_per_launch"] / (walk_ms * 1e-3) / 1e12
     if form == "plain":
-        kname, kern, peak, bound = "k_walk_plain", "k_walk_plain (FP64 walk + fused half kick)", \
-            FP64_PEAK_TFLOPS, "valu_fp64"
+        # small systems take a wavefront per body (the library's rule on n and theta)
+        kname = "k_walk_wave" if n <= 16384 or (n <= 20480 and theta <= 1.2) else "k_walk_plain"
+        kern, peak, bound = f"{kname} (FP64 walk + fused half kick)", FP64_PEAK_TFLOPS, "valu_fp64"
         peak_note = "FP64 vector peak"
     else:
         kname, kern, peak, bound = "k_walk_mixed", \
