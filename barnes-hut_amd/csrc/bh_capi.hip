@@ -180,7 +180,7 @@ int reserve(bh_ctx* c, size_t n)
     A(t.ukey, N); A(t.leaf_first, N + 1); A(t.delta, N); A(t.rep, N); A(t.is_rep, N);
     A(t.bidx, N); A(t.cnt_hi, N); A(t.suffix, N + 1);
     A(t.bdepth, N); A(t.blo, N); A(t.bhi, N); A(t.child, 8 * N);
-    A(t.parent, 2 * N); A(t.windex, 2 * N); A(t.raw, 8 * N); A(t.lraw, 8 * N); A(t.lbox, 12 * N); A(t.lsec, 2 * N); A(t.walk, 2 * N);
+    A(t.parent, 2 * N); A(t.windex, 2 * N); A(t.raw, 8 * N); A(t.lraw, 8 * N); A(t.lbox, bh::staging_doubles(N)); A(t.lsec, 2 * N); A(t.walk, 2 * N);
     A(t.gflag, N); A(t.gtile, bh::tile_sum_words(N)); A(c->bsys_w, N); A(t.sys, bh::kMaxSystems); A(t.deep, N);
     A(t.pyr, bh::kPyrDoubles * bh::pyr_entries(N));
     t.pyr_cap = static_cast<uint32_t>(N);
@@ -196,7 +196,7 @@ int reserve(bh_ctx* c, size_t n)
     HIP_TRY(c, hipMemsetAsync(t.sort_tmp, 0, bh::sort_tmp_words(N) * sizeof(uint32_t), c->stream));
     A(t.sc, 1);
     A(c->partials, 6 * bh::kBoxBlocks);
-    A(c->runs, 2 * (N / bh::kHeavyRun + bh::kMaxSystems + 1) + bh::kMaxSystems + 1);
+    A(c->runs, 2 * bh::max_heavy_runs(N) + bh::kMaxSystems + 1);
 #undef A
     HIP_TRY(c, hipMemsetAsync(t.sc, 0, sizeof(StepScalars), c->stream));
     c->cap = N;
@@ -420,8 +420,8 @@ int check_device_errors(bh_ctx* c)
     return BH_OK;
 }
 
-// Staging area of the host transfers: the light boxes (96 bytes a body, rebuilt
-// by every mixed evaluation before it reads them).
+// Staging area of the host transfers and of the heavy set: the light boxes
+// (staging_doubles(cap), rebuilt by every mixed evaluation before it reads them).
 unsigned char* staging(const bh_ctx* c) { return reinterpret_cast<unsigned char*>(c->tb.lbox); }
 
 constexpr size_t kChunk = size_t{4} << 20;
@@ -598,6 +598,7 @@ int configure_systems(bh_ctx* c, const std::vector<int64_t>& counts)
     const uint32_t n_runs = static_cast<uint32_t>(runs.size() / 2);
     sys_run[S] = n_runs;
     runs.insert(runs.end(), sys_run.begin(), sys_run.end());
+    if (n_runs > bh::max_heavy_runs(c->cap)) return fail(c, BH_ERR_STATE, "%u runs of bodies > %zu", n_runs, bh::max_heavy_runs(c->cap));
     if (item > c->heavy_item_cap) return fail(c, BH_ERR_STATE, "heavy work items %u > %zu", item, c->heavy_item_cap);
     // k_kick_drift_box: blocks in proportion to the bodies (one per 1024, at
     // least one per system), scaled down to at most kBoxGrid: k_keys reads

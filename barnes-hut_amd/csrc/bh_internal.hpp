@@ -22,6 +22,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "bh_limits.hpp"
+
 namespace bh {
 
 constexpr int kMaxDepth = 21;
@@ -53,8 +55,6 @@ constexpr uint32_t kMetaMore = 1u << 12;
 constexpr uint32_t kMetaMidShift = 15;
 constexpr size_t kWaveMax = 20480;            // (at most 2 n - 1 walk indices: 16 bits)
 
-constexpr int kMaxHeavy = 16;     // bodies per system summed directly in FP64 by the mixed forms
-constexpr int kMaxSystems = 256;  // systems per context (the sort's system pass uses 8-bit digits)
 constexpr uint8_t kNoSplit = 0xff;   // delta of a boundary between two systems
 
 // Per-system scalars.  Fixed by the system layout: body range, heavy count
@@ -331,7 +331,7 @@ struct TreeBuffers {
     uint32_t* windex;     // walk index
     double* raw;          // 4 per node: mass, sum m*x, sum m*y, sum m*z
     double* lraw;         // the same over light bodies only (mixed forms), or null
-    double* lbox;         // 6 per node: bounding box of the light bodies (min xyz, max xyz)
+    double* lbox;         // 6 per node: bounding box of the light bodies (min xyz, max xyz); staging_doubles(N)
     double* lsec;         // per node: sum of m |x|^2 over the light bodies (mixed forms)
     uint32_t* gflag;      // walk-group start flags (mixed forms), cleared per step
     uint32_t* gtile;      // flags set per 256-body tile (the group scan's tile sums), cleared per step
@@ -580,8 +580,6 @@ void launch_new_bodies(const Bodies& b, size_t n, bool own_ids, hipStream_t s);
 // n_heavy is given): runs of kHeavyRun rows of one system, run r = rows
 // run_sys[2 r + 1] * kHeavyRun .. of system run_sys[2 r], system s's runs
 // sys_run[s] .. sys_run[s + 1] - 1.  scratch: heavy_scratch_bytes(n_runs).
-constexpr uint32_t kHeavyRun = 4096;
-size_t heavy_scratch_bytes(uint32_t n_runs);
 void launch_heavy_set(const Bodies& b, const TreeBuffers& tb, const uint32_t* run_sys, uint32_t n_runs,
                       const uint32_t* sys_run, uint8_t* bsys, void* scratch, hipStream_t s);
 

@@ -68,10 +68,6 @@ __global__ __launch_bounds__(kNT) void k_new_bodies(Bodies b, size_t n, int own_
 
 // ------------------------------------------------------------- heavy set
 // Bodies in order of descending mass, then of ascending row.
-struct Pick {
-    double m;
-    uint32_t i;   // row; kNoRow: none
-};
 constexpr uint32_t kNoRow = 0xffffffffu;
 
 __device__ inline bool heavier(const Pick& a, const Pick& b)
@@ -216,8 +212,6 @@ __global__ __launch_bounds__(kNT) void k_row_systems(Bodies b, TreeBuffers tb, c
 inline unsigned nblk(size_t n) { return static_cast<unsigned>((n + kNT - 1) / kNT); }
 
 }  // namespace
-
-size_t heavy_scratch_bytes(uint32_t n_runs) { return sizeof(Pick) * kMaxHeavy * static_cast<size_t>(n_runs); }
 
 void launch_split3(const double* v, size_t n, double* x, double* y, double* z, hipStream_t s)
 {
