@@ -67,15 +67,6 @@ __global__ __launch_bounds__(kNT) void k_new_bodies(Bodies b, size_t n, int own_
 }
 
 // ------------------------------------------------------------- heavy set
-// Bodies in order of descending mass, then of ascending row.
-constexpr uint32_t kNoRow = 0xffffffffu;
-
-__device__ inline bool heavier(const Pick& a, const Pick& b)
-{
-    if (a.i == kNoRow || b.i == kNoRow) return b.i == kNoRow && a.i != kNoRow;
-    return a.m > b.m || (!(b.m > a.m) && a.i < b.i);
-}
-
 // The heaviest of the block's picks, in every thread.
 __device__ inline Pick block_heaviest(Pick p)
 {
@@ -165,7 +156,7 @@ __global__ __launch_bounds__(kNT) void k_heavy_candidates(const double* __restri
         kMaxHeavy,
         [&](auto f) {
 #pragma unroll 8
-            for (uint32_t i = lo + threadIdx.x; i < hi; i += kNT) f(Pick{m[i], i});
+            for (uint32_t i = lo + threadIdx.x; i < hi; i += kNT) f(pick(m[i], i));
         },
         cand + static_cast<size_t>(blockIdx.x) * kMaxHeavy);
 }

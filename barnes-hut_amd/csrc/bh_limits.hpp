@@ -4,6 +4,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "bh_pick.hpp"
+
 namespace bh {
 
 constexpr int kMaxHeavy = 16;     // bodies per system summed directly in FP64 by the mixed forms
@@ -11,10 +13,6 @@ constexpr int kMaxSystems = 256;  // systems per context (the sort's system pass
 
 // The heavy set is chosen over runs of at most kHeavyRun rows of one system,
 // each of which leaves kMaxHeavy candidates (Pick) in a scratch area.
-struct Pick {
-    double m;
-    uint32_t i;   // row; kNoRow: none
-};
 constexpr uint32_t kHeavyRun = 4096;
 
 // a system of k bodies has ceil(k / kHeavyRun) <= k / kHeavyRun + 1 runs
