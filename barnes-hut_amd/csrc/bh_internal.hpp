@@ -99,7 +99,7 @@ struct StepScalars {
     alignas(128) uint64_t work_sum[8][16];
     uint64_t work_prev;
     uint32_t groups_prev;   // groups of that walk
-    uint32_t n_big;    // key order: groups shared by a block's wavefronts (listed in MixedBuffers::chunk)
+    uint32_t n_big;    // key order: groups over the sharing limit (the first kMaxShared are listed in MixedBuffers::chunk)
     uint32_t n_coop;   // cost order: the same, the first of the order
 };
 

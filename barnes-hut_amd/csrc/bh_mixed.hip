@@ -351,7 +351,10 @@ __device__ inline void group_first(size_t i, size_t n, uint32_t gid, const Bodie
         bool big = tb.sc->work_prev != 0u && b.pcost[i] > share_limit(tb.sc, mb.walk_waves);
         if (big) {
             const uint32_t k = atomicAdd(&tb.sc->n_big, 1u);
-            big = k < kMaxShared;   // (at most waves^2 / (kShare x groups) or 8 x waves exceed the limit)
+            // (at most waves^2 / (kShare x groups) or 8 x waves groups of the previous
+            // walk exceed the limit; smaller groups since, each with the work of the
+            // group its bodies were in, can be more: the rest are not shared)
+            big = k < kMaxShared;
             if (big) mb.chunk[k] = gid;
         }
         mb.gbig[gid] = big ? 1u : 0u;
@@ -1284,7 +1287,7 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3))) void k
             C = G <= 2u * nblk ? G : 0u;
             listed = use_order;
         } else {
-            C = min(use_order ? sc->n_coop : sc->n_big, G);
+            C = min(use_order ? sc->n_coop : min(sc->n_big, kMaxShared), G);
             listed = true;
         }
     }
