@@ -1247,7 +1247,7 @@ __device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, 
                 ae->mb.g_work[g] = work;
                 ae->mb.g_t0[g] = t_start;
                 ae->mb.g_t1[g] = wall_clock64();
-                ae->mb.g_worker[g] = blockIdx.x * kWaves + static_cast<uint32_t>(w);
+                ae->mb.g_worker[g] = blockIdx.x * kWaves + (threadIdx.x >> 6);   // (w is 0 for a lone wavefront)
             }
             group_sync<NW>();   // the next group writes the exchanged sums and the list
     return work;

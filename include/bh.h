@@ -265,7 +265,8 @@ int bh_get_groups(bh_ctx *ctx, int64_t *n_groups, int64_t capacity, uint32_t *fi
 
 /* Timeline of the last mixed walk: for each group the device wall clock
  * (100 MHz ticks) when a worker wave took it and when it finished, and the
- * worker's index.  Arrays sized by the group count of bh_get_groups. */
+ * worker's index (block x 4 + wave; a group shared by a block's four waves has
+ * the first one's).  Arrays sized by the group count of bh_get_groups. */
 int bh_get_group_timeline(bh_ctx *ctx, int64_t capacity, uint64_t *t_start, uint64_t *t_end, uint32_t *worker);
 
 /* Walk work of each group of the last mixed walk: its list cost + visited
