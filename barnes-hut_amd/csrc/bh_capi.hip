@@ -153,7 +153,10 @@ int dalloc(bh_ctx* c, T** p, size_t count)
     void* q = nullptr;
     if (count == 0) count = 1;
     hipError_t e = hipMalloc(&q, count * sizeof(T));
-    if (e != hipSuccess) return fail(c, BH_ERR_NOMEM, "hipMalloc(%zu bytes): %s", count * sizeof(T), hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here; the next call's launches are not to blame for it
+        return fail(c, BH_ERR_NOMEM, "hipMalloc(%zu bytes): %s", count * sizeof(T), hipGetErrorString(e));
+    }
     c->allocs.push_back(q);
     *p = static_cast<T*>(q);
     return BH_OK;
@@ -203,6 +206,14 @@ int reserve(bh_ctx* c, size_t n)
     return BH_OK;
 }
 
+// A bh_set_bodies that found no room has freed the buffers of the bodies before
+// (whose count c->n still is): nothing may be launched on them.
+int check_held(bh_ctx* c)
+{
+    if (c->n > 0 && c->cap == 0) return fail(c, BH_ERR_STATE, "no bodies: the last bh_set_bodies failed");
+    return BH_OK;
+}
+
 // One force evaluation with optional leading kick + drift and trailing kick.
 constexpr int kRing = 512;
 constexpr float kHistoryDrop = 0.2f;   // share of training samples drawn without their history features
@@ -214,6 +225,7 @@ int run_force(bh_ctx* c, int form, double theta, double G, double soft2, bool ki
     if (form != BH_FORM_PLAIN && form != BH_FORM_MIXED && form != BH_FORM_LEARNED)
         return fail(c, BH_ERR_ARG, "unknown form %d", form);
     if (c->n == 0) return BH_OK;
+    if (const int rc = check_held(c)) return rc;
     const bool mixed = form != BH_FORM_PLAIN;
     if (mixed && c->n >= (size_t{1} << 26))
         return fail(c, BH_ERR_ARG, "the mixed forms take at most 2^26 - 1 bodies");
@@ -874,6 +886,7 @@ int bh_get_bodies(bh_ctx* c, bh_vec3* pos, bh_vec3* vel, double* mass, uint64_t*
     if (check_ctx(c)) return BH_ERR_ARG;
     c->err.clear();
     if (c->n == 0) return BH_OK;
+    if (const int rc = check_held(c)) return rc;
     return download(c, pos, vel, mass, ids, acc);
 }
 
@@ -893,6 +906,7 @@ int bh_step(bh_ctx* c, int64_t nsteps, double dt)
     if (check_ctx(c)) return BH_ERR_ARG;
     c->err.clear();
     if (nsteps < 0) return fail(c, BH_ERR_ARG, "negative step count");
+    if (const int rc = check_held(c)) return rc;
     if (c->ring.empty()) {
         c->ring.resize(5 * kRing, nullptr);
         for (auto& e : c->ring) HIP_TRY(c, hipEventCreate(&e));
@@ -1166,6 +1180,7 @@ int bh_set_systems(bh_ctx* c, int64_t n_systems, const int64_t* counts)
     if (n_systems < 1 || n_systems > bh::kMaxSystems || !counts)
         return fail(c, BH_ERR_ARG, "1..%d systems", bh::kMaxSystems);
     if (c->n == 0) return fail(c, BH_ERR_STATE, "no bodies (bh_set_bodies first)");
+    if (const int rc = check_held(c)) return rc;
     // a force evaluation sorts the bodies over the whole index range while
     // they form one system, so fixed ranges would no longer hold the systems
     // the caller concatenated
@@ -1443,6 +1458,7 @@ int bh_direct_sum(bh_ctx* c, int64_t m, const int64_t* idx, double G, double sof
     c->err.clear();
     if (m < 0 || (m > 0 && (!idx || !acc_out))) return fail(c, BH_ERR_ARG, "bad sample arguments");
     if (m == 0) return BH_OK;
+    if (const int rc = check_held(c)) return rc;
     for (int64_t k = 0; k < m; ++k)
         if (idx[k] < 0 || idx[k] >= static_cast<int64_t>(c->n))
             return fail(c, BH_ERR_ARG, "sample index %lld out of range", (long long)idx[k]);
