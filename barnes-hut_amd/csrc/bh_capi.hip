@@ -496,7 +496,9 @@ struct ChunkPool {
             }
         }
         void* p = nullptr;
-        return hipHostMalloc(&p, 2 * kChunk, hipHostMallocPortable) == hipSuccess ? static_cast<unsigned char*>(p) : nullptr;
+        if (hipHostMalloc(&p, 2 * kChunk, hipHostMallocPortable) == hipSuccess) return static_cast<unsigned char*>(p);
+        (void)hipGetLastError();   // the download does without
+        return nullptr;
     }
     void give(unsigned char* p)
     {
@@ -541,9 +543,10 @@ int download_chunks(bh_ctx* c, const Part (&part)[5], size_t total, unsigned cha
 }
 
 // The parts of the bodies the caller wants (others null), packed on the
-// device.  Up to one chunk they come over one by one; more takes the pinned
-// chunks (300,149 bodies 5.9 -> 1.8 ms, 4,194,304 102 -> 18 ms, against
-// component arrays copied to pageable vectors and joined on the host).
+// device.  Up to one chunk, and where no pinned memory is to be had, they come
+// over one by one; more takes the pinned chunks (300,149 bodies 5.9 -> 1.8 ms,
+// 4,194,304 102 -> 18 ms, against component arrays copied to pageable vectors
+// and joined on the host).
 int download(bh_ctx* c, bh_vec3* pos, bh_vec3* vel, double* mass, uint64_t* ids, bh_vec3* acc)
 {
     Part part[5] = {{reinterpret_cast<unsigned char*>(pos), c->n * 24, 0}, {reinterpret_cast<unsigned char*>(vel), c->n * 24, 0},
@@ -564,15 +567,14 @@ int download(bh_ctx* c, bh_vec3* pos, bh_vec3* vel, double* mass, uint64_t* ids,
                                      reinterpret_cast<uint64_t*>(dev[4])},
                     c->stream);
     HIP_TRY(c, hipGetLastError());
-    if (total <= kChunk) {
+    unsigned char* const pinned = total > kChunk ? g_chunks.take() : nullptr;
+    if (!pinned) {
         for (int k = 0; k < 5; ++k)
             if (part[k].bytes)
                 HIP_TRY(c, hipMemcpyAsync(part[k].host, dev[k], part[k].bytes, hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         return BH_OK;
     }
-    unsigned char* const pinned = g_chunks.take();
-    if (!pinned) return fail(c, BH_ERR_NOMEM, "hipHostMalloc(%zu bytes) failed", 2 * kChunk);
     const int rc = download_chunks(c, part, total, pinned);
     if (rc) (void)hipStreamSynchronize(c->stream);   // no transfer into the pair any more
     g_chunks.give(pinned);
