@@ -561,6 +561,7 @@ int download(bh_ctx* c, bh_vec3* pos, bh_vec3* vel, double* mass, uint64_t* ids,
         total += part[k].bytes;
     }
     if (total == 0) return BH_OK;
+    (void)hipGetLastError();   // an error left by the caller's own HIP calls is not this launch's
     bh::launch_pack(c->cur, c->n,
                     bh::PackedBodies{reinterpret_cast<double*>(dev[0]), reinterpret_cast<double*>(dev[1]),
                                      reinterpret_cast<double*>(dev[2]), reinterpret_cast<double*>(dev[3]),
@@ -633,6 +634,7 @@ int configure_systems(bh_ctx* c, const std::vector<int64_t>& counts)
         c->tb.box_blocks = first;
     }
     hipStream_t st = c->stream;
+    (void)hipGetLastError();   // an error left by the caller's own HIP calls is not these launches'
     HIP_TRY(c, hipMemcpyAsync(c->tb.sys, sys.data(), S * sizeof(bh::SysScalars), hipMemcpyHostToDevice, st));
     HIP_TRY(c, hipMemcpyAsync(c->runs, runs.data(), runs.size() * sizeof(uint32_t), hipMemcpyHostToDevice, st));
     TreeBuffers tb = c->tb;

@@ -40,3 +40,17 @@ def test_calls_after_an_upload_without_room(bh):
         again = run()
     for k in ("pos", "vel", "acc", "ids"):
         assert np.array_equal(again[k].view(np.uint64), want[k].view(np.uint64))
+
+
+def test_transfers_after_an_error_of_the_caller(bh):
+    """An error that the caller's own HIP calls left on the runtime's record does
+    not make an upload or a download fail."""
+    print("[gpu-case] error of the caller", file=sys.stderr, flush=True)
+    hip = C.CDLL("libamdhip64.so.7")
+    pos, vel, mass = bh.generate(bh.GEN_BELT, 5, 3000)
+    with bh.Engine(form=bh.FORM_MIXED) as e:
+        for call in (lambda: e.set_bodies(pos, vel, mass), lambda: e.set_systems([1000, 2000]), lambda: e.get_bodies()):
+            assert hip.hipSetDevice(9999) != 0
+            assert hip.hipPeekAtLastError() != 0
+            s = call()
+        assert np.array_equal(s["pos"], pos)
