@@ -63,7 +63,8 @@ struct bh_ctx {
     int sched = BH_SCHED_KEY_ORDER;   // schedule of the MIXED form
     int split = 0;                    // chunks per worker of the split schedule (0: heaviest first)
     bool sort_near = true;            // key sort: near-sorted front end (false: full radix sort)
-    int moment_cut = -1;              // deep cutoff of the tree moments (-1: chosen at graph capture)
+    int moment_cut = -1;              // deep cutoff of the tree moments (-1: plain_cutoff)
+    int deep_chosen = -1;             // the cutoff chosen at graph capture (-1: none since the bodies were set)
     bool model_ready = false;         // the LEARNED cost model is trained
     // cost model (allocated once per context, independent of N)
     ModelBuffers md{};
@@ -219,6 +220,14 @@ constexpr int kRing = 512;
 constexpr float kHistoryDrop = 0.2f;   // share of training samples drawn without their history features
 constexpr int kHeavy = bh::kMaxHeavy;
 
+// deep cutoff of the plain form's tree moments
+int plain_cutoff(const bh_ctx* c)
+{
+    if (c->moment_cut >= 0) return c->moment_cut;
+    if (c->n <= bh::kDeepWhole) return 0;
+    return c->deep_chosen >= 0 ? c->deep_chosen : bh::moments_cutoff(c->n);
+}
+
 int run_force(bh_ctx* c, int form, double theta, double G, double soft2, bool kick_before, bool drift,
               double dt, bool kick_after, const hipEvent_t* ev)
 {
@@ -260,9 +269,7 @@ int run_force(bh_ctx* c, int form, double theta, double G, double soft2, bool ki
         tb.lraw = nullptr;
         tb.gflag = nullptr;
         tb.gtile = nullptr;
-        // an eager step's launches, and a small tree's in a graph too
-        if (c->moment_cut < 0 && (c->n <= bh::kDeepWhole || tb.deep_from == bh::kMaxDepth))
-            tb.deep_from = bh::moments_cutoff(c->n);
+        tb.deep_from = plain_cutoff(c);
     } else {
         tb.deep_from = bh::kMaxDepth;   // the light-moment pyramid needs no list of deep nodes
     }
@@ -681,12 +688,8 @@ std::vector<double> graph_key(const bh_ctx* c, double dt)
 
 int choose_deep_from(bh_ctx* c)
 {
-    if (c->moment_cut >= 0) {
-        c->tb.deep_from = c->moment_cut;
-        return BH_OK;
-    }
-    // run_force sums a small tree in one workgroup; the mixed forms sum no depths
-    if (c->n <= bh::kDeepWhole || c->cfg.form != BH_FORM_PLAIN) return BH_OK;
+    // fixed, or the whole tree; the mixed forms sum no depths
+    if (c->moment_cut >= 0 || c->n <= bh::kDeepWhole || c->cfg.form != BH_FORM_PLAIN) return BH_OK;
     StepScalars sc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     HIP_TRY(c, hipMemcpy(&sc, c->tb.sc, sizeof sc, hipMemcpyDeviceToHost));
@@ -697,7 +700,7 @@ int choose_deep_from(bh_ctx* c)
     for (const uint8_t d : depth) ++hist[d < bh::kMaxDepth ? d : bh::kMaxDepth];
     int from = bh::kMaxDepth;
     while (from > 1 && hist[from - 1] == 0) --from;
-    c->tb.deep_from = from;
+    c->deep_chosen = from;
     return BH_OK;
 }
 
@@ -861,6 +864,7 @@ int bh_set_bodies(bh_ctx* c, int64_t n, const bh_vec3* pos, const bh_vec3* vel, 
     c->have_groups = false;
     c->prev_counts = false;
     c->evaluated = false;
+    c->deep_chosen = -1;
     if (n == 0) {
         c->n_sys = 1;
         c->tb.n_sys = 1;
@@ -1380,7 +1384,6 @@ int bh_set_moment_cutoff(bh_ctx* c, int cutoff)
     if (cutoff < -1 || cutoff > bh::kMaxDepth) return fail(c, BH_ERR_ARG, "moment cutoff %d outside [-1, %d]", cutoff,
                                                           bh::kMaxDepth);
     c->moment_cut = cutoff;
-    if (cutoff >= 0) c->tb.deep_from = cutoff;
     drop_graphs(c);
     return BH_OK;
 }

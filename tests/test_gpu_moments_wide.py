@@ -1,0 +1,59 @@
+"""GPU test of the tree moments of wide systems: one body far outside a belt puts
+nearly every branching node deep in the tree, where a single workgroup must not
+be left to sum all of a large system.  The automatic cutoff may not be slower
+than one launch per depth, and gives the same bits; where it once was, it took
+two to three times as long, so the limit of 1.3 leaves room for timing noise."""
+import sys
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+HOUR = 1.0 / 24.0
+ROOM = 1.3
+
+
+def say(*a):
+    print("[gpu-case]", *a, file=sys.stderr, flush=True)
+
+
+def bits(a):
+    return np.ascontiguousarray(a).view(np.uint64)
+
+
+def wide(bh, n, pairs=0):
+    """A belt with one body at 1,000 AU, and pairs of bodies one cell apart (most
+    of them split at the last depth)."""
+    pos, vel, m = bh.generate(bh.GEN_BELT, 3, n)
+    pos[n - 1] = [700.0, 500.0, 500.0]
+    cell = (pos.max(0) - pos.min(0)) / 2 ** 21
+    for k in range(pairs):
+        pos[20 + 2 * k] = pos[21 + 2 * k] + [cell[0], 0.0, 0.0]
+        vel[20 + 2 * k] = vel[21 + 2 * k]
+    return pos, vel, m
+
+
+def test_cutoff_chosen_for_a_graph_is_kept(bh):
+    n = 60000
+    data = wide(bh, n, pairs=200)
+    took, ref = {}, None
+    for cut in (21, -1):
+        say("graph cutoff", cut)
+        with bh.Engine(theta=1.05) as e:
+            e.set_moment_cutoff(cut)
+            e.set_bodies(*data)
+            e.step(4, HOUR)
+            t = []
+            for _ in range(9):
+                t0 = time.perf_counter()
+                e.step(10, HOUR)
+                t.append(time.perf_counter() - t0)
+            took[cut] = np.median(t)
+            assert e.graph_replays() > 80
+            s = e.get_bodies()
+        ref = ref or s
+        for k in ("pos", "vel", "acc"):
+            assert np.array_equal(bits(s[k]), bits(ref[k])), (cut, k)
+    say("ms a step", {k: 1e2 * v for k, v in took.items()})
+    assert took[-1] <= ROOM * took[21]
