@@ -386,15 +386,22 @@ void launch_permute(const Bodies& src, const Bodies& dst, const TreeBuffers& tb,
 // (one launch per populated depth, the plain form's order).
 void launch_build_tree(const Bodies& b, size_t n, TreeBuffers& tb, bool moments, hipStream_t s);
 void launch_tree_moments(size_t n, TreeBuffers& tb, hipStream_t s);
-// TreeBuffers::deep_from of the plain form when nothing is known of the tree.
-// Up to kDeepWhole bodies one workgroup sums all of it (a level takes it about
-// 0.9 us, a launch of a graph 1.3, of a stream 3: a step at 3,000 bodies takes
-// 248 us with cutoff 0, 252 with 10, 267 with 21; at 6,000 321, 315, 327).  Up
-// to 2^16 bodies few nodes lie at depth 10 and below (19,054: 487, 436, 447 us;
-// 60,000: 1061, 554, 567); larger trees get a launch per depth until a graph
-// capture has looked at one (choose_deep_from).
+// TreeBuffers::deep_from of the plain form.  Up to kDeepWhole bodies one
+// workgroup sums the whole tree; above that a graph takes the cutoff chosen from
+// a tree when it is captured (choose_deep_from).  Where nothing is known of the
+// tree (a step that is not replayed, the static evaluation) the workgroup may
+// have to sum all of it whatever the cutoff: one body far outside a belt puts
+// nearly every branching node at depth 10 and below.  So it does up to
+// kDeepBlind bodies, where that is faster than one launch per depth for every
+// shape of tree measured (a step with cutoff 0, and 21, us: 4,097 bodies belt
+// 131, 149, belt with a body at 1,000 AU 128, 144, cube 110, 127; 8,192 bodies
+// 179, 185, and 161, 164, and 134, 139; 10,000 bodies 200, 200, and 178, 176,
+// and 149, 151), and larger trees get a launch per depth.  (Cutoff 10 saves
+// 11 us of 200 to 570 where few nodes lie that deep, but 65,536 bodies with one
+// far away took 752 us a step with it and 268 with 21.)
 constexpr size_t kDeepWhole = 4096;
-inline int moments_cutoff(size_t n) { return n <= kDeepWhole ? 0 : n <= 65536 ? 10 : kMaxDepth; }
+constexpr size_t kDeepBlind = 8192;
+inline int moments_cutoff(size_t n) { return n <= kDeepBlind ? 0 : kMaxDepth; }
 // the mixed forms' light moments and boxes of the branching nodes, from the
 // pyramid of their leaves (four launches at every size)
 void launch_light_moments(size_t n, TreeBuffers& tb, hipStream_t s);

@@ -200,8 +200,9 @@ int bh_get_sort_stats(bh_ctx *ctx, int *near_path, int64_t *sorted_keys);
  * single workgroup, depth by depth, in one launch.  cutoff -1 (default): the
  * whole tree up to 4,096 bodies; else chosen from the current tree whenever a
  * step graph is captured, one below its deepest branching node (so the empty
- * depths cost one launch, not one each), and 10 up to 65,536 bodies or 21
- * until then; 0..21 fixes it (21: one launch per depth throughout).  Every cutoff
+ * depths cost one launch, not one each), and until then the whole tree up to
+ * 8,192 bodies and 21 above; 0..21 fixes it (21: one launch per depth
+ * throughout).  Every cutoff
  * gives the same bits. */
 int bh_set_moment_cutoff(bh_ctx *ctx, int cutoff);
 

@@ -57,3 +57,25 @@ def test_cutoff_chosen_for_a_graph_is_kept(bh):
             assert np.array_equal(bits(s[k]), bits(ref[k])), (cut, k)
     say("ms a step", {k: 1e2 * v for k, v in took.items()})
     assert took[-1] <= ROOM * took[21]
+
+
+@pytest.mark.parametrize("n", [4097, 8192, 8193, 30000, 65536])
+def test_cutoff_where_nothing_is_known_of_the_tree(bh, n):
+    data = wide(bh, n)
+    took, ref = {}, None
+    for cut in (21, -1):
+        say("eager cutoff", n, cut)
+        with bh.Engine(theta=1.05) as e:
+            e.set_graph(False)
+            e.set_bodies(*data)
+            e.set_moment_cutoff(cut)
+            t = []
+            for _ in range(15):
+                e.compute_accelerations(theta=1.05)
+                t.append(e.phase_ms()[2])
+            took[cut] = np.median(t)
+            s = e.get_bodies()
+        ref = ref or s
+        assert np.array_equal(bits(s["acc"]), bits(ref["acc"])), cut
+    say("ms of the tree", took)
+    assert took[-1] <= ROOM * took[21]
