@@ -359,7 +359,7 @@ int run_force(bh_ctx* c, int form, double theta, double G, double soft2, bool ki
         c->have_groups = true;
         return BH_OK;
     }
-    bh::launch_walk_order(c->n, tb, s);
+    bh::launch_walk_order(c->cur, c->n, tb, theta * theta, soft2, s);
     MARK(3);
     bh::WalkParams p{theta * theta, G, soft2, half_dt, kick_after ? 1 : 0};
     const bool cnt = c->counting;

@@ -54,6 +54,13 @@ constexpr uint32_t kMetaChain = 1u << 11;     // leaf chain starts above depth 2
 constexpr uint32_t kMetaMore = 1u << 12;
 constexpr uint32_t kMetaMidShift = 15;
 constexpr size_t kWaveMax = 20480;            // (at most 2 n - 1 walk indices: 16 bits)
+// Above kWaveFew bodies the plain walk of such a system looks at the length of
+// the lists first: k_walk_records counts the nodes that kListSamples of its
+// bodies would test into the rows of StepScalars::queue, one per XCD (the mixed
+// walk's, free here).
+constexpr size_t kWaveFew = 5500;
+constexpr uint32_t kListSamples = 16;
+__host__ __device__ inline bool counts_lists(size_t n) { return n > kWaveFew && n <= kWaveMax; }
 
 constexpr uint8_t kNoSplit = 0xff;   // delta of a boundary between two systems
 
@@ -219,15 +226,16 @@ __device__ inline double inv_sqrt_in_range(double x)
 // written by other XCDs, so every line's first touch goes to memory, and a
 // walk meets its lines one dependent load after the other.  (Plain walk of
 // 3,000 bodies 0.172 -> 0.148 ms, 19,054 0.355 -> 0.320, 50,021 0.534 ->
-// 0.489.)  Blocks of kThreads; bytes a multiple of 16.
+// 0.489.)  Blocks of kThreads; bytes a multiple of 16; the first `blocks` blocks
+// of the grid, all of which call it.
 constexpr size_t kWarmBytes = size_t{4} << 20;
 
 template <uint32_t kThreads = 256>
-__device__ inline void warm_l2(const void* base, size_t bytes)
+__device__ inline void warm_l2(const void* base, size_t bytes, uint32_t blocks = gridDim.x)
 {
     const uint4* p = static_cast<const uint4*>(base);
     const uint32_t total = static_cast<uint32_t>(bytes / sizeof(uint4));
-    const uint32_t xcd_blocks = (gridDim.x - (blockIdx.x & 7u) + 7u) / 8u;   // of this XCD
+    const uint32_t xcd_blocks = (blocks - (blockIdx.x & 7u) + 7u) / 8u;   // of this XCD
     const uint32_t stride = xcd_blocks * kThreads;
     constexpr uint32_t kU = 8;
     for (uint32_t i = blockIdx.x / 8u * kThreads + threadIdx.x; i < total; i += kU * stride) {
@@ -405,8 +413,9 @@ inline int moments_cutoff(size_t n) { return n <= kDeepBlind ? 0 : kMaxDepth; }
 // the mixed forms' light moments and boxes of the branching nodes, from the
 // pyramid of their leaves (four launches at every size)
 void launch_light_moments(size_t n, TreeBuffers& tb, hipStream_t s);
-// Walk-order records of the plain walk (after launch_build_tree).
-void launch_walk_order(size_t n, TreeBuffers& tb, hipStream_t s);
+// Walk-order records of the plain walk (after launch_build_tree), and for
+// counts_lists(n) the tests of the sample bodies.
+void launch_walk_order(const Bodies& b, size_t n, TreeBuffers& tb, double theta2, double soft2, hipStream_t s);
 
 struct WalkParams {
     double theta2, G, soft2, half_dt;

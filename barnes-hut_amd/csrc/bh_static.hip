@@ -232,7 +232,7 @@ int bh_compute_accelerations_static(int64_t n, const bh_vec3* pos, const double*
     L.tb.deep_from = moments_cutoff(N);
     launch_permute(L.cur, L.alt, L.tb, N, s);
     launch_build_tree(L.alt, N, L.tb, true, s);
-    launch_walk_order(N, L.tb, s);
+    launch_walk_order(L.alt, N, L.tb, theta * theta, soft2, s);
     const WalkParams p{theta * theta, G, soft2, 0.0, 0};
     launch_walk_plain(L.alt, N, L.tb, p, nullptr, nullptr, nullptr, s);
     k_static_scatter<<<static_cast<unsigned>((N + kNT - 1) / kNT), kNT, 0, s>>>(N, L.alt, acc_out);

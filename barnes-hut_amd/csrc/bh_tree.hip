@@ -923,10 +923,11 @@ __device__ inline double finish_com(double raw, double m)
     return (z * z + m * c) / (z + m);
 }
 
-// kMetaMore and the middle child of node t (see kMetaMore).  Children are in
+// kMetaMore and the middle child of node t (see kMetaMore), and the children of
+// a branching one.  Children are in
 // walk order from octant 7 down; the second half of c of them, from the
 // (c + 1) / 2-th, is a chain of its own.
-__device__ inline uint32_t child_chains(const TreeBuffers& tb, uint32_t M, uint32_t t, uint32_t par)
+__device__ inline uint32_t child_chains(const TreeBuffers& tb, uint32_t M, uint32_t t, uint32_t par, uint32_t& kids)
 {
     uint32_t meta = 0;
     if (par != kNone) {
@@ -955,15 +956,17 @@ __device__ inline uint32_t child_chains(const TreeBuffers& tb, uint32_t M, uint3
         // (not the first child, so no ancestor ends with it)
         const uint32_t w = mid < M ? suffix_count(tb, M, mid) - 1 : suffix_count(tb, M, tb.bhi[mid - M] + 1);
         meta |= (w & 0xffffu) << kMetaMidShift;
+        kids = all;
     }
     return meta;
 }
 
-__global__ __launch_bounds__(kNT) void k_walk_records(size_t n, TreeBuffers tb)
+// The record nd of node t (none past the last) and its place in the walk;
+// returns the children of a branching node (up to kWaveMax bodies; else 0).
+__device__ inline uint32_t walk_record(size_t t, size_t n, const TreeBuffers& tb, WalkNode& nd)
 {
-    const size_t t = static_cast<size_t>(blockIdx.x) * kNT + threadIdx.x;
     const uint32_t M = tb.sc->n_leaves, B = tb.sc->n_branch;
-    if (t >= static_cast<size_t>(M) + B) return;
+    if (t >= static_cast<size_t>(M) + B) return 0;
     const bool leaf = t < M;
     uint32_t w, skip, lo, test_depth;
     if (leaf) {
@@ -984,14 +987,13 @@ __global__ __launch_bounds__(kNT) void k_walk_records(size_t n, TreeBuffers tb)
     const uint32_t T = M + B;
     if (w >= T || skip > T || skip <= w) {
         atomicOr(&tb.sc->error, kErrWalkIndex);
-        return;
+        return 0;
     }
     const uint32_t par = tb.parent[t];
     const uint32_t top = (par == kNone) ? 0u : static_cast<uint32_t>(tb.bdepth[par - M]) + 1u;
     tb.windex[t] = w;
     const double* r = tb.raw + 4 * t;
     const double m = r[0];
-    WalkNode nd;
     if (0.0 + m == 0) {
         nd.x = nd.y = nd.z = 0.0;
         nd.m = 0.0;
@@ -1009,7 +1011,8 @@ __global__ __launch_bounds__(kNT) void k_walk_records(size_t n, TreeBuffers tb)
     nd.side2 = leaf ? (chain_leaf ? tb.sys[0].side2[kMaxDepth - 1] : INFINITY) : tb.sys[0].side2[test_depth];
     nd.skip = skip;
     uint32_t meta = test_depth | (top << kMetaTopShift);
-    if (n <= kWaveMax) meta |= child_chains(tb, M, static_cast<uint32_t>(t), par);
+    uint32_t kids = 0;
+    if (n <= kWaveMax) meta |= child_chains(tb, M, static_cast<uint32_t>(t), par, kids);
     if (leaf) {
         meta |= kMetaLeaf;
         if (top <= kMaxDepth - 1) meta |= kMetaChain;
@@ -1020,6 +1023,51 @@ __global__ __launch_bounds__(kNT) void k_walk_records(size_t n, TreeBuffers tb)
         const uint32_t e = tb.leaf_first[t + 1];
         for (uint32_t i = tb.leaf_first[t]; i < e; ++i) tb.self_w[i] = w;
     }
+    return kids;
+}
+
+// In a system that counts_lists, the tests that kListSamples bodies make of the
+// children of the nodes they open, added up over the branching nodes.  Whether a
+// body comes to a node at all is not looked at (where it accepts an ancestor it
+// mostly accepts the node too: within 7% of the walk's tests up to theta 1.2, up
+// to twice as many at 2).  The samples' positions are on their way while the
+// record is made.  (19,054 bodies: 8.0 -> 9.9 us, and the walk waits 1.3 us for
+// the counts.)
+__global__ __launch_bounds__(kNT) void k_walk_records(const double* __restrict__ px, const double* __restrict__ py,
+                                                      const double* __restrict__ pz, size_t n, TreeBuffers tb,
+                                                      double theta2, double soft2)
+{
+    __shared__ double4 s_at[kListSamples];
+    const bool lists = counts_lists(n);
+    double x = 0.0, y = 0.0, z = 0.0;
+    if (lists && threadIdx.x < kListSamples) {
+        const size_t i = (2 * threadIdx.x + 1) * n / (2 * kListSamples);
+        x = px[i];
+        y = py[i];
+        z = pz[i];
+    }
+    WalkNode nd{};
+    const uint32_t kids = walk_record(static_cast<size_t>(blockIdx.x) * kNT + threadIdx.x, n, tb, nd);
+    if (!lists) return;
+    if (threadIdx.x < kListSamples) s_at[threadIdx.x] = make_double4(x, y, z, 0.0);
+    __syncthreads();
+    const uint64_t any = __ballot(kids != 0u);
+    if (any == 0) return;
+    // the children of the nodes that a sample opens: sums of the bits of kids
+    uint64_t bit[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) bit[k] = __ballot(((kids >> k) & 1u) != 0u);
+    uint32_t tests = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kListSamples; ++q) {
+        const double4 at = s_at[q];
+        const double dx = nd.x - at.x, dy = nd.y - at.y, dz = nd.z - at.z;
+        const double r2 = dx * dx + dy * dy + dz * dz + soft2;
+        const uint64_t open = __ballot(nd.m != 0.0 && !(nd.side2 < theta2 * r2));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) tests += static_cast<uint32_t>(__popcll(open & bit[k])) << k;
+    }
+    if ((threadIdx.x & 63) == 0 && tests != 0u) atomicAdd(&tb.sc->queue[blockIdx.x & 7u][0], tests);
 }
 
 inline unsigned nblk(size_t n) { return static_cast<unsigned>((n + kNT - 1) / kNT > 0 ? (n + kNT - 1) / kNT : 1); }
@@ -1077,12 +1125,12 @@ void launch_build_tree(const Bodies& b, size_t n, TreeBuffers& tb, bool moments,
     if (moments) launch_tree_moments(n, tb, s);
 }
 
-void launch_walk_order(size_t n, TreeBuffers& tb, hipStream_t s)
+void launch_walk_order(const Bodies& b, size_t n, TreeBuffers& tb, double theta2, double soft2, hipStream_t s)
 {
     k_suffix_input<<<nblk(n), kNT, 0, s>>>(n, tb, tb.is_rep);
     scan_tile_offsets(tb.scan_tmp, n, s);
     scan_tile_apply(tb.is_rep, n, tb.scan_tmp, tb.suffix, &tb.sc->n_nodes, s);
-    k_walk_records<<<nblk(2 * n), kNT, 0, s>>>(n, tb);
+    k_walk_records<<<nblk(2 * n), kNT, 0, s>>>(b.px, b.py, b.pz, n, tb, theta2, soft2);
 }
 
 }  // namespace bh

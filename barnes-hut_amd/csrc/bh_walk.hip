@@ -294,6 +294,54 @@ __device__ inline Vec3 contribution(const WalkNode& nd, double px, double py, do
     return {s * dx, s * dy, s * dz};
 }
 
+__device__ inline void store_acc(const Bodies& b, size_t i, const Vec3& a, const WalkParams& p)
+{
+    store_acc(b, i, 0, a.x, p);
+    store_acc(b, i, 1, a.y, p);
+    store_acc(b, i, 2, a.z, p);
+}
+
+// One body's walk by one lane; the fetch of the next record comes before the
+// arithmetic of an accepted one.
+__device__ inline Vec3 walk_alone(const WalkNode* __restrict__ walk, uint32_t T, double px, double py, double pz,
+                                  uint32_t self, const WalkParams& p)
+{
+    Vec3 a{0.0, 0.0, 0.0};
+    WalkNode nd = load_node(walk, 0, T);
+    for (uint32_t cur = 0; cur < T;) {
+        const Decision d = decide(nd, px, py, pz, cur == self, p);
+        const uint32_t next = d.open ? cur + 1 : max(nd.skip, cur + 1);
+        const WalkNode nn = load_node(walk, next, T);
+        if (d.accept) {
+            const double s = pull(d.r2, nd.m, p.G);
+            a.x += s * d.dx;
+            a.y += s * d.dy;
+            a.z += s * d.dz;
+        }
+        cur = next;
+        nd = nn;
+    }
+    return a;
+}
+
+// Whether the per-lane walk is the faster one, by the tests of a mean body V:
+// 32 V < n - kWaveFew.  A wavefront's time for a body hardly depends on its
+// list, a lane's is proportional to it.  (n and theta alone do not tell: the
+// same limits for all had Kuiper belts of 20,480 bodies walked 1.4 times as long
+// as per lane, cubes 1.7 times, at the theta at which belts gain.)  Walks in us
+// per lane and by wavefronts (belt, Kuiper belt, cube; V in brackets): 8,192 bodies theta 1.05 187, 71 (809),
+// 87, 52 (212), 58, 48 (78); 12,288 theta 1.05 216, 114 (950), 80, 85 (256), 64,
+// 73 (84); 20,480 theta 1.05 279, 195 (915), 100, 139 (289), 73, 126 (97), theta
+// 0.5 747, 665 (2,990), 307, 246 (1,121), 163, 137 (532).
+__device__ inline bool short_lists(const StepScalars* sc, size_t n)
+{
+    uint32_t tests = 0;
+#pragma unroll
+    for (uint32_t x = 0; x < kXcds; ++x) tests += sc->queue[x][0];
+    static_assert(kListSamples == 16, "the tests of the samples are 16 V");
+    return 2 * tests < n - kWaveFew;
+}
+
 // Orders this wavefront's LDS accesses for its lanes (the LDS serves one
 // wavefront's instructions in order, so nothing is waited for).
 __device__ inline void wave_sync()
@@ -314,6 +362,15 @@ __global__ __launch_bounds__(64 * kWaves) void k_walk_wave(Bodies b, size_t n, u
     unsigned long long* const bits = all_bits + wave * words;
     WaveLds& l = ls[wave];
     const uint32_t T = min(sc->n_nodes, static_cast<uint32_t>(2 * n));
+    if (counts_lists(n) && short_lists(sc, n)) {
+        // per lane, as k_walk_plain does it
+        const uint32_t g = static_cast<uint32_t>((n + 64 * kWaves - 1) / (64 * kWaves)), used = (g + kXcds - 1) / kXcds * kXcds;
+        if (blockIdx.x >= used) return;
+        warm_l2<64 * kWaves>(walk, T * sizeof(WalkNode), used);
+        const size_t i = static_cast<size_t>(xcd_block(blockIdx.x, g)) * (64 * kWaves) + threadIdx.x;
+        if (i < n) store_acc(b, i, walk_alone(walk, T, b.px[i], b.py[i], b.pz[i], self_w[i], p), p);
+        return;
+    }
     warm_l2<64 * kWaves>(walk, T * sizeof(WalkNode));
     const size_t i = static_cast<size_t>(xcd_block(blockIdx.x, grid_blocks)) * kWaves + wave;
     if (i >= n || T == 0) return;
@@ -377,22 +434,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_walk_wave(Bodies b, size_t n, u
     wave_sync();
 
     if (!ok) {
-        if (lane) return;
-        double ax = 0.0, ay = 0.0, az = 0.0;
-        for (uint32_t cur = 0; cur < T;) {
-            const WalkNode nd = load_node(walk, cur, T);
-            const Decision d = decide(nd, px, py, pz, cur == self, p);
-            if (d.accept) {
-                const Vec3 c = contribution(nd, px, py, pz, p);
-                ax += c.x;
-                ay += c.y;
-                az += c.z;
-            }
-            cur = d.open ? cur + 1 : max(nd.skip, cur + 1);
-        }
-        store_acc(b, i, 0, ax, p);
-        store_acc(b, i, 1, ay, p);
-        store_acc(b, i, 2, az, p);
+        if (lane == 0) store_acc(b, i, walk_alone(walk, T, px, py, pz, self, p), p);
         return;
     }
 
@@ -483,14 +525,6 @@ __global__ __launch_bounds__(64 * kWaves) void k_walk_wave(Bodies b, size_t n, u
     if (lane < 3) store_acc(b, i, lane, acc, p);
 }
 
-// A wavefront per body up to 16,384 bodies, and to kWaveMax where the list is
-// not very short (theta <= 1.2): the work grows with n, the per-lane chains
-// hardly do.  Walk in ms, per-lane and by wavefronts (belt): 16,384 bodies
-// 0.273 and 0.170 (theta 1.05), 0.099 and 0.099 (theta 2); 20,000 bodies 0.300
-// and 0.203 (1.05), 0.797 and 0.741 (0.5), 0.104 and 0.117 (2); 24,000 bodies
-// 0.313 and 0.305 (1.05), 0.87 and 1.2 (0.5).
-bool by_wavefronts(size_t n, double theta2) { return n <= 16384 || (n <= kWaveMax && theta2 <= 1.44); }
-
 // How many walk indices a lane may be ahead of its wavefront's last one (0: no
 // limit).  The lanes of a wavefront drift apart, and then every lane's record
 // is a line of its own: 44 lines a visit at 300k bodies, one L1 lookup each for
@@ -525,7 +559,7 @@ void launch_walk_plain(const Bodies& b, size_t n, const TreeBuffers& tb, const W
     if (cnt_accept && cnt_open && cnt_test)
         k_walk_plain<true, false><<<grid, kNT, 0, s>>>(b, n, g, tb.walk, tb.self_w, tb.sc, tb.sys, p, 0u, cnt_accept, cnt_open,
                                                 cnt_test);
-    else if (by_wavefronts(n, p.theta2)) {
+    else if (n <= kWaveMax) {
         const uint32_t words = static_cast<uint32_t>((2 * n + 63) / 64);
         const uint32_t gw = static_cast<uint32_t>((n + kWaves - 1) / kWaves);
         k_walk_wave<<<(gw + kXcds - 1) / kXcds * kXcds, 64 * kWaves, kWaves * words * sizeof(uint64_t), s>>>(

@@ -441,8 +441,8 @@ def main():
     walk_ms = head["phase_ms"]["walk_kick"]
     achieved = work["flops_per_launch"] / (walk_ms * 1e-3) / 1e12
     if form == "plain":
-        # small systems take a wavefront per body (the library's rule on n and theta)
-        kname = "k_walk_wave" if n <= 16384 or (n <= 20480 and theta <= 1.2) else "k_walk_plain"
+        # small systems take a wavefront per body (or, where their lists are short, a lane, in the same kernel)
+        kname = "k_walk_wave" if n <= 20480 else "k_walk_plain"
         kern, peak, bound = f"{kname} (FP64 walk + fused half kick)", FP64_PEAK_TFLOPS, "valu_fp64"
         peak_note = "FP64 vector peak"
     else:
