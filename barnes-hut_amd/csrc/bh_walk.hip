@@ -329,10 +329,13 @@ __device__ inline Vec3 walk_alone(const WalkNode* __restrict__ walk, uint32_t T,
 // list, a lane's is proportional to it.  (n and theta alone do not tell: the
 // same limits for all had Kuiper belts of 20,480 bodies walked 1.4 times as long
 // as per lane, cubes 1.7 times, at the theta at which belts gain.)  Walks in us
-// per lane and by wavefronts (belt, Kuiper belt, cube; V in brackets): 8,192 bodies theta 1.05 187, 71 (809),
-// 87, 52 (212), 58, 48 (78); 12,288 theta 1.05 216, 114 (950), 80, 85 (256), 64,
-// 73 (84); 20,480 theta 1.05 279, 195 (915), 100, 139 (289), 73, 126 (97), theta
-// 0.5 747, 665 (2,990), 307, 246 (1,121), 163, 137 (532).
+// per lane and by wavefronts (belt, Kuiper belt, cube; V in brackets): 8,192
+// bodies theta 1.05 190, 73 (677), 90, 54 (212), 44, 36 (78); 12,288 theta 1.05
+// 218, 116 (786), 81, 86 (226), 48, 55 (84); 20,480 theta 1.05 285, 200 (894),
+// 100, 139 (279), 53, 91 (90), theta 0.5 744, 664 (2,990), 315, 253 (1,121), 171,
+// 143 (532).  Over seven shapes, 5,000 to 20,480 bodies and theta 0.3 to 3 the
+// choice is within 5% of the better walk in 356 of 378 cases, and up to theta 1.2
+// in 246 of 252; 1.26 the worst of those (a cube of 8,192 bodies, 44 us for 35).
 __device__ inline bool short_lists(const StepScalars* sc, size_t n)
 {
     uint32_t tests = 0;
@@ -537,11 +540,16 @@ __global__ __launch_bounds__(64 * kWaves) void k_walk_wave(Bodies b, size_t n, u
 // 0.94, 0.89 / 1.03 / 1.12 / 1.25; 300k 2.12, 2.06 / 2.04 / 2.08 / 2.20, theta
 // 0.5 11.6, 11.0 / 10.7 / 10.4 / 10.1; Trojan 300k theta 0.7 5.4, 5.1 / 4.9 /
 // 4.6 / 4.3; Kuiper 300k theta 0.7 1.35, 1.24 / 1.20 / 1.20 / 1.28; Trojan 1M
-// 7.8, 6.7 / 6.1 / 5.9 / 5.8.
+// 7.8, 6.7 / 6.1 / 5.9 / 5.8.  With the rule against no limit, belt / Trojan /
+// Kuiper: 100k theta 0.5 0.96 / 0.96 / 1.01, 1.05 0.98 / 0.96 / 1.06; 130k theta
+// 0.5 0.92 / 0.96 / 0.98, 1.05 0.94 / 0.98 / 0.99; 300k theta 1.05 0.94 / 0.91 /
+// 0.94, 2 0.93 / 0.91 / 1.10; 1M theta 1.05 0.81 / 0.79 / 0.91.  Above theta 1.2
+// it lost below 160k: 100k theta 1.5 0.97 / 1.06 / 1.04, 2 1.12 / 1.09 / 1.08,
+// 130k 1.5 1.04 / 1.01 / 1.03, 2 1.06 / 1.10 / 1.08.
 uint32_t walk_lead(size_t n, double theta2)
 {
     if (n < 100000) return 0u;
-    if (n < 160000) return 30000u;
+    if (n < 160000) return theta2 > 1.44 ? 0u : 30000u;
     return theta2 < 0.64 ? 4000u : 10000u;
 }
 
