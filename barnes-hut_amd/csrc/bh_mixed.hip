@@ -901,355 +901,355 @@ __device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, 
     uint32_t* slots = reinterpret_cast<uint32_t*>(lds + kListBytes) + w * 64;
     uint32_t* stk = reinterpret_cast<uint32_t*>(lds + kListBytes + kRoundSlots * 4);
     double* part_sum = reinterpret_cast<double*>(lds);
-            const uint64_t t_start = wall_clock64();
-            const WalkArgsP ag = args_here(args);
-            const uint32_t b0 = uni(ag->mb.gfirst[g]);
-            const uint32_t cnt = uni(ag->mb.gfirst[g + 1]) - b0;
-            // lane = body for the box, the heavy bodies and the results
-            const bool valid = static_cast<uint32_t>(lane) < cnt;
-            const uint32_t i = b0 + (valid ? static_cast<uint32_t>(lane) : 0u);
-            const double x = ag->b.px[i], y = ag->b.py[i], z = ag->b.pz[i];
-            // virtual lanes: share and body of pass v (share >> 8 | body; a lane
-            // past the last share repeats share 0 and its sum is never read)
-            const uint32_t S = list_shares(cnt), invS = (65535u + S) / S;
-            uint32_t vl[V];
-    #pragma unroll
-            for (int v = 0; v < V; ++v) {
-                const uint32_t t = static_cast<uint32_t>((v * NW + w) * 64 + lane);
-                const uint32_t sh = t / cnt;
-                vl[v] = (t - sh * cnt) | ((sh < S ? sh : 0u) << 8);
-            }
-            const double lox = wave_min(x), loy = wave_min(y), loz = wave_min(z);
-            const double hix = wave_max(x), hiy = wave_max(y), hiz = wave_max(z);
-            const double cx = 0.5 * (lox + hix), cy = 0.5 * (loy + hiy), cz = 0.5 * (loz + hiz);
-            const double hx = 0.5 * (hix - lox), hy = 0.5 * (hiy - loy), hz = 0.5 * (hiz - loz);
-            const float ox = static_cast<float>(x - cx);
-            const float oy = static_cast<float>(y - cy);
-            const float oz = static_cast<float>(z - cz);
-            Acc3 acc[V];
-            uint32_t ln = 0, sp = 1, n_inter = 0, n_visit = 0, n_steps = 0;
-            bool overflow = false;
-            const uint32_t gsys = ag->tb.n_sys == 1 ? 0u : uni(ag->tb.bsys[b0]);
-            const MNode* __restrict__ nodes = ag->mb.node;
-            const float r2_0 = list_r2_floor(nodes[gsys].gm, static_cast<float>(ag->p.soft2));   // the system's root
-            // heavy bodies of the system: FP64 direct sum, the ranks k = q mod 4 in
-            // rank order into partial q (one or more of the four per wavefront),
-            // the partials added in order
-            double hax = 0.0, hay = 0.0, haz = 0.0;
-            {
-                const SysScalars* sy = ag->tb.sys + gsys;
-                const uint32_t nh = sy->n_heavy;
-                const double soft2 = ag->p.soft2, grav = ag->p.G;
-                // lane k loads heavy body k (one load latency for all of them); the
-                // loop reads them back as wave constants
-                uint32_t hj = kNone;
-                double hpx = 0.0, hpy = 0.0, hpz = 0.0, hpm = 0.0;
-                if (static_cast<uint32_t>(lane) < nh) {
-                    hj = sy->heavy_slot[lane];
-                    hpx = ag->b.px[hj];
-                    hpy = ag->b.py[hj];
-                    hpz = ag->b.pz[hj];
-                    hpm = ag->b.m[hj];
-                }
-    #pragma unroll 1
-                for (int v = 0; v < V; ++v) {
-                    double sx = 0.0, sy_ = 0.0, sz = 0.0;
-                    for (uint32_t k = static_cast<uint32_t>(v * NW + w); k < nh; k += 4u) {
-                        const uint32_t j = lane_u32(hj, k);
-                        const double dx = lane_f64(hpx, k) - x, dy = lane_f64(hpy, k) - y, dz = lane_f64(hpz, k) - z;
-                        const double r2 = dx * dx + dy * dy + dz * dz + soft2;
-                        const bool pair = j != i && r2 > 0.0;
-                        const double invR = __all(inv_sqrt_takes(r2) | !pair) ? inv_sqrt_in_range(pair ? r2 : 1.0)
-                                                                              : 1.0 / sqrt(pair ? r2 : 1.0);
-                        const double s = grav * lane_f64(hpm, k) * (invR * invR * invR);
-                        if (pair) {
-                            sx += s * dx;
-                            sy_ += s * dy;
-                            sz += s * dz;
-                        }
-                    }
-                    if (NW == 1) {
-                        hax += sx;
-                        hay += sy_;
-                        haz += sz;
-                    } else {
-                        double* q = part_sum + (v * NW + w) * 192 + lane;
-                        q[0] = sx;
-                        q[64] = sy_;
-                        q[128] = sz;
-                    }
+    const uint64_t t_start = wall_clock64();
+    const WalkArgsP ag = args_here(args);
+    const uint32_t b0 = uni(ag->mb.gfirst[g]);
+    const uint32_t cnt = uni(ag->mb.gfirst[g + 1]) - b0;
+    // lane = body for the box, the heavy bodies and the results
+    const bool valid = static_cast<uint32_t>(lane) < cnt;
+    const uint32_t i = b0 + (valid ? static_cast<uint32_t>(lane) : 0u);
+    const double x = ag->b.px[i], y = ag->b.py[i], z = ag->b.pz[i];
+    // virtual lanes: share and body of pass v (share >> 8 | body; a lane
+    // past the last share repeats share 0 and its sum is never read)
+    const uint32_t S = list_shares(cnt), invS = (65535u + S) / S;
+    uint32_t vl[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const uint32_t t = static_cast<uint32_t>((v * NW + w) * 64 + lane);
+        const uint32_t sh = t / cnt;
+        vl[v] = (t - sh * cnt) | ((sh < S ? sh : 0u) << 8);
+    }
+    const double lox = wave_min(x), loy = wave_min(y), loz = wave_min(z);
+    const double hix = wave_max(x), hiy = wave_max(y), hiz = wave_max(z);
+    const double cx = 0.5 * (lox + hix), cy = 0.5 * (loy + hiy), cz = 0.5 * (loz + hiz);
+    const double hx = 0.5 * (hix - lox), hy = 0.5 * (hiy - loy), hz = 0.5 * (hiz - loz);
+    const float ox = static_cast<float>(x - cx);
+    const float oy = static_cast<float>(y - cy);
+    const float oz = static_cast<float>(z - cz);
+    Acc3 acc[V];
+    uint32_t ln = 0, sp = 1, n_inter = 0, n_visit = 0, n_steps = 0;
+    bool overflow = false;
+    const uint32_t gsys = ag->tb.n_sys == 1 ? 0u : uni(ag->tb.bsys[b0]);
+    const MNode* __restrict__ nodes = ag->mb.node;
+    const float r2_0 = list_r2_floor(nodes[gsys].gm, static_cast<float>(ag->p.soft2));   // the system's root
+    // heavy bodies of the system: FP64 direct sum, the ranks k = q mod 4 in
+    // rank order into partial q (one or more of the four per wavefront),
+    // the partials added in order
+    double hax = 0.0, hay = 0.0, haz = 0.0;
+    {
+        const SysScalars* sy = ag->tb.sys + gsys;
+        const uint32_t nh = sy->n_heavy;
+        const double soft2 = ag->p.soft2, grav = ag->p.G;
+        // lane k loads heavy body k (one load latency for all of them); the
+        // loop reads them back as wave constants
+        uint32_t hj = kNone;
+        double hpx = 0.0, hpy = 0.0, hpz = 0.0, hpm = 0.0;
+        if (static_cast<uint32_t>(lane) < nh) {
+            hj = sy->heavy_slot[lane];
+            hpx = ag->b.px[hj];
+            hpy = ag->b.py[hj];
+            hpz = ag->b.pz[hj];
+            hpm = ag->b.m[hj];
+        }
+#pragma unroll 1
+        for (int v = 0; v < V; ++v) {
+            double sx = 0.0, sy_ = 0.0, sz = 0.0;
+            for (uint32_t k = static_cast<uint32_t>(v * NW + w); k < nh; k += 4u) {
+                const uint32_t j = lane_u32(hj, k);
+                const double dx = lane_f64(hpx, k) - x, dy = lane_f64(hpy, k) - y, dz = lane_f64(hpz, k) - z;
+                const double r2 = dx * dx + dy * dy + dz * dz + soft2;
+                const bool pair = j != i && r2 > 0.0;
+                const double invR = __all(inv_sqrt_takes(r2) | !pair) ? inv_sqrt_in_range(pair ? r2 : 1.0)
+                                                                      : 1.0 / sqrt(pair ? r2 : 1.0);
+                const double s = grav * lane_f64(hpm, k) * (invR * invR * invR);
+                if (pair) {
+                    sx += s * dx;
+                    sy_ += s * dy;
+                    sz += s * dz;
                 }
             }
+            if (NW == 1) {
+                hax += sx;
+                hay += sy_;
+                haz += sz;
+            } else {
+                double* q = part_sum + (v * NW + w) * 192 + lane;
+                q[0] = sx;
+                q[64] = sy_;
+                q[128] = sz;
+            }
+        }
+    }
+    if (NW > 1) {
+        __syncthreads();
+        for (int q = 0; q < 4; ++q) {
+            hax += part_sum[q * 192 + lane];
+            hay += part_sum[q * 192 + 64 + lane];
+            haz += part_sum[q * 192 + 128 + lane];
+        }
+    }
+    // relative opening test: a node is also opened while its quadrupole
+    // scale G Q / D^4 exceeds alpha x the smallest heavy-body acceleration
+    // of the group (the acceleration every body of these systems is made of)
+    const double ah = valid ? sqrt(hax * hax + hay * hay + haz * haz) : INFINITY;
+    const double aref = wave_min(ah);
+    const double alpha = ag->p.alpha, theta2 = ag->p.theta2;
+    const double qlim = (alpha > 0.0 && aref > 0.0 && aref < INFINITY) ? alpha * aref : INFINITY;
+    // up to theta^2 = kSafe2 (and without a limit) the extent test implies the rest
+    const bool relative = theta2 > kSafe2 && __any(qlim < INFINITY);
+    bool deep = false;      // the stack was over kNarrowRoom
+    bool recount = false;   // the second pass of a training walk
+    if (tid == 0) stk[0] = stack_range(gsys, 1, false);   // the root of the group's system
+    group_sync<NW>();   // (also: every wavefront has read the exchanged sums)
+    for (bool last = false; !last;) {
+        // pop up to 64 ranges, one per lane, while the stack cannot
+        // overflow; when it is empty one more turn flushes the rest of the list
+        last = sp == 0u || overflow;
+        Ranges r{0u, 0u, 0u, 0u};
+        if (!last) {
+            deep |= sp > kNarrowRoom;
+            const uint32_t P = pop_count(sp, recount);
+            const bool has = static_cast<uint32_t>(lane) < P;
+            const uint32_t e = has ? stk[sp - 1 - lane] : 0u;
+            sp -= P;
+            r.count = has ? ((e >> 27) & 7u) + 1u : 0u;
+            const uint32_t incl = wave_incl_scan(r.count);
+            r.total = lane_u32(incl, 63);
+            r.excl = incl - r.count;
+            r.info = (e & 0x87ffffffu) - r.excl;
+            n_visit += r.total;
+            if (NW == 1) write_slots(r, slots);
+        }
+        uint32_t ent = 0u;
+        MNode nd{};
+        if (static_cast<uint32_t>(w) * 64u < r.total) ent = fetch_slot<NW>(r, static_cast<uint32_t>(w) * 64u, slots, nodes, nd);
+        uint32_t base = 0;
+        do {
+            // the opening test; a leaf of one body is always accepted, one
+            // of several never (its bodies are), and lanes without a node
+            // have no mass
+            const double rx = nd.x - cx, ry = nd.y - cy, rz = nd.z - cz;
+            const double ex = fmax(fabs(rx) - hx, 0.0);
+            const double ey = fmax(fabs(ry) - hy, 0.0);
+            const double ez = fmax(fabs(rz) - hz, 0.0);
+            const double d2 = ex * ex + ey * ey + ez * ez;
+            bool pass = nd.size2 < theta2 * d2;
+            if (relative) pass &= nd.size2 <= kSafe2 * d2 || static_cast<double>(nd.gq) <= qlim * (d2 * d2);
+            const bool live = nd.gm != 0.f;
+            const uint32_t push = nd.push, info = nd.info;
+            bool app = live && (pass || info == (kMLeaf | 1u));
+            const bool open = live && !app;
+            const bool open_big = open && info > (kMLeaf | 8u);
+            float4 q = make_float4(static_cast<float>(rx), static_cast<float>(ry), static_cast<float>(rz), nd.gm);
+            if (static_cast<int32_t>(ent) < 0) app = body_entry(args_here(args), ent & 0x7fffffffu, cx, cy, cz, q);
+            // the next chunk's nodes are on their way while this chunk is
+            // listed (without the prefetch: +4% on the 300k walk)
+            const uint32_t sb_n = base + static_cast<uint32_t>((NW + w) * 64);
+            ent = 0u;
+            nd.gm = 0.f;
+            if (sb_n < r.total) ent = fetch_slot<NW>(r, sb_n, slots, nodes, nd);
+            // list entries and stack pushes of this chunk (one per lane at
+            // most), and leaves of more than 8 co-keyed bodies (see below)
+            uint64_t am = __ballot(app);
+            const uint64_t pm = __ballot(open && !open_big);
+            uint64_t big = __ballot(open_big);
+            // counts: entries | pushes << 10 | chunks with such leaves << 20,
+            // of all NW chunks and of those before this wavefront's
+            const uint32_t word = static_cast<uint32_t>(__popcll(am)) |
+                                  static_cast<uint32_t>(__popcll(pm)) << 10 | (big ? 1u << 20 : 0u);
+            uint32_t all = word, before = 0;
+            uint32_t* const row = s_word[turn_no & 1u];
             if (NW > 1) {
+                if (lane == 0) row[w] = word;
                 __syncthreads();
-                for (int q = 0; q < 4; ++q) {
-                    hax += part_sum[q * 192 + lane];
-                    hay += part_sum[q * 192 + 64 + lane];
-                    haz += part_sum[q * 192 + 128 + lane];
+                ++turn_no;
+                all = 0;
+#pragma unroll
+                for (int c = 0; c < NW; ++c) {
+                    const uint32_t v = row[c];
+                    before += c < w ? v : 0u;
+                    all += v;
                 }
+                all = uni(all);
+                before = uni(before);
             }
-            // relative opening test: a node is also opened while its quadrupole
-            // scale G Q / D^4 exceeds alpha x the smallest heavy-body acceleration
-            // of the group (the acceleration every body of these systems is made of)
-            const double ah = valid ? sqrt(hax * hax + hay * hay + haz * haz) : INFINITY;
-            const double aref = wave_min(ah);
-            const double alpha = ag->p.alpha, theta2 = ag->p.theta2;
-            const double qlim = (alpha > 0.0 && aref > 0.0 && aref < INFINITY) ? alpha * aref : INFINITY;
-            // up to theta^2 = kSafe2 (and without a limit) the extent test implies the rest
-            const bool relative = theta2 > kSafe2 && __any(qlim < INFINITY);
-            bool deep = false;      // the stack was over kNarrowRoom
-            bool recount = false;   // the second pass of a training walk
-            if (tid == 0) stk[0] = stack_range(gsys, 1, false);   // the root of the group's system
-            group_sync<NW>();   // (also: every wavefront has read the exchanged sums)
-            for (bool last = false; !last;) {
-                // pop up to 64 ranges, one per lane, while the stack cannot
-                // overflow; when it is empty one more turn flushes the rest of the list
-                last = sp == 0u || overflow;
-                Ranges r{0u, 0u, 0u, 0u};
-                if (!last) {
-                    deep |= sp > kNarrowRoom;
-                    const uint32_t P = pop_count(sp, recount);
-                    const bool has = static_cast<uint32_t>(lane) < P;
-                    const uint32_t e = has ? stk[sp - 1 - lane] : 0u;
-                    sp -= P;
-                    r.count = has ? ((e >> 27) & 7u) + 1u : 0u;
-                    const uint32_t incl = wave_incl_scan(r.count);
-                    r.total = lane_u32(incl, 63);
-                    r.excl = incl - r.count;
-                    r.info = (e & 0x87ffffffu) - r.excl;
-                    n_visit += r.total;
-                    if (NW == 1) write_slots(r, slots);
-                }
-                uint32_t ent = 0u;
-                MNode nd{};
-                if (static_cast<uint32_t>(w) * 64u < r.total) ent = fetch_slot<NW>(r, static_cast<uint32_t>(w) * 64u, slots, nodes, nd);
-                uint32_t base = 0;
-                do {
-                    // the opening test; a leaf of one body is always accepted, one
-                    // of several never (its bodies are), and lanes without a node
-                    // have no mass
-                    const double rx = nd.x - cx, ry = nd.y - cy, rz = nd.z - cz;
-                    const double ex = fmax(fabs(rx) - hx, 0.0);
-                    const double ey = fmax(fabs(ry) - hy, 0.0);
-                    const double ez = fmax(fabs(rz) - hz, 0.0);
-                    const double d2 = ex * ex + ey * ey + ez * ez;
-                    bool pass = nd.size2 < theta2 * d2;
-                    if (relative) pass &= nd.size2 <= kSafe2 * d2 || static_cast<double>(nd.gq) <= qlim * (d2 * d2);
-                    const bool live = nd.gm != 0.f;
-                    const uint32_t push = nd.push, info = nd.info;
-                    bool app = live && (pass || info == (kMLeaf | 1u));
-                    const bool open = live && !app;
-                    const bool open_big = open && info > (kMLeaf | 8u);
-                    float4 q = make_float4(static_cast<float>(rx), static_cast<float>(ry), static_cast<float>(rz), nd.gm);
-                    if (static_cast<int32_t>(ent) < 0) app = body_entry(args_here(args), ent & 0x7fffffffu, cx, cy, cz, q);
-                    // the next chunk's nodes are on their way while this chunk is
-                    // listed (without the prefetch: +4% on the 300k walk)
-                    const uint32_t sb_n = base + static_cast<uint32_t>((NW + w) * 64);
-                    ent = 0u;
-                    nd.gm = 0.f;
-                    if (sb_n < r.total) ent = fetch_slot<NW>(r, sb_n, slots, nodes, nd);
-                    // list entries and stack pushes of this chunk (one per lane at
-                    // most), and leaves of more than 8 co-keyed bodies (see below)
-                    uint64_t am = __ballot(app);
-                    const uint64_t pm = __ballot(open && !open_big);
-                    uint64_t big = __ballot(open_big);
-                    // counts: entries | pushes << 10 | chunks with such leaves << 20,
-                    // of all NW chunks and of those before this wavefront's
-                    const uint32_t word = static_cast<uint32_t>(__popcll(am)) |
-                                          static_cast<uint32_t>(__popcll(pm)) << 10 | (big ? 1u << 20 : 0u);
-                    uint32_t all = word, before = 0;
-                    uint32_t* const row = s_word[turn_no & 1u];
-                    if (NW > 1) {
-                        if (lane == 0) row[w] = word;
+            const uint32_t need = (all >> 10) & 0x3ffu;
+            if (sp + need > static_cast<uint32_t>(kStackCap)) {
+                if (tid == 0) atomicOr(&sc->error, kErrStack);
+                overflow = true;
+            } else {
+                // one range per opened node or leaf of at most 8 bodies
+                if (open && !open_big) stk[sp + ((before >> 10) & 0x3ffu) + rank_below(pm)] = push;
+                sp += need;
+            }
+            if (!last && all < (1u << 20) && ln + (all & 0x3ffu) <= static_cast<uint32_t>(kListCap)) {
+                if (app) list[ln + (before & 0x3ffu) + rank_below(am)] = q;
+                ln += all & 0x3ffu;
+                n_inter += all & 0x3ffu;
+            } else {
+                // The list is flushed before the chunk that does not fit (and
+                // at the end).  A leaf of more than 8 co-keyed bodies
+                // (duplicate or nearly coincident positions) puts its bodies
+                // on the list directly, 64 at a time, so the stack does not
+                // grow with its size: while a round holds such leaves its
+                // chunks take turns, wavefront `turn` appending its entries,
+                // then its leaves' bodies.
+                const bool turns = all >= (1u << 20);
+                uint32_t turn = 0, big_k0 = 0;
+                for (bool more = true, first = true; more; first = false) {
+                    uint32_t words[NW];   // entries of each chunk, | 1 << 20 while its leaves have bodies left
+                    const bool mine = !turns || turn == static_cast<uint32_t>(w);
+                    am = __ballot(app && mine);
+                    if (NW == 1) {
+                        words[0] = static_cast<uint32_t>(__popcll(am)) | (big ? 1u << 20 : 0u);
+                    } else if (first) {
+#pragma unroll
+                        for (int c = 0; c < NW; ++c)
+                            words[c] = !turns || c == 0 ? uni(row[c]) & 0x1003ffu : 0u;
+                    } else {
+                        uint32_t* const rw = s_word[turn_no & 1u];
+                        if (lane == 0)
+                            rw[w] = static_cast<uint32_t>(__popcll(am)) | (mine && big ? 1u << 20 : 0u);
                         __syncthreads();
                         ++turn_no;
-                        all = 0;
-    #pragma unroll
+#pragma unroll
+                        for (int c = 0; c < NW; ++c) words[c] = uni(rw[c]);
+                    }
+                    for (int c0 = 0;;) {
+                        uint32_t l1 = ln, at = 0;
+                        int c1 = c0;
+#pragma unroll
                         for (int c = 0; c < NW; ++c) {
-                            const uint32_t v = row[c];
-                            before += c < w ? v : 0u;
-                            all += v;
-                        }
-                        all = uni(all);
-                        before = uni(before);
-                    }
-                    const uint32_t need = (all >> 10) & 0x3ffu;
-                    if (sp + need > static_cast<uint32_t>(kStackCap)) {
-                        if (tid == 0) atomicOr(&sc->error, kErrStack);
-                        overflow = true;
-                    } else {
-                        // one range per opened node or leaf of at most 8 bodies
-                        if (open && !open_big) stk[sp + ((before >> 10) & 0x3ffu) + rank_below(pm)] = push;
-                        sp += need;
-                    }
-                    if (!last && all < (1u << 20) && ln + (all & 0x3ffu) <= static_cast<uint32_t>(kListCap)) {
-                        if (app) list[ln + (before & 0x3ffu) + rank_below(am)] = q;
-                        ln += all & 0x3ffu;
-                        n_inter += all & 0x3ffu;
-                    } else {
-                        // The list is flushed before the chunk that does not fit (and
-                        // at the end).  A leaf of more than 8 co-keyed bodies
-                        // (duplicate or nearly coincident positions) puts its bodies
-                        // on the list directly, 64 at a time, so the stack does not
-                        // grow with its size: while a round holds such leaves its
-                        // chunks take turns, wavefront `turn` appending its entries,
-                        // then its leaves' bodies.
-                        const bool turns = all >= (1u << 20);
-                        uint32_t turn = 0, big_k0 = 0;
-                        for (bool more = true, first = true; more; first = false) {
-                            uint32_t words[NW];   // entries of each chunk, | 1 << 20 while its leaves have bodies left
-                            const bool mine = !turns || turn == static_cast<uint32_t>(w);
-                            am = __ballot(app && mine);
-                            if (NW == 1) {
-                                words[0] = static_cast<uint32_t>(__popcll(am)) | (big ? 1u << 20 : 0u);
-                            } else if (first) {
-    #pragma unroll
-                                for (int c = 0; c < NW; ++c)
-                                    words[c] = !turns || c == 0 ? uni(row[c]) & 0x1003ffu : 0u;
-                            } else {
-                                uint32_t* const rw = s_word[turn_no & 1u];
-                                if (lane == 0)
-                                    rw[w] = static_cast<uint32_t>(__popcll(am)) | (mine && big ? 1u << 20 : 0u);
-                                __syncthreads();
-                                ++turn_no;
-    #pragma unroll
-                                for (int c = 0; c < NW; ++c) words[c] = uni(rw[c]);
-                            }
-                            for (int c0 = 0;;) {
-                                uint32_t l1 = ln, at = 0;
-                                int c1 = c0;
-    #pragma unroll
-                                for (int c = 0; c < NW; ++c) {
-                                    if (c >= c0 && c == c1 && l1 + (words[c] & 0x3ffu) <= static_cast<uint32_t>(kListCap)) {
-                                        if (c == w) at = l1;
-                                        l1 += words[c] & 0x3ffu;
-                                        ++c1;
-                                    }
-                                }
-                                if (w >= c0 && w < c1 && ((am >> lane) & 1u)) list[at + rank_below(am)] = q;
-                                n_inter += l1 - ln;
-                                ln = l1;
-                                c0 = c1;
-                                if (c0 == NW && !last) break;
-                                // flush: padded with entries of no mass to S shares
-                                const uint32_t len = share_len(ln, S, invS, cnt);
-                                if (tid < 64 && ln + static_cast<uint32_t>(lane) < S * len)
-                                    list[ln + static_cast<uint32_t>(lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
-                                group_sync<NW>();
-    #pragma unroll
-                                for (int v = 0; v < V; ++v) {
-                                    if (!recount && static_cast<uint32_t>((v * NW + w) * 64) < S * cnt) {
-                                        const int src = static_cast<int>(vl[v] & 0xffu);
-                                        share_sum(list + (vl[v] >> 8) * len, len, __shfl(ox, src, 64), __shfl(oy, src, 64),
-                                                  __shfl(oz, src, 64), r2_0, acc[v]);
-                                    }
-                                }
-                                n_steps += list_cost(ln, cnt);
-                                group_sync<NW>();
-                                ln = 0;
-                                if (c0 == NW) break;
-                            }
-                            more = turns;
-                            if (turns) {
-                                // the next 64 bodies of this turn's leaves, or the next turn
-                                if ((words[turn] >> 20) != 0u) {
-                                    if (turn == static_cast<uint32_t>(w)) {
-                                        const uint32_t l = static_cast<uint32_t>(__builtin_ctzll(big));
-                                        const uint32_t j0 = lane_u32(push, l) & 0x07ffffffu, c = lane_u32(info, l) & ~kMLeaf;
-                                        const uint32_t j = j0 + big_k0 + static_cast<uint32_t>(lane);
-                                        app = j < j0 + c && body_entry(args_here(args), j, cx, cy, cz, q);
-                                        big_k0 += 64u;
-                                        if (big_k0 >= c) {
-                                            big_k0 = 0;
-                                            big &= big - 1;
-                                        }
-                                    }
-                                } else {
-                                    more = ++turn < static_cast<uint32_t>(NW);
-                                }
+                            if (c >= c0 && c == c1 && l1 + (words[c] & 0x3ffu) <= static_cast<uint32_t>(kListCap)) {
+                                if (c == w) at = l1;
+                                l1 += words[c] & 0x3ffu;
+                                ++c1;
                             }
                         }
+                        if (w >= c0 && w < c1 && ((am >> lane) & 1u)) list[at + rank_below(am)] = q;
+                        n_inter += l1 - ln;
+                        ln = l1;
+                        c0 = c1;
+                        if (c0 == NW && !last) break;
+                        // flush: padded with entries of no mass to S shares
+                        const uint32_t len = share_len(ln, S, invS, cnt);
+                        if (tid < 64 && ln + static_cast<uint32_t>(lane) < S * len)
+                            list[ln + static_cast<uint32_t>(lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
+                        group_sync<NW>();
+#pragma unroll
+                        for (int v = 0; v < V; ++v) {
+                            if (!recount && static_cast<uint32_t>((v * NW + w) * 64) < S * cnt) {
+                                const int src = static_cast<int>(vl[v] & 0xffu);
+                                share_sum(list + (vl[v] >> 8) * len, len, __shfl(ox, src, 64), __shfl(oy, src, 64),
+                                          __shfl(oz, src, 64), r2_0, acc[v]);
+                            }
+                        }
+                        n_steps += list_cost(ln, cnt);
+                        group_sync<NW>();
+                        ln = 0;
+                        if (c0 == NW) break;
                     }
-                    base += NW * 64u;
-                } while (base < r.total && !overflow);
-                if (last && deep && !recount && !overflow && args_here(args)->p.count_narrow != 0) {
-                    last = false;
-                    recount = true;
-                    sp = 1u;
-                    n_inter = n_visit = n_steps = 0u;
-                    if (tid == 0) stk[0] = stack_range(gsys, 1, false);
-                }
-                group_sync<NW>();   // the next round reads the stack
-            }
-            // the virtual lanes' sums (a Kahan sum's value is s - c: c holds the
-            // negative of the rounding lost), added in FP64 in share order
-            double lacc[3];
-            if (NW == 1) {
-    #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-    #pragma unroll
-                    for (int v = 0; v < V; ++v)
-                        part_sum[v * 64 + lane] = static_cast<double>(a == 0 ? acc[v].sx : (a == 1 ? acc[v].sy : acc[v].sz)) -
-                                                  static_cast<double>(a == 0 ? acc[v].cx : (a == 1 ? acc[v].cy : acc[v].cz));
-                    __builtin_amdgcn_wave_barrier();
-                    double t = 0.0;
-                    for (uint32_t k = 0; k < S; ++k) t += part_sum[k * cnt + (valid ? lane : 0)];
-                    lacc[a] = t;
-                    __builtin_amdgcn_wave_barrier();
-                }
-            } else {
-    #pragma unroll
-                for (int v = 0; v < V; ++v) {
-                    double* q = part_sum + (v * NW + w) * 64 + lane;
-                    q[0] = static_cast<double>(acc[v].sx) - static_cast<double>(acc[v].cx);
-                    q[256] = static_cast<double>(acc[v].sy) - static_cast<double>(acc[v].cy);
-                    q[512] = static_cast<double>(acc[v].sz) - static_cast<double>(acc[v].cz);
-                }
-                __syncthreads();
-    #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    double t = 0.0;
-                    if (a % NW == w)
-                        for (uint32_t k = 0; k < S; ++k) t += part_sum[a * 256 + k * cnt + (valid ? lane : 0)];
-                    lacc[a] = t;
+                    more = turns;
+                    if (turns) {
+                        // the next 64 bodies of this turn's leaves, or the next turn
+                        if ((words[turn] >> 20) != 0u) {
+                            if (turn == static_cast<uint32_t>(w)) {
+                                const uint32_t l = static_cast<uint32_t>(__builtin_ctzll(big));
+                                const uint32_t j0 = lane_u32(push, l) & 0x07ffffffu, c = lane_u32(info, l) & ~kMLeaf;
+                                const uint32_t j = j0 + big_k0 + static_cast<uint32_t>(lane);
+                                app = j < j0 + c && body_entry(args_here(args), j, cx, cy, cz, q);
+                                big_k0 += 64u;
+                                if (big_k0 >= c) {
+                                    big_k0 = 0;
+                                    big &= big - 1;
+                                }
+                            }
+                        } else {
+                            more = ++turn < static_cast<uint32_t>(NW);
+                        }
+                    }
                 }
             }
-            // heavy bodies take their accelerations from k_heavy_direct instead;
-            // axis a is written by wavefront a mod NW
-            const WalkArgsP ae = args_here(args);
-            const uint32_t work = n_steps + n_visit / 2u;
-            if (valid && ae->b.hrank[i] < 0) {
-                const bool kick = ae->p.kick != 0;
-                const double half_dt = ae->p.half_dt;
-                const double ax = hax + lacc[0];
-                const double ay = hay + lacc[1];
-                const double az = haz + lacc[2];
-                if (0 % NW == w) {
-                    ae->b.ax[i] = ax;
-                    if (kick) ae->b.vx[i] = ae->b.vx[i] + half_dt * ax;
-                }
-                if (1 % NW == w) {
-                    ae->b.ay[i] = ay;
-                    if (kick) ae->b.vy[i] = ae->b.vy[i] + half_dt * ay;
-                }
-                if (2 % NW == w) {
-                    ae->b.az[i] = az;
-                    if (kick) ae->b.vz[i] = ae->b.vz[i] + half_dt * az;
-                }
-            }
-            // the group's work, the schedules' cost unit: the flushes' costs plus
-            // half the visits (a visit measured half the time of a list step on
-            // the 300k walk)
-            if (valid && w == 0) ae->b.pcost[i] = work;
-            if (tid == 0) {
-                ae->mb.g_inter[g] = n_inter;
-                ae->mb.g_visit[g] = n_visit;
-                ae->mb.g_work[g] = work;
-                ae->mb.g_t0[g] = t_start;
-                ae->mb.g_t1[g] = wall_clock64();
-                ae->mb.g_worker[g] = blockIdx.x * kWaves + (threadIdx.x >> 6);   // (w is 0 for a lone wavefront)
-            }
-            group_sync<NW>();   // the next group writes the exchanged sums and the list
+            base += NW * 64u;
+        } while (base < r.total && !overflow);
+        if (last && deep && !recount && !overflow && args_here(args)->p.count_narrow != 0) {
+            last = false;
+            recount = true;
+            sp = 1u;
+            n_inter = n_visit = n_steps = 0u;
+            if (tid == 0) stk[0] = stack_range(gsys, 1, false);
+        }
+        group_sync<NW>();   // the next round reads the stack
+    }
+    // the virtual lanes' sums (a Kahan sum's value is s - c: c holds the
+    // negative of the rounding lost), added in FP64 in share order
+    double lacc[3];
+    if (NW == 1) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+                part_sum[v * 64 + lane] = static_cast<double>(a == 0 ? acc[v].sx : (a == 1 ? acc[v].sy : acc[v].sz)) -
+                                          static_cast<double>(a == 0 ? acc[v].cx : (a == 1 ? acc[v].cy : acc[v].cz));
+            __builtin_amdgcn_wave_barrier();
+            double t = 0.0;
+            for (uint32_t k = 0; k < S; ++k) t += part_sum[k * cnt + (valid ? lane : 0)];
+            lacc[a] = t;
+            __builtin_amdgcn_wave_barrier();
+        }
+    } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            double* q = part_sum + (v * NW + w) * 64 + lane;
+            q[0] = static_cast<double>(acc[v].sx) - static_cast<double>(acc[v].cx);
+            q[256] = static_cast<double>(acc[v].sy) - static_cast<double>(acc[v].cy);
+            q[512] = static_cast<double>(acc[v].sz) - static_cast<double>(acc[v].cz);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            double t = 0.0;
+            if (a % NW == w)
+                for (uint32_t k = 0; k < S; ++k) t += part_sum[a * 256 + k * cnt + (valid ? lane : 0)];
+            lacc[a] = t;
+        }
+    }
+    // heavy bodies take their accelerations from k_heavy_direct instead;
+    // axis a is written by wavefront a mod NW
+    const WalkArgsP ae = args_here(args);
+    const uint32_t work = n_steps + n_visit / 2u;
+    if (valid && ae->b.hrank[i] < 0) {
+        const bool kick = ae->p.kick != 0;
+        const double half_dt = ae->p.half_dt;
+        const double ax = hax + lacc[0];
+        const double ay = hay + lacc[1];
+        const double az = haz + lacc[2];
+        if (0 % NW == w) {
+            ae->b.ax[i] = ax;
+            if (kick) ae->b.vx[i] = ae->b.vx[i] + half_dt * ax;
+        }
+        if (1 % NW == w) {
+            ae->b.ay[i] = ay;
+            if (kick) ae->b.vy[i] = ae->b.vy[i] + half_dt * ay;
+        }
+        if (2 % NW == w) {
+            ae->b.az[i] = az;
+            if (kick) ae->b.vz[i] = ae->b.vz[i] + half_dt * az;
+        }
+    }
+    // the group's work, the schedules' cost unit: the flushes' costs plus
+    // half the visits (a visit measured half the time of a list step on
+    // the 300k walk)
+    if (valid && w == 0) ae->b.pcost[i] = work;
+    if (tid == 0) {
+        ae->mb.g_inter[g] = n_inter;
+        ae->mb.g_visit[g] = n_visit;
+        ae->mb.g_work[g] = work;
+        ae->mb.g_t0[g] = t_start;
+        ae->mb.g_t1[g] = wall_clock64();
+        ae->mb.g_worker[g] = blockIdx.x * kWaves + (threadIdx.x >> 6);   // (w is 0 for a lone wavefront)
+    }
+    group_sync<NW>();   // the next group writes the exchanged sums and the list
     return work;
 }
 
