@@ -4,14 +4,14 @@
 // Walk groups.  Bodies are cut into groups of at most 64 Morton-consecutive
 // bodies that follow the tree: a cell with <= 64 bodies whose parent holds
 // more is a bucket; consecutive sibling buckets are packed while they fit in
-// 64; a leaf with more than 64 co-keyed bodies is split.  One wavefront walks
-// the tree once per group, one lane per body.
+// 64; a leaf with more than 64 co-keyed bodies is split.  The tree is walked
+// once per group: by one wavefront, or by the four of a block for a group that
+// would end late (share_limit), with the same bits.
 //
 // Opening test per group (the extent test): a node is accepted when
-// b^2 < theta^2 * D^2, with b
-// the distance from the node's centre of mass to the farthest corner of the
-// bounding box of its light bodies (the node's true extent, <= the cell
-// diagonal) and D the FP64 distance from that centre of mass to the group's
+// b^2 < theta^2 * D^2, with b the distance from the node's centre of mass to
+// the farthest corner of the bounding box of its light bodies (the node's true
+// extent, <= the cell diagonal) and D the FP64 distance from that centre of mass to the group's
 // bounding box.  Every body of the group is at least D away, so each body
 // sees the node inside a cone of half-angle ~theta, the same accuracy class
 // as the reference's per-body test (src/traversal.cpp:78), but measured on
@@ -28,17 +28,18 @@
 // lanes test the nodes of their range in FP64.  Accepted nodes and the bodies
 // of reached leaves go into an LDS interaction list as FP32 (x - c, y - c,
 // z - c, G m) with c the group centre (FP64), so the offsets keep FP32
-// precision near the group.  A full list is cut into shares, so that every
-// lane has one whatever the group's size, and evaluated in
-// FP32 FMA over blocks of 32 entries, each block sum added into a
+// precision near the group.  A full list is cut into shares, one for each of
+// up to 256 virtual lanes (share and body) whatever the group's size, and
+// evaluated in FP32 FMA over blocks of 32 entries, each block sum added into a
 // Kahan-compensated FP32 accumulator.  A group's own bodies appear in the
 // list with offsets bit-identical to the lane's own, so the self term has
 // dx = dy = dz = 0 and adds +0 (r^2 starts from a small positive floor).
 //
 // Heavy bodies (the central mass and planets: the heaviest bodies, up to 16)
 // are not in the light moments; every light body adds them by an FP64 direct
-// sum in rank order, and the heavy bodies themselves get an FP64 direct sum
-// over all bodies (k_heavy_direct).  The sum of the two parts is FP64.
+// sum (the ranks k = q mod 4 into partial q, in rank order, then the four
+// partials), and the heavy bodies themselves get an FP64 direct sum over all
+// bodies (heavy_item, k_heavy_final).  The sum of the two parts is FP64.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1214,7 +1215,7 @@ __device__ __forceinline__ uint32_t walk_group(WalkArgsP args, StepScalars* sc, 
             lacc[a] = t;
         }
     }
-    // heavy bodies take their accelerations from k_heavy_direct instead;
+    // heavy bodies take their accelerations from k_heavy_final instead;
     // axis a is written by wavefront a mod NW
     const WalkArgsP ae = args_here(args);
     const uint32_t work = n_steps + n_visit / 2u;
@@ -1457,7 +1458,7 @@ __global__ __launch_bounds__(kNT) void k_heavy_final(Bodies b, TreeBuffers tb, M
 
 // ------------------------------------------------------------ schedule
 // Longest-processing-time order of the groups for the dynamic queue: groups
-// go into 64 buckets of descending estimated cost (two buckets per octave)
+// go into 128 buckets of descending estimated cost (eight buckets per octave)
 // and the queue serves the costliest bucket first.  The order inside a bucket
 // is whatever the atomics give: it changes timing only, never results.
 //

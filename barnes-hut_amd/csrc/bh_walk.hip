@@ -238,10 +238,11 @@ __global__ __launch_bounds__(kNT) void k_walk_plain(Bodies b, size_t n, uint32_t
 // word of the bitmap take, and then the contributions; and the accepted nodes
 // as they were found, whose place the ordered ones take.  More than kFound are
 // read off the bitmap in pieces instead.  A full stack, or more visits than
-// the tree has nodes, sends the body to the walk by one lane.
-// Walk of 3,000 bodies (theta 1.05) 0.140 -> 0.028 ms, 8,000 0.206 -> 0.080,
-// 19,054 0.297 -> 0.197, the last bound by vector instructions and by the
-// latency of a wavefront's rounds (16 wavefronts a CU, by their LDS).
+// the tree has nodes, sends the body to the walk by one lane (walk_alone).
+// Walks of a belt, theta 1.05, per lane and by wavefronts: 3,000 bodies 0.121 and
+// 0.028 ms, 8,000 0.188 and 0.072, 20,480 0.277 and 0.204, the last bound by
+// vector instructions and by the latency of a wavefront's rounds (16 wavefronts a
+// CU, by their LDS).  Where the lists are short the lanes are faster: short_lists.
 constexpr uint32_t kStack = 1024;       // (950 the deepest seen with no limit, at theta 0.1)
 constexpr uint32_t kFound = 1536;
 constexpr uint32_t kWaves = 4;          // bodies of a block, independent of each other
@@ -561,7 +562,8 @@ void launch_walk_plain(const Bodies& b, size_t n, const TreeBuffers& tb, const W
     const uint32_t g = static_cast<uint32_t>((n + kNT - 1) / kNT);
     if (g == 0) return;
     // the XCD-contiguous mapping covers blocks [0, 8 * ceil(g / 8)); blocks
-    // mapped past g return at once
+    // mapped past g have no bodies, but take their part in the L2 sweep, whose
+    // slices count every block of the grid
     const uint32_t grid = ((g + kXcds - 1) / kXcds) * kXcds;
     const uint32_t lead = walk_lead(n, p.theta2);
     if (cnt_accept && cnt_open && cnt_test)
