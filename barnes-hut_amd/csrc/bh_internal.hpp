@@ -600,7 +600,7 @@ void launch_heavy_set(const Bodies& b, const TreeBuffers& tb, const uint32_t* ru
                       const uint32_t* sys_run, uint8_t* bsys, void* scratch, hipStream_t s);
 
 // FP64 direct sum for m sample bodies over the bodies of each sample's system
-// (Neumaier-compensated).
+// (compensated sums, ExactSum).
 void launch_direct_sum(const Bodies& b, const TreeBuffers& tb, const int64_t* idx, size_t m, double G, double soft2,
                        double* acc3, hipStream_t s);
 

@@ -87,7 +87,8 @@ const char *bh_last_error(const bh_ctx *ctx);
 /* Upload n bodies (replaces the reference's rank-0 read + scatter,
  * src/main.cpp:117-171).  ids may be NULL (then ids = 0..n-1 in row order,
  * as src/io.cpp:73).  Resets time to 0 and the accelerations to zero
- * (src/main.cpp:175). */
+ * (src/main.cpp:175).  A call that finds no room (BH_ERR_NOMEM) leaves no
+ * bodies, those of before neither: calls that need them return BH_ERR_STATE. */
 int bh_set_bodies(bh_ctx *ctx, int64_t n, const bh_vec3 *pos, const bh_vec3 *vel,
                   const double *mass, const uint64_t *ids);
 /* Number of bodies held by ctx. */
