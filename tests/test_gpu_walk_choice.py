@@ -9,6 +9,8 @@ import sys
 import numpy as np
 import pytest
 
+from test_zz_no_alloc import Hip
+
 pytestmark = pytest.mark.gpu
 HOUR = 1.0 / 24.0
 
@@ -66,3 +68,25 @@ def test_short_lists_are_walked_per_lane(bh, name, theta):
             took.append(np.median(t))
     say("ms of the walk", took)
     assert took[0] <= 1.4 * took[1]
+
+
+@pytest.mark.parametrize("name,n", [("cube", 12288), ("belt", 12288), ("clusters", 20480)])
+def test_static_evaluation_chooses_too(bh, name, n):
+    say("static walk choice", name, n)
+    pos, vel, mass = shape(bh, name, n)
+    with bh.Engine(theta=1.05) as e:
+        e.set_counting(True)
+        e.set_bodies(pos, vel, mass)
+        e.compute_accelerations(theta=1.05)
+        st = e.get_bodies()
+    want = np.empty_like(pos)
+    want[st["ids"].astype(np.int64)] = st["acc"]
+    hip = Hip(bh)
+    try:
+        dpos, dm, dacc = hip.put(pos), hip.put(mass), hip.alloc(24 * n)
+        for _ in range(2):
+            assert bh.load().bh_compute_accelerations_static(n, dpos, dm, 1.05, bh.G, 0.0, dacc, None) == 0
+            hip.sync()
+            assert np.array_equal(bits(hip.get(dacc, (n, 3))), bits(want))
+    finally:
+        hip.free()
